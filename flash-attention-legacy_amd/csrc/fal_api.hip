@@ -178,14 +178,16 @@ static int fal_fwd_impl(const void* q, const void* k, const void* v, void* o, fl
   }
   // pipelined kernel with at least two items per CU: one persistent workgroup per CU
   // walks pairs of query tiles
+  const int ncu = device_cu_count();
   if (!p.kchunk && fwd_pipe_ok((int)head_dim)) {
-    const int ncu = device_cu_count();
     if (FAL_FWD_PERSIST && ncu > 0 && nblocks >= 2 * (int64_t)ncu) {
       p.persist = 1;
       const int64_t pairs = (int64_t)(p.n_qtiles + 1) / 2 * batch * (heads_q / (p.gqa4 ? 4 : 1));
       nblocks = std::min<int64_t>(pairs, ncu);
     }
   }
+  if (is_causal && !p.kchunk && !p.persist && !p.gqa4)
+    p.lpt = fwd_causal_order((int)head_dim, nblocks, batch * heads_q, ncu);
   if (nblocks > 0x7fffffff) return fail(FAL_ERR_INVALID, "problem too large for one launch");
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e = launch_fwd(p, (int)head_dim, is_causal != 0, dim3((unsigned)nblocks), st);

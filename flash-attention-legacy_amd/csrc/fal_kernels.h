@@ -45,6 +45,9 @@ struct FwdParams {
   // (n_qtiles counts 64-row tiles, the grid B * Hq/4 * n_qtiles), so under a causal mask
   // every wave stops at the same diagonal tile.
   int gqa4;
+  // Causal batched grid of one query tile per workgroup: 0 = head by head; otherwise longest
+  // tiles first over all heads, reversed from this rank on (fwd_item; fwd_causal_order).
+  int lpt;
   // pipelined kernel: persistent grid (one workgroup per CU walking pairs of query tiles)
   int persist;
 };
@@ -121,6 +124,9 @@ int fwd_block_m_varlen(int d);   // query rows per workgroup of a packed-sequenc
 int fwd_block_n(int d);
 // Split-KV plan for a batched forward: sets kchunk / nsplit (kchunk 0 = no split) and
 // returns the workspace bytes the split needs (0 without a split).
+// FwdParams::lpt of a causal grid of `nblocks` workgroups over `units` heads (batch x query
+// head) on a GPU of `ncu` compute units.
+int fwd_causal_order(int d, int64_t nblocks, int64_t units, int ncu);
 size_t fwd_split_plan(int64_t B, int64_t Hq, int64_t Nq, int64_t Nk, int d, int causal, int* kchunk, int* nsplit);
 hipError_t launch_fwd_combine(const FwdParams& p, int d, int causal, hipStream_t st);
 // Rows of up to two packed [rows, heads, d] 16-bit tensors that the schedule kernel
