@@ -170,16 +170,21 @@ static int fal_fwd_impl(const void* q, const void* k, const void* v, void* o, fl
     p.part_o = static_cast<float*>(workspace);
     p.part_ml = p.part_o + (size_t)batch * heads_q * p.nsplit * seqlen_q * head_dim;
   }
+  const int ncu = device_cu_count();
+  const bool pipe = !p.kchunk && fwd_pipe_ok((int)head_dim);
+  if (pipe && !fwd_wide_pays(batch, heads_q, heads_kv, seqlen_q, seqlen_k, is_causal != 0, ncu)) {
+    p.narrow = 1;
+    p.n_qtiles = cdiv((int)seqlen_q, fwd_block_m_varlen((int)head_dim));
+  }
   int64_t nblocks = (int64_t)p.n_qtiles * batch * heads_q * p.nsplit;
-  if (!p.kchunk && fwd_gqa4_ok((int)head_dim, heads_q, heads_kv)) {
+  if (pipe && !p.narrow && fwd_gqa4_ok((int)head_dim, heads_q, heads_kv)) {
     p.gqa4 = 1;
     p.n_qtiles = cdiv((int)seqlen_q, 64);
     nblocks = (int64_t)p.n_qtiles * batch * (heads_q / 4);
   }
   // pipelined kernel with at least two items per CU: one persistent workgroup per CU
   // walks pairs of query tiles
-  const int ncu = device_cu_count();
-  if (!p.kchunk && fwd_pipe_ok((int)head_dim)) {
+  if (pipe && !p.narrow) {
     if (FAL_FWD_PERSIST && ncu > 0 && nblocks >= 2 * (int64_t)ncu) {
       p.persist = 1;
       const int64_t pairs = (int64_t)(p.n_qtiles + 1) / 2 * batch * (heads_q / (p.gqa4 ? 4 : 1));

@@ -1100,8 +1100,9 @@ static hipError_t launch_fwd_t(const FwdParams& p, int causal, dim3 grid, hipStr
 template <int D>
 static hipError_t launch_fwd_d(const FwdParams& p, int causal, dim3 grid, hipStream_t st) {
   // packed sequences keep their own tile configuration, except under the four-heads
-  // layout, which runs the batched (pipelined) kernel over the work list
-  if (p.cu_q && !p.gqa4)
+  // layout, which runs the batched (pipelined) kernel over the work list; batched calls
+  // take that configuration too where it is the faster one (fwd_wide_pays)
+  if ((p.cu_q && !p.gqa4) || p.narrow)
     return p.bf16 ? launch_fwd_t<bf16_t, D, true>(p, causal, grid, st)
                   : launch_fwd_t<half_t, D, true>(p, causal, grid, st);
   return p.bf16 ? launch_fwd_t<bf16_t, D, false>(p, causal, grid, st)
@@ -1180,6 +1181,46 @@ int fwd_causal_order(int d, int64_t nblocks, int64_t units, int ncu) {
   if (ncu <= 0 || nblocks <= ncu || nblocks > 16 * (int64_t)ncu) return 0;
   if (d <= 128 && nblocks <= 2 * (int64_t)ncu) return units % 8 == 0 ? ncu / 8 : ncu;
   return kAll;
+}
+
+// Head dim 128 has two batched kernels.  The pipelined one (one 256-row workgroup per CU, 1.7 us
+// per 64-key tile) is the faster per flop on a full GPU; the C++ loop on 128-row workgroups,
+// two per CU, costs 1.06 us per tile and workgroup then and 1.15 alone, so it wins where the
+// pipelined grid leaves CUs idle, ends in a nearly empty round, or pays its start and end
+// (about 10 us, overlapped by nothing) for a few tiles.  The estimates below are fitted to 50
+// shapes of MI355X times (batch 1-128, 100-8192 rows, MHA and GQA, causal or not): they pick
+// the faster kernel or the pipelined one on each.  us, pipelined / 128-row: 1 x 32/8 heads x
+// 1531 causal 43 / 34, 4 x 32/8 x 512 causal 24 / 19, 5 x 28/4 x 777 causal 87 / 44,
+// 4 x 16 x 1024 causal 37 / 30, 32 x 16 x 256 41 / 33; 2 x 32/8 x 2048 causal 76 / 82,
+// 1 x 32/8 x 2048 non-causal 66 / 73.
+// The 128-row workgroups copy twice the K/V per flop.  A long causal grid of one item per CU
+// lets CUs idle, which at the board's power limit comes back as clock, also for the kernels
+// around it: 2 x 16 x 2048 causal alone takes 62 / 54 us, but a training step of it 195 / 197.
+// Such grids need a margin.
+bool fwd_wide_pays(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int causal, int ncu) {
+  if (ncu <= 0 || Nq <= 0 || Nk <= 0) return true;
+  const double cus = ncu;
+  auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const int64_t n = up(causal ? std::min(Nk, up(Nq, 64) * 64) : Nk, 64);   // key tiles of the last rows
+  // key tiles summed over `tiles` query tiles of 64 * k rows
+  auto steps = [&](int64_t tiles, int64_t k) {
+    const int64_t m = causal ? std::min(tiles, n / k) : 0;
+    return (double)k * m * (m + 1) / 2 + (double)(tiles - m) * n;
+  };
+  const double narrow = std::max(6 + 1.15 * n, (causal ? 12 : 9) + 1.06 * B * Hq * steps(up(Nq, 128), 2) / cus);
+  const bool gqa4 = fwd_gqa4_ok(128, Hq, Hkv);
+  const int64_t k = gqa4 ? 1 : 4, units = B * Hq / (gqa4 ? 4 : 1), tiles = up(Nq, 64 * k), items = tiles * units;
+  double wide;
+  if (items >= 2 * (int64_t)ncu) {        // persistent: rounds of pairs of items
+    const int64_t pairs = up(tiles, 2);
+    wide = 6 + up(pairs * units, ncu) * (1.63 * steps(tiles, k) / pairs + (tiles > 1 ? 10 : 5));
+  } else if (!causal) {
+    wide = up(items, ncu) * (10 + 1.72 * n);
+  } else {
+    wide = 10 + std::max(1.72 * n, (1.8 * units * steps(tiles, k) + 7.0 * items) / cus);
+    if (n >= 24) wide /= 1.4;
+  }
+  return wide <= narrow;
 }
 
 template <class T, int D>

@@ -45,6 +45,9 @@ struct FwdParams {
   // (n_qtiles counts 64-row tiles, the grid B * Hq/4 * n_qtiles), so under a causal mask
   // every wave stops at the same diagonal tile.
   int gqa4;
+  // Batched head_dim 128 on 128-row workgroups, two per CU (the packed-sequence
+  // configuration), instead of the pipelined kernel (fwd_wide_pays).
+  int narrow;
   // Causal batched grid of one query tile per workgroup: 0 = head by head; otherwise longest
   // tiles first over all heads, reversed from this rank on (fwd_item; fwd_causal_order).
   int lpt;
@@ -124,6 +127,8 @@ int fwd_block_m_varlen(int d);   // query rows per workgroup of a packed-sequenc
 int fwd_block_n(int d);
 // Split-KV plan for a batched forward: sets kchunk / nsplit (kchunk 0 = no split) and
 // returns the workspace bytes the split needs (0 without a split).
+// True when the pipelined kernel is the faster of head_dim 128's two for this batched call.
+bool fwd_wide_pays(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int causal, int ncu);
 // FwdParams::lpt of a causal grid of `nblocks` workgroups over `units` heads (batch x query
 // head) on a GPU of `ncu` compute units.
 int fwd_causal_order(int d, int64_t nblocks, int64_t units, int ncu);

@@ -32,3 +32,39 @@ def check_forward(B, Hq, Hkv, Nq, Nk, d, causal):
 ])
 def test_causal_order(B, Hq, Hkv, N, d):
     check_forward(B, Hq, Hkv, N, N, d, True)
+
+
+# head_dim 128 where the pipelined grid would leave CUs idle or end in a nearly empty round:
+# 128-row workgroups.  GQA ratios 7, 4 and 1; one, two and several query tiles, the last of
+# one row and of 128; fewer workgroups than CUs, up to two per CU and more; Nq != Nk.
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,Nq,Nk", [
+    (1, 28, 4, 333, 333),
+    (2, 8, 8, 130, 517),
+    (9, 32, 8, 129, 129),
+    (5, 28, 4, 257, 192),
+    (3, 16, 16, 640, 640),
+    (20, 16, 4, 64, 65),
+])
+def test_head_dim_128_small_grid(B, Hq, Hkv, Nq, Nk, causal):
+    check_forward(B, Hq, Hkv, Nq, Nk, 128, causal)
+
+
+# ... and where the pipelined persistent grid stays the faster one: one full round of 256
+# pairs of query tiles (odd and even tile counts; four heads per workgroup and 256 rows of
+# one head; Nq != Nk; a negative scale).
+@pytest.mark.parametrize("B,Hq,Hkv,Nq,Nk,sign,causal", [
+    (2, 16, 4, 4032, 4032, 1, True),
+    (2, 16, 4, 4032, 4032, -1, True),
+    (2, 16, 16, 3840, 3840, 1, True),
+    (2, 16, 8, 4090, 4090, 1, False),
+    (2, 16, 4, 4032, 5000, 1, False),
+    (2, 16, 4, 4096, 3000, 1, True),
+])
+def test_head_dim_128_full_grid(B, Hq, Hkv, Nq, Nk, sign, causal):
+    from flash_attn_legacy import hip_ext
+    from test_fwd_gpu import check_groups
+    q, k, v = randn((B, Hq, Nq, 128), 3), randn((B, Hkv, Nk, 128), 4), randn((B, Hkv, Nk, 128), 5)
+    scale = sign * 128 ** -0.5
+    o, lse = hip_ext.forward(q, k, v, scale, causal)
+    check_groups(o, lse, q, k, v, scale, causal, [(b, g) for b in range(B) for g in range(Hkv)])
