@@ -346,20 +346,21 @@ int fal_fwd_varlen_bf16(const void* q, const void* k, const void* v, void* o, fl
 // ---------------------------------------------------------------------------
 // Backward workspace: delta [rows] fp32, plus, for head dims without the query-outer
 // dQ kernel, the fp32 dQ accumulator [rows, d] in front of it.
-static size_t bwd_acc_bytes(size_t rows, int64_t head_dim) {
-  return bwd_split_dq(head_dim_ok(head_dim) ? (int)head_dim : 0) ? 0 : align256(rows * head_dim * sizeof(float));
+static size_t bwd_acc_bytes(size_t rows, int64_t head_dim, bool batched) {
+  return bwd_split_dq(head_dim_ok(head_dim) ? (int)head_dim : 0, batched) ? 0 : align256(rows * head_dim * sizeof(float));
 }
 
-// Batched head_dim 128 also holds the lsd array: per (batch, query head, 64-row tile)
-// 64 values of -L*log2(e)/c and 64 of -D.
+// Batched head_dim 128 and 256 also hold the lsd array: per (batch, query head, tile of 64
+// or 32 rows) a value of -L*log2(e)/c and one of -D per row.
 static size_t bwd_lsd_bytes(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim) {
   if (!head_dim_ok(head_dim) || !bwd_pipe((int)head_dim)) return 0;
-  return align256((size_t)batch * heads_q * ((seqlen_q + 63) / 64) * 128 * sizeof(float));
+  const int64_t bm = bwd_pipe_bm((int)head_dim);
+  return align256((size_t)batch * heads_q * ((seqlen_q + bm - 1) / bm) * 2 * bm * sizeof(float));
 }
 
 size_t fal_bwd_workspace_size(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim) {
   const size_t rows = (size_t)batch * heads_q * seqlen_q;
-  return bwd_acc_bytes(rows, head_dim) + align256(rows * sizeof(float)) +
+  return bwd_acc_bytes(rows, head_dim, true) + align256(rows * sizeof(float)) +
          bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim);
 }
 
@@ -397,7 +398,7 @@ static int fill_bwd_common(BwdParams& p, const void* dout, const void* q, const 
 
 static int run_bwd(BwdParams& p, int d, int causal, dim3 grid, dim3 dq_grid, bool batched, hipStream_t st) {
   hipError_t e;
-  if (bwd_split_dq(d)) {
+  if (bwd_split_dq(d, batched)) {
     // dQ kernel first: it also computes D = rowsum(dO * O), which the dK/dV kernel
     // reads, so no preprocessing launch is needed
     if (dq_grid.x > 0 && dq_grid.y > 0) {
@@ -438,7 +439,7 @@ static int fal_bwd_impl(const void* dout, const void* q, const void* k, const vo
     return fail(FAL_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu", need, workspace_bytes);
   if (batch == 0 || (seqlen_k == 0 && seqlen_q == 0)) return ok();
   const size_t rows = (size_t)batch * heads_q * seqlen_q;
-  const size_t acc = bwd_acc_bytes(rows, head_dim);
+  const size_t acc = bwd_acc_bytes(rows, head_dim, true);
   p.dq_acc = acc ? static_cast<float*>(workspace) : nullptr;
   p.delta = reinterpret_cast<float*>(static_cast<char*>(workspace) + acc);
   if (bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim))
@@ -487,8 +488,8 @@ size_t fal_bwd_varlen_workspace_size(int64_t num_seqs, int64_t total_q, int64_t 
   const int d = head_dim_ok(head_dim) ? (int)head_dim : 128;
   const int bn = bwd_block_n(d);
   const size_t cap = (size_t)((total_k + bn - 1) / bn + num_seqs);
-  size_t bytes = bwd_acc_bytes(rows, head_dim) + align256(rows * sizeof(float)) + align256(cap * sizeof(int2));
-  if (bwd_split_dq(d)) {
+  size_t bytes = bwd_acc_bytes(rows, head_dim, false) + align256(rows * sizeof(float)) + align256(cap * sizeof(int2));
+  if (bwd_split_dq(d, false)) {
     const int bm = bwd_dq_block_m(d);
     bytes += align256((size_t)((total_q + bm - 1) / bm + num_seqs) * sizeof(int2));
   }
@@ -522,7 +523,7 @@ static int fal_bwd_varlen_impl(const void* dout, const void* q, const void* k, c
   if (total_q == 0 && total_k == 0) return ok();
   const size_t rows = (size_t)total_q * heads_q;
   char* ws = static_cast<char*>(workspace);
-  const size_t acc = bwd_acc_bytes(rows, head_dim);
+  const size_t acc = bwd_acc_bytes(rows, head_dim, false);
   p.dq_acc = acc ? reinterpret_cast<float*>(ws) : nullptr;
   ws += acc;
   p.delta = reinterpret_cast<float*>(ws);
@@ -553,7 +554,7 @@ static int fal_bwd_varlen_impl(const void* dout, const void* q, const void* k, c
                                         work, cap, st, &zkv);
   if (e != hipSuccess) return launch_status(e, "fal_bwd_varlen schedule");
   dim3 dq_grid(0, 0);
-  if (bwd_split_dq((int)head_dim)) {
+  if (bwd_split_dq((int)head_dim, false)) {
     // query tiles for the dQ kernel, grouped by sequence (as the forward's list)
     const int bm = bwd_dq_block_m((int)head_dim);
     const int capq = (int)((total_q + bm - 1) / bm + num_seqs);

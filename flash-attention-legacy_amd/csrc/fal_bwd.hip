@@ -16,7 +16,9 @@
 //     accumulators straight into the B operands of dV^T += dO^T P and
 //     dK^T += Q^T dS (dO^T and Q^T from the Q/dO tiles via ds_read_b64_tr_b16);
 //     dK/dV stay in registers until the end.
-// * head_dim 256: bwd_pre_kernel (D, zeroed fp32 dQ accumulator), bwd_kernel
+//   Batched head_dim 128 and 256 run both as software-pipelined asm loops
+//   (bwd_kv_pipe_kernel, bwd_dq_kernel with PIPE).
+// * packed head_dim 256: bwd_pre_kernel (D, zeroed fp32 dQ accumulator), bwd_kernel
 //   (KV-outer, dS^T staged in LDS, dQ = dS K added with fp32 atomics; all 256 dK/dV
 //   columns accumulate in one pass, with K read from its LDS tile) and bwd_post_kernel
 //   (dQ cast to fp16).
@@ -812,36 +814,41 @@ bwd2_kernel(BwdParams p) {
 
 
 // --------------------------------------------------------------------------
-// dK/dV kernel for head_dim 128, batched (bwd_kv_pipe_kernel): one wave per SIMD and a
-// software-pipelined query-tile loop written as one inline-asm block (fal_bwd_pipe.inc,
+// dK/dV kernel for head_dim 128 and 256, batched (bwd_kv_pipe_kernel): one wave per SIMD and
+// a software-pipelined query-tile loop written as one inline-asm block (fal_bwd_pipe.inc,
 // generated by gen_bwd_pipe.py).  A workgroup owns 128 keys of one KV head, each wave
 // 32 keys whose K and V fragments stay in registers; the items (query head of the
-// group, 64-row query tile) stream through a 4-slot LDS ring of Q/dO tiles copied two
-// items ahead.  Per item the S and dP accumulators start at -L*log2(e)/c and -D, read
-// from the tile-major array `lsd` that bwd_dq_kernel writes, so P = exp2(c*S) and
-// dS = P*dP.  The products of item i-1 (dV^T += dO^T P, dK^T += Q^T dS), the
-// exponentials of item i and the products of item i+1 (S = Q K^T, dP = dO V^T)
+// group, query tile of 64 rows, or of 32 for head_dim 256) stream through a 4-slot LDS ring
+// of Q/dO tiles copied two items ahead.  Per item the S and dP accumulators start at
+// -L*log2(e)/c and -D, read from the tile-major array `lsd` that bwd_dq_kernel writes, so
+// P = exp2(c*S) and dS = P*dP.  The products of item i-1 (dV^T += dO^T P, dK^T += Q^T dS),
+// the exponentials of item i and the products of item i+1 (S = Q K^T, dP = dO V^T)
 // overlap inside the wave; no cross-wave sum is needed.  Same math as bwd2_kernel.
+// Bound by the MFMA stream (64 per item; 916 TFLOP/s of products at head_dim 128).  Head dim
+// 256 replaced the fp32-atomic form, which its atomics bound at 1 TB/s: both kernels of
+// B2 x 16/8 heads x 2048 causal 957 -> 322 us, B2 x 16 x 4096 2147 -> 942 (non-causal
+// 4053 -> 1709).
 // --------------------------------------------------------------------------
 #ifndef FAL_BWD_PIPE
 #define FAL_BWD_PIPE 1
 #endif
 constexpr int kPipeBN = 128;    // keys per workgroup
-// dK/dV hand-off in LDS after the loop: per wave, dV then dK*scale, 16 pieces of 512
+// dK/dV hand-off in LDS after the loop: per wave, dV then dK*scale, D/8 pieces of 512
 // bytes each, kKvOStr apart so the row-wise reads of the epilogue spread over the banks
 constexpr int kKvOStr = 528;
-constexpr int kKvOPart = 16 * kKvOStr;
-constexpr int kKvOWave = 2 * kKvOPart;
-constexpr int kPipeBM = 64;     // query rows per item
+template <int D>
+constexpr int pipe_bm() { return D == 256 ? 32 : 64; }   // query rows per item
 
-template <class T, bool CAUSAL>
+template <class T, int D, bool CAUSAL>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 bwd_kv_pipe_kernel(BwdParams p) {
   using V8 = vec8<T>;
-  using TL = SwizzledTile<128>;
-  constexpr int CPR = TL::CPR;
-  // 4 slots of (Q tile, dO tile) and 4 slots of (64 Ls, 64 Dn) values
-  __shared__ __attribute__((aligned(1024))) char smem[4 * 32768 + 4 * 512];
+  using TL = SwizzledTile<D>;
+  constexpr int CPR = TL::CPR, KS = D / 16, kPipeBM = pipe_bm<D>();
+  constexpr int kKvOPart = (D / 8) * kKvOStr, kKvOWave = 2 * kKvOPart;
+  // 4 slots of (Q tile, dO tile) and 4 slots of Ls and Dn values; then the hand-off
+  constexpr int kRing = 4 * 32768 + 4 * 512;
+  __shared__ __attribute__((aligned(1024))) char smem[kRing > 4 * kKvOWave ? kRing : 4 * kKvOWave];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -902,11 +909,13 @@ bwd_kv_pipe_kernel(BwdParams p) {
   const uint32_t p_qrb = (uint32_t)(p.q_ss * 2), p_drb = (uint32_t)(p.do_ss * 2);
   const int p_nq = nq, p_nqt = nqt;
   const int64_t qstep = (int64_t)kPipeBM * p.q_ss * 2, dstep = (int64_t)kPipeBM * p.do_ss * 2;
+  // head_dim 256: an item's copies leave the resources 16 rows on
+  const int64_t qhalf = D == 256 ? 16 * p.q_ss * 2 : 0, dhalf = D == 256 ? 16 * p.do_ss * 2 : 0;
 
   // K and V of this wave's 32 keys of key tile kt (B operands), buffer loads: keys past
   // the end read as zeros.  The second tile's are loaded right after the first tile's
   // loop, so their latency overlaps that tile's epilogue.
-  V8 kreg[8], vreg[8];
+  V8 kreg[KS], vreg[KS];
   auto load_kv = [&](int kt) {
     // one resource per key tile: its rows inside the sequence, offsets from its first row
     const int n0 = kt * kPipeBN;
@@ -920,7 +929,7 @@ bwd_kv_pipe_kernel(BwdParams p) {
     const int r = ws * 32 + l32;
     const int ko = (int)(r * p.k_ss * 2) + hh * 16, vo = (int)(r * p.v_ss * 2) + hh * 16;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
+    for (int t = 0; t < KS; ++t) {
       kreg[t] = __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(krs, ko + t * 32, 0, 0));
       vreg[t] = __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(vrs, vo + t * 32, 0, 0));
     }
@@ -942,30 +951,36 @@ bwd_kv_pipe_kernel(BwdParams p) {
       const uint64_t dob = (uint64_t)(uintptr_t)((const T*)p.dout + (int64_t)b * p.do_sb +
                                                  (int64_t)hq0 * p.do_sh + (int64_t)qt0 * kPipeBM * p.do_ss);
       const uint64_t lb = (uint64_t)(uintptr_t)(p.lsd + (((int64_t)b * p.Hq + hq0) * nqt + qt0) * 2 * kPipeBM);
-      const int64_t qwrap = p.q_sh * 2 - (int64_t)(ntq - 1) * qstep;
-      const int64_t dwrap = p.do_sh * 2 - (int64_t)(ntq - 1) * dstep;
+      const int64_t qwrap = p.q_sh * 2 - (int64_t)(ntq - 1) * qstep - qhalf;
+      const int64_t dwrap = p.do_sh * 2 - (int64_t)(ntq - 1) * dstep - dhalf;
       const uint32_t p_qb_lo = (uint32_t)qb, p_qb_hi = (uint32_t)(qb >> 32) & 0xffffu;
       const uint32_t p_db_lo = (uint32_t)dob, p_db_hi = (uint32_t)(dob >> 32) & 0xffffu;
       const uint32_t p_lb_lo = (uint32_t)lb, p_lb_hi = (uint32_t)(lb >> 32) & 0xffffu;
-      const uint32_t p_qs_lo = (uint32_t)qstep, p_qs_hi = (uint32_t)((uint64_t)qstep >> 32);
+      const uint32_t p_qs_lo = (uint32_t)(qstep - qhalf), p_qs_hi = (uint32_t)((uint64_t)(qstep - qhalf) >> 32);
       const uint32_t p_qw_lo = (uint32_t)qwrap, p_qw_hi = (uint32_t)((uint64_t)qwrap >> 32);
-      const uint32_t p_ds_lo = (uint32_t)dstep, p_ds_hi = (uint32_t)((uint64_t)dstep >> 32);
+      const uint32_t p_ds_lo = (uint32_t)(dstep - dhalf), p_ds_hi = (uint32_t)((uint64_t)(dstep - dhalf) >> 32);
       const uint32_t p_dw_lo = (uint32_t)dwrap, p_dw_hi = (uint32_t)((uint64_t)dwrap >> 32);
       const uint32_t p_ldw = (uint32_t)(1 + qt0) * 2 * kPipeBM * 4;   // last tile of a head -> first of the next
       const int p_qt0 = qt0, p_nitems = nitems;
       const int p_kw0 = CAUSAL ? kw0 : -(1 << 30);
-      if constexpr (std::is_same<T, half_t>::value)
+      constexpr bool F16 = std::is_same<T, half_t>::value;
+      if constexpr (D == 128 && F16)
         asm volatile(FAL_BWDP_ASM_F16 : FAL_BWDP_OUTS : FAL_BWDP_INS : FAL_BWDP_CLOBBERS);
-      else
+      if constexpr (D == 128 && !F16)
         asm volatile(FAL_BWDP_ASM_BF16 : FAL_BWDP_OUTS : FAL_BWDP_INS : FAL_BWDP_CLOBBERS);
+      if constexpr (D == 256 && F16)
+        asm volatile(FAL_BWDP256_ASM_F16 : FAL_BWDP256_OUTS : FAL_BWDP256_INS : FAL_BWDP256_CLOBBERS);
+      if constexpr (D == 256 && !F16)
+        asm volatile(FAL_BWDP256_ASM_BF16 : FAL_BWDP256_OUTS : FAL_BWDP256_INS : FAL_BWDP256_CLOBBERS);
     }
     if (tile_i == 0 && kt_b >= 0) load_kv(kt_b);
     // dV then dK*scale of this wave's keys: piece pc = db*4 + g4 of lane (hh, l32) holds
     // columns 8*pc + hh*4 .. +3 of key kw0 + l32, at which*kKvOPart + pc*kKvOStr + lane*8.
-    // Written back row-wise: each 16-byte store instruction covers 4 whole 256-byte rows.
+    // Written back row-wise: each 16-byte store instruction covers whole rows.
     {
+      constexpr int RPI = 64 / CPR;            // rows per store instruction
       const char* wb = smem + ws * kKvOWave;
-      const int cch = lane & 15;
+      const int cch = lane % CPR;
       // buffer resources over this wave's keys inside the sequence: stores past the end
       // are dropped (no branch, no 64-bit address per store)
       const int nkw = max(min(nk - kw0, 32), 0);
@@ -974,29 +989,31 @@ bwd_kv_pipe_kernel(BwdParams p) {
                     (uint32_t)((int64_t)nkw * p.dv_ss * 2)),
           make_rsrc((T*)p.dk + (int64_t)b * p.dk_sb + (int64_t)hkv * p.dk_sh + (int64_t)kw0 * p.dk_ss,
                     (uint32_t)((int64_t)nkw * p.dk_ss * 2))};
-      const int vo[2] = {((lane >> 4) * (int)p.dv_ss + cch * 8) * 2, ((lane >> 4) * (int)p.dk_ss + cch * 8) * 2};
-      const int rstep[2] = {(int)p.dv_ss * 8, (int)p.dk_ss * 8};   // 4 rows, in bytes
+      const int vo[2] = {((lane / CPR) * (int)p.dv_ss + cch * 8) * 2, ((lane / CPR) * (int)p.dk_ss + cch * 8) * 2};
+      const int rstep[2] = {(int)p.dv_ss * 2 * RPI, (int)p.dk_ss * 2 * RPI};   // rows of an instruction, in bytes
 #pragma unroll
-      for (int which = 0; which < 2; ++which) {
-        u32x4 x[8];
+      for (int which = 0; which < 2; ++which)
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-          const int r = jj * 4 + (lane >> 4);
-          const char* src = wb + which * kKvOPart + cch * kKvOStr;
-          const uint2 lo = *reinterpret_cast<const uint2*>(src + r * 8);
-          const uint2 hi = *reinterpret_cast<const uint2*>(src + (32 + r) * 8);
-          x[jj] = nitems > 0 ? u32x4{lo.x, lo.y, hi.x, hi.y} : u32x4{0u, 0u, 0u, 0u};
+        for (int j0 = 0; j0 < 32 / RPI; j0 += 8) {
+          u32x4 x[8];
+#pragma unroll
+          for (int jj = 0; jj < 8; ++jj) {
+            const int r = (j0 + jj) * RPI + lane / CPR;
+            const char* src = wb + which * kKvOPart + cch * kKvOStr;
+            const uint2 lo = *reinterpret_cast<const uint2*>(src + r * 8);
+            const uint2 hi = *reinterpret_cast<const uint2*>(src + (32 + r) * 8);
+            x[jj] = nitems > 0 ? u32x4{lo.x, lo.y, hi.x, hi.y} : u32x4{0u, 0u, 0u, 0u};
+          }
+#pragma unroll
+          for (int jj = 0; jj < 8; ++jj) buffer_store16(rs[which], vo[which] + (j0 + jj) * rstep[which], x[jj]);
         }
-#pragma unroll
-        for (int jj = 0; jj < 8; ++jj) buffer_store16(rs[which], vo[which] + jj * rstep[which], x[jj]);
-      }
     }
   }
 }
 
 // --------------------------------------------------------------------------
-// Query-outer dQ kernel for head_dim 32, 64, 96 and 128 (the KV-outer kernel above then
-// produces only dK/dV).  Same structure as the forward kernel: a workgroup owns
+// Query-outer dQ kernel for head_dim 32, 64, 96 and 128, and batched 256 (the KV-outer
+// kernel above then produces only dK/dV).  Same structure as the forward kernel: a workgroup owns
 // 32*NW query rows of one query head, each wave 32 rows whose Q and dO slices stay
 // in VGPRs as the B operands of S^T = K Q^T and dP^T = V dO^T; K/V tiles of BN keys
 // are staged in swizzled LDS by direct buffer loads, double-buffered.  Per tile:
@@ -1008,15 +1025,14 @@ bwd_kv_pipe_kernel(BwdParams p) {
 #ifndef FAL_BWD_DQ_PAIR
 #define FAL_BWD_DQ_PAIR 1
 #endif
-// pipelined dQ loop's hand-off in LDS: 16 blocks of 1 KB per wave, kDqOStr apart (row-wise
+// pipelined dQ loop's hand-off in LDS: D/8 blocks of 1 KB per wave, kDqOStr apart (row-wise
 // reads of the epilogue spread over the banks)
 constexpr int kDqOStr = 1040;
-constexpr int kDqOWave = 16 * kDqOStr;
 #ifndef FAL_BWD_DQ_WPE
 #define FAL_BWD_DQ_WPE 2
 #endif
 #ifndef FAL_BWD_DQ_PIPE
-#define FAL_BWD_DQ_PIPE 1   // batched head_dim 128: software-pipelined key-tile loop (fal_dq_pipe.inc)
+#define FAL_BWD_DQ_PIPE 1   // batched head_dim 128 (and 256): software-pipelined key-tile loop (fal_dq_pipe.inc)
 #endif
 template <class T, int D, int NW, int BN, bool CAUSAL, bool PIPE = false>
 __global__ void __launch_bounds__(NW * 64)
@@ -1033,11 +1049,14 @@ bwd_dq_kernel(BwdParams p) {
   constexpr int PART = BN * CPR * 8;
   constexpr int IPT = BN * CPR / (NW * 64);
   static_assert(BN * CPR % (NW * 64) == 0, "tile must split evenly over the waves");
-  // PIPE (batched, head_dim 128): the key-tile loop is the software-pipelined asm block
-  // of fal_dq_pipe.inc at one wave per SIMD, with a ring of 4 K/V tiles
-  static_assert(!PIPE || (D == 128 && NW == 4 && BN == 64), "the pipelined loop is written for this shape");
+  // PIPE (batched, head_dim 128 and 256): the key-tile loop is the software-pipelined asm
+  // block of fal_dq_pipe.inc at one wave per SIMD, with a ring of 4 K/V tiles
+  static_assert(!PIPE || ((D == 128 || D == 256) && NW == 4 && BN * D == 8192),
+                "the pipelined loop is written for these shapes");
+  constexpr int kDqOWave = (D / 8) * kDqOStr, kPipeBM = pipe_bm<D>();
+  constexpr int NRING = (PIPE ? 4 : 2) * 2 * PART;
 
-  __shared__ __attribute__((aligned(1024))) T smem[(PIPE ? 4 : 2) * 2 * PART];
+  __shared__ __attribute__((aligned(1024))) T smem[PIPE && 2 * kDqOWave > NRING ? 2 * kDqOWave : NRING];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1124,12 +1143,12 @@ bwd_dq_kernel(BwdParams p) {
   if (hh == 0 && row < nq) p.delta[lrow + (int64_t)row * p.l_ss] = drow;
   const float c = p.scale_log2;
   if (p.lsd && hh == 0) {
-    // tile-major copy for bwd_kv_pipe_kernel, 64 rows per tile: -L*log2(e)/c, then -D.
+    // tile-major copy for bwd_kv_pipe_kernel, kPipeBM rows per tile: -L*log2(e)/c, then -D.
     // Rows past the end (up to the tile boundary) and rows without keys get the value
     // whose exponent c * x is -inf, and -D = 0.
-    const int nt64 = cdiv(nq, kPipeBM);
-    if (row < nt64 * kPipeBM) {
-      float* t = p.lsd + (((int64_t)b * p.Hq + hq) * nt64 + row / kPipeBM) * 2 * kPipeBM + row % kPipeBM;
+    const int nt = cdiv(nq, kPipeBM);
+    if (row < nt * kPipeBM) {
+      float* t = p.lsd + (((int64_t)b * p.Hq + hq) * nt + row / kPipeBM) * 2 * kPipeBM + row % kPipeBM;
       const bool live = row < nq && lrow2 != INFINITY;
       t[0] = live ? -lrow2 / c : (c > 0.f ? -INFINITY : INFINITY);
       t[kPipeBM] = row < nq ? -drow : 0.f;
@@ -1202,43 +1221,52 @@ bwd_dq_kernel(BwdParams p) {
     const int p_jend = ntiles, p_nk = nk;
     const int p_wrow = CAUSAL ? wrow0 : 0x3fffffff;
     if (ntiles > 0) {
-      if constexpr (std::is_same<T, half_t>::value)
+      constexpr bool F16 = std::is_same<T, half_t>::value;
+      if constexpr (D == 128 && F16)
         asm volatile(FAL_DQP_ASM_F16 : FAL_DQP_OUTS : FAL_DQP_INS : FAL_DQP_CLOBBERS);
-      else
+      if constexpr (D == 128 && !F16)
         asm volatile(FAL_DQP_ASM_BF16 : FAL_DQP_OUTS : FAL_DQP_INS : FAL_DQP_CLOBBERS);
+      if constexpr (D == 256 && F16)
+        asm volatile(FAL_DQP256_ASM_F16 : FAL_DQP256_OUTS : FAL_DQP256_INS : FAL_DQP256_CLOBBERS);
+      if constexpr (D == 256 && !F16)
+        asm volatile(FAL_DQP256_ASM_BF16 : FAL_DQP256_OUTS : FAL_DQP256_INS : FAL_DQP256_CLOBBERS);
     }
     {
       // dQ^T block g = db*4 + g4 of lane (hh, l32) holds columns 8g + hh*4 .. +3 of row
       // m0 + ws*32 + l32 at ws*kDqOWave + lane*16 + g*kDqOStr; written back row-wise,
-      // each 16-byte store instruction covering 4 whole rows
+      // each 16-byte store instruction covering whole rows
+      constexpr int RPI = 64 / CPR;            // rows per store instruction
       const char* wb = (const char*)smem + ws * kDqOWave;
-      const int cch = lane & 15;
+      const int cch = lane % CPR;
       // a buffer resource over this wave's rows inside the sequence: stores past the end
       // are dropped (no branch, no 64-bit address per store)
       const int wr0 = m0 + ws * 32;
       const __amdgpu_buffer_rsrc_t dqrs =
           make_rsrc((T*)p.dq + (int64_t)b * p.dq_sb + (int64_t)hq * p.dq_sh + (int64_t)(q_off + wr0) * p.dq_ss,
                     (uint32_t)((int64_t)max(min(nq - wr0, 32), 0) * p.dq_ss * 2));
-      const int dvo = ((lane >> 4) * (int)p.dq_ss + cch * 8) * 2;
-      f32x4 a0[8], a1[8];
+      const int dvo = ((lane / CPR) * (int)p.dq_ss + cch * 8) * 2;
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        const int r = jj * 4 + (lane >> 4);
-        a0[jj] = a1[jj] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (ntiles > 0) {
-          a0[jj] = *reinterpret_cast<const f32x4*>(wb + r * 16 + cch * kDqOStr);
-          a1[jj] = *reinterpret_cast<const f32x4*>(wb + (32 + r) * 16 + cch * kDqOStr);
+      for (int j0 = 0; j0 < 32 / RPI; j0 += 8) {
+        f32x4 a0[8], a1[8];
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) {
+          const int r = (j0 + jj) * RPI + lane / CPR;
+          a0[jj] = a1[jj] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (ntiles > 0) {
+            a0[jj] = *reinterpret_cast<const f32x4*>(wb + r * 16 + cch * kDqOStr);
+            a1[jj] = *reinterpret_cast<const f32x4*>(wb + (32 + r) * 16 + cch * kDqOStr);
+          }
         }
-      }
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        V8 h;
+        for (int jj = 0; jj < 8; ++jj) {
+          V8 h;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          h[e] = (T)(a0[jj][e] * p.scale);
-          h[4 + e] = (T)(a1[jj][e] * p.scale);
+          for (int e = 0; e < 4; ++e) {
+            h[e] = (T)(a0[jj][e] * p.scale);
+            h[4 + e] = (T)(a1[jj][e] * p.scale);
+          }
+          buffer_store16(dqrs, dvo + (j0 + jj) * RPI * (int)p.dq_ss * 2, __builtin_bit_cast(u32x4, h));
         }
-        buffer_store16(dqrs, dvo + jj * 4 * (int)p.dq_ss * 2, __builtin_bit_cast(u32x4, h));
       }
     }
     continue;
@@ -1383,18 +1411,19 @@ int bwd_block_n(int d) {
   return split_d(d) ? FAL_BWD2_NW * 16 : kBwdNW * 32;
 }
 
-bool bwd_pipe(int d) { return FAL_BWD_PIPE && d == 128; }
+bool bwd_pipe(int d) { return FAL_BWD_PIPE && (d == 128 || d == 256); }
+int bwd_pipe_bm(int d) { return d == 256 ? pipe_bm<256>() : pipe_bm<128>(); }
 
 template <class T, int D>
 static hipError_t launch_bwd_t(const BwdParams& p, int causal, dim3 grid, hipStream_t st) {
-  if constexpr (D == 128) {
+  if constexpr (D == 128 || D == 256) {
     if (!p.cu_q && p.lsd) {
       const int nkt = cdiv(p.Nk, kPipeBN);
       grid.x = (unsigned)((causal ? (nkt + 1) / 2 : nkt) * p.B * p.Hkv);
       if (causal)
-        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, true>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, true>), grid, dim3(256), 0, st, p);
       else
-        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, false>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, false>), grid, dim3(256), 0, st, p);
       return hipGetLastError();
     }
   }
@@ -1424,7 +1453,7 @@ static hipError_t launch_bwd_d(const BwdParams& p, int causal, dim3 grid, hipStr
 #endif
 constexpr int kDqNW = 4;
 
-bool bwd_split_dq(int d) { return split_d(d) && !fused_d(d); }
+bool bwd_split_dq(int d, bool batched) { return (split_d(d) && !fused_d(d)) || (batched && bwd_pipe(d)); }
 int bwd_dq_block_m(int d) {
   (void)d;
   return kDqNW * 32;
@@ -1434,20 +1463,24 @@ template <class T, int D>
 static hipError_t launch_bwd_dq_t(const BwdParams& p, int causal, dim3 grid, hipStream_t st) {
   if (!p.cu_q && causal && FAL_BWD_DQ_PAIR)
     grid.x = (unsigned)((cdiv(p.Nq, kDqNW * 32) + 1) / 2) * p.B * p.Hq;
-  if constexpr (D == 128) {
+  if constexpr (D == 128 || D == 256) {
     if (!p.cu_q && FAL_BWD_DQ_PIPE) {
+      constexpr int BN = 8192 / D;
       if (causal)
-        hipLaunchKernelGGL((bwd_dq_kernel<T, D, kDqNW, 64, true, true>), grid, dim3(kDqNW * 64), 0, st, p);
+        hipLaunchKernelGGL((bwd_dq_kernel<T, D, kDqNW, BN, true, true>), grid, dim3(kDqNW * 64), 0, st, p);
       else
-        hipLaunchKernelGGL((bwd_dq_kernel<T, D, kDqNW, 64, false, true>), grid, dim3(kDqNW * 64), 0, st, p);
+        hipLaunchKernelGGL((bwd_dq_kernel<T, D, kDqNW, BN, false, true>), grid, dim3(kDqNW * 64), 0, st, p);
       return hipGetLastError();
     }
   }
-  if (causal)
-    hipLaunchKernelGGL((bwd_dq_kernel<T, D, kDqNW, FAL_BWD_DQ_BN, true>), grid, dim3(kDqNW * 64), 0, st, p);
-  else
-    hipLaunchKernelGGL((bwd_dq_kernel<T, D, kDqNW, FAL_BWD_DQ_BN, false>), grid, dim3(kDqNW * 64), 0, st, p);
-  return hipGetLastError();
+  if constexpr (split_d(D)) {
+    if (causal)
+      hipLaunchKernelGGL((bwd_dq_kernel<T, D, kDqNW, FAL_BWD_DQ_BN, true>), grid, dim3(kDqNW * 64), 0, st, p);
+    else
+      hipLaunchKernelGGL((bwd_dq_kernel<T, D, kDqNW, FAL_BWD_DQ_BN, false>), grid, dim3(kDqNW * 64), 0, st, p);
+    return hipGetLastError();
+  }
+  return hipErrorInvalidValue;
 }
 
 template <int D>
@@ -1461,6 +1494,7 @@ hipError_t launch_bwd_dq(const BwdParams& p, int d, int causal, dim3 grid, hipSt
     case 64: return launch_bwd_dq_d<64>(p, causal, grid, st);
     case 96: return launch_bwd_dq_d<96>(p, causal, grid, st);
     case 128: return launch_bwd_dq_d<128>(p, causal, grid, st);
+    case 256: return launch_bwd_dq_d<256>(p, causal, grid, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -92,7 +92,7 @@ struct BwdParams {
   int total_q;        // varlen: rows of the packed Q (row-wise kernels)
   int total_k;        // varlen: rows of the packed K/V
   int bf16;           // element type of every fp16/bf16 tensor: 0 fp16, 1 bf16
-  float* lsd;         // batched head_dim 128: per 64-row tile, -L*log2(e)/c then -D (null: unused)
+  float* lsd;         // batched head_dim 128 and 256: per query tile, -L*log2(e)/c then -D (null: unused)
 };
 
 // KV-cache decode (one query token per sequence).
@@ -163,10 +163,11 @@ hipError_t launch_bwd(const BwdParams& p, int d, int causal, dim3 grid, hipStrea
 hipError_t launch_bwd_pre(const BwdParams& p, int d, int rows_batched, hipStream_t st);
 hipError_t launch_bwd_post(const BwdParams& p, int d, hipStream_t st);
 // head dims whose dQ comes from the query-outer kernel (no fp32 accumulator)
-bool bwd_split_dq(int d);
+bool bwd_split_dq(int d, bool batched);
 int bwd_dq_block_m(int d);
 // batched head_dim d uses bwd_kv_pipe_kernel (workspace holds the lsd array)
 bool bwd_pipe(int d);
+int bwd_pipe_bm(int d);   // its query rows per item
 hipError_t launch_bwd_dq(const BwdParams& p, int d, int causal, dim3 grid, hipStream_t st);
 
 int decode_chunk(int d, int B, int Hkv, int max_seqlen);

@@ -1,6 +1,7 @@
-"""Generates fal_bwd_pipe.inc: the query-tile loop of the head_dim-128 dK/dV kernel
-(bwd_kv_pipe_kernel) as a single inline-asm block, software-pipelined inside one wave
-at one wave per SIMD.
+"""Generates fal_bwd_pipe.inc: the query-tile loop of the head_dim-128 and -256 dK/dV
+kernels (bwd_kv_pipe_kernel) as a single inline-asm block each, software-pipelined inside
+one wave at one wave per SIMD.  Sizes below are head_dim 128's; head_dim 256 differs only
+in what the last paragraph of this text lists.
 
 A workgroup owns 128 keys of one KV head; wave w owns keys kw0 = n0 + 32w .. +31 and
 keeps their K and V fragments in registers (B operands).  It walks the items (query
@@ -39,6 +40,18 @@ Register plan (per lane; one wave per SIMD: 256 VGPRs and 256 AGPRs):
   s[88:89] compare mask, s90..s93 and s95 temporaries, s94 next item to copy
   v0..v103, a128..a191 and s0..s71 are left to the compiler (K and V arrive in AGPRs).
 
+Head dim 256: an item is 32 query rows (one row block), so a Q or dO tile is 16 KB again
+and an item has the same 64 MFMAs with half the exponentials.  dV^T and dK^T take all 256
+AGPRs, K and V arrive in VGPRs (128), and the rest is cut to fit:
+  v[192:223], v[224:255]  item sets: S, dP (16 each)
+  v[160:191]  fragment ring (8 x 4) of both products, and the temporaries where no
+              fragment is in flight
+  v[152:159], v[144:151], v143  QA, TA and LA, moved on by one slot per use (an XOR of the
+              chunk index gives the eight addresses; chunks 16..31 are 256 bytes on)
+  s96/s97     record counts of the tiles' second 16 rows: the copies of rows 16..31 reuse
+              the offsets of rows 0..15 from a base 16 rows on
+  Ls/Dn slots hold 32 + 32 values (256 bytes), copied by one load.
+
 The output is deterministic text, tracked under csrc/gen/; build.py checks the tracked
 file against render() and rewrites it only when asked (--regen).
 """
@@ -62,48 +75,34 @@ DEFAULTS = {
 ADIST, BDIST = 4, 6
 DEFAULT_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "gen", "fal_bwd_pipe.inc")
 
-SET = (128, 192)
-QA = 112
-TA = 120
-LA = 104
-T0, T1, T2, T3 = 108, 109, 110, 111
-AR = 192
-BR = 224
 SM0, SJ, SQF, SQC = 72, 73, 74, 75
 SQ, SD, SL = 76, 80, 84
 SM = 88
 ST0, ST1, ST2, ST3, ST4 = 90, 91, 92, 93, 95
 SF = 94
+SQ2, SD2 = 96, 97
 RSRC_W3 = "0x00020000"
 MEASURE, ABL = False, set()
 
 # ---- operands: (name, constraint, C++ expression) ----
-OUTS = []
-INS = []
-for t in range(8):
-    INS.append((f"K{t}", "a", f"kreg[{t}]"))
-for t in range(8):
-    INS.append((f"V{t}", "a", f"vreg[{t}]"))
-for t in range(8):
-    INS.append((f"qa{t}", "v", f"p_qa[{t}]"))
-for hf in range(2):
-    for db in range(4):
-        INS.append((f"ta{hf}{db}", "v", f"p_ta[{hf}][{db}]"))
-for i in range(4):
-    INS.append((f"qo{i}", "v", f"p_qo[{i}]"))
-for i in range(4):
-    INS.append((f"do{i}", "v", f"p_do[{i}]"))
-INS += [("la", "v", "p_la"), ("lo4", "v", "p_lo4"), ("lo4b", "v", "p_lo4b"), ("lk", "v", "p_lk"),
-        ("olds", "v", "p_olds")]
-INS += [(n, "s", f"p_{n}") for n in (
-    "qb_lo", "qb_hi", "db_lo", "db_hi", "lb_lo", "lb_hi",
-    "qs_lo", "qs_hi", "qw_lo", "qw_hi", "ds_lo", "ds_hi", "dw_lo", "dw_hi", "ldw",
-    "qrb", "drb", "nq", "nqt", "qt0", "nitems", "c", "negc", "kw0", "lbase", "ldbase", "scale")]
-IDX = {name: i for i, (name, _, _) in enumerate(OUTS + INS)}
-
-
-def op(name):
-    return f"%{IDX[name]}"
+def operands(d):
+    f = "a" if d == 128 else "v"
+    ins = [(f"K{t}", f, f"kreg[{t}]") for t in range(d // 16)]
+    ins += [(f"V{t}", f, f"vreg[{t}]") for t in range(d // 16)]
+    if d == 128:
+        ins += [(f"qa{t}", "v", f"p_qa[{t}]") for t in range(8)]
+        ins += [(f"ta{hf}{db}", "v", f"p_ta[{hf}][{db}]") for hf in range(2) for db in range(4)]
+    else:
+        ins += [("qa0", "v", "p_qa[0]"), ("ta0", "v", "p_ta[0][0]")]
+    noff = 4 if d == 128 else 2
+    ins += [(f"qo{i}", "v", f"p_qo[{i}]") for i in range(noff)]
+    ins += [(f"do{i}", "v", f"p_do[{i}]") for i in range(noff)]
+    ins += [("la", "v", "p_la"), ("lo4", "v", "p_lo4")] + ([("lo4b", "v", "p_lo4b")] if d == 128 else [])
+    ins += [("lk", "v", "p_lk"), ("olds", "v", "p_olds")]
+    names = ("qb_lo", "qb_hi", "db_lo", "db_hi", "lb_lo", "lb_hi",
+             "qs_lo", "qs_hi", "qw_lo", "qw_hi", "ds_lo", "ds_hi", "dw_lo", "dw_hi", "ldw",
+             "qrb", "drb", "nq", "nqt", "qt0", "nitems", "c", "negc", "kw0", "lbase", "ldbase", "scale")
+    return ins + [(n, "s", f"p_{n}") for n in names]
 
 
 def v(n):
@@ -119,12 +118,32 @@ def ar(n, k):
 
 
 class Emitter:
-    def __init__(self, bf16):
+    def __init__(self, d, bf16):
         self.lines = []
+        self.d, self.ks, self.db = d, d // 16, d // 32
+        self.nrb = 256 // d                 # 32-row blocks per item
+        self.rowb = 2 * d                   # bytes of a tile row
+        self.ldb = 256 * self.nrb           # bytes of an item's Ls and Dn
+        if d == 128:
+            self.SET, self.AR, self.BR, self.ring = (128, 192), 192, 224, "a"
+            self.QA, self.TA, self.LA, self.T, self.vlow = 112, 120, 104, (108, 109, 110, 111), 104
+            self.nacc = 128
+        else:
+            self.SET, self.AR, self.BR, self.ring = (192, 224), 160, 160, "v"
+            self.QA, self.TA, self.LA, self.T, self.vlow = 152, 144, 143, (160, 161, 162, 163), 143
+            self.nacc = 256
+        self.idx = {name: i for i, (name, _, _) in enumerate(operands(d))}
         self.mf = "v_mfma_f32_32x32x16_bf16" if bf16 else "v_mfma_f32_32x32x16_f16"
         self.cvt = "v_cvt_pk_bf16_f32" if bf16 else "v_cvt_pk_f16_f32"
         self.nlabel = 0
         self.skip_mf = False
+
+    def op(self, name):
+        return f"%{self.idx[name]}"
+
+    def fr(self, n, k):
+        """k registers of the fragment ring's file from n"""
+        return f"{self.ring}[{n}:{n + k - 1}]"
 
     def e(self, s):
         self.lines.append(s)
@@ -149,9 +168,9 @@ class Emitter:
         the quarter-rate exponentials spread between the MFMAs: the multiply by c runs
         two elements ahead, dS one element behind its exponential, and a pair is packed
         once both of its dS products are done."""
-        s0 = SET[par] + 16 * rb
-        d0 = SET[par] + 32 + 16 * rb
-        muls = [f"v_mul_f32 {v(s0 + j)}, {op('c')}, {v(s0 + j)}" for j in range(16)]
+        s0 = self.SET[par] + 16 * rb
+        d0 = s0 + 16 * self.nrb
+        muls = [f"v_mul_f32 {v(s0 + j)}, {self.op('c')}, {v(s0 + j)}" for j in range(16)]
         ops = muls[:2]
         for st in range(19):
             if st + 2 < 16:
@@ -171,21 +190,21 @@ class Emitter:
     def a_prod(self, par):
         """A: S and dP of an item into SET[par] from the slot whose addresses are in QA/LA."""
         reads, mf = [], []
-        base = SET[par]
-        for blk in range(4):                      # S rb0, S rb1, dP rb0, dP rb1
+        base, nblk = self.SET[par], 2 * self.nrb
+        for blk in range(nblk):                   # S of each row block, then dP of each
             for g4 in range(4):
-                off = (256 if blk >= 2 else 0) + (blk % 2) * 128 + g4 * 32
-                reads.append(f"ds_read_b128 {vr(base + 16 * blk + 4 * g4, 4)}, {v(LA)} offset:{off}")
+                off = (self.ldb // 2 if blk >= self.nrb else 0) + (blk % self.nrb) * 128 + g4 * 32
+                reads.append(f"ds_read_b128 {vr(base + 16 * blk + 4 * g4, 4)}, {v(self.LA)} offset:{off}")
         k = 0
-        for t in range(8):
-            for blk in range(4):
-                rb = blk % 2
-                off = (DOFF if blk >= 2 else 0) + rb * 8192
-                slot = AR + 4 * (k % 8)
-                reads.append(f"ds_read_b128 {ar(slot, 4)}, {v(QA + t)} offset:{off}")
+        for t in range(self.ks):
+            for blk in range(nblk):
+                rb = blk % self.nrb
+                off = (DOFF if blk >= self.nrb else 0) + rb * 8192 + (t // 8) * 256
+                slot = self.AR + 4 * (k % 8)
+                reads.append(f"ds_read_b128 {self.fr(slot, 4)}, {v(self.QA + t % 8)} offset:{off}")
                 acc = vr(base + 16 * blk, 16)
-                bop = op(f"K{t}") if blk < 2 else op(f"V{t}")
-                mf.append((f"{self.mf} {acc}, {ar(slot, 4)}, {bop}, {acc}", 16 + k))
+                bop = self.op(f"K{t}") if blk < self.nrb else self.op(f"V{t}")
+                mf.append((f"{self.mf} {acc}, {self.fr(slot, 4)}, {bop}, {acc}", 4 * nblk + k))
                 k += 1
         return reads, mf
 
@@ -193,19 +212,20 @@ class Emitter:
         """B: dV^T += dO^T P and dK^T += Q^T dS of the item packed in SET[par], from the
         slot whose transposed-read addresses are in TA."""
         reads, mf = [], []
-        base = SET[par]
+        base = self.SET[par]
         k = 0
-        for ks in range(4):
+        for ks in range(2 * self.nrb):
             rb, t2 = ks // 2, ks % 2
-            for db in range(4):
+            for db in range(self.db):
                 for which in range(2):               # dV, dK
-                    slot = BR + 4 * (k % 8)
-                    off = (DOFF if which == 0 else 0) + ks * 4096
+                    slot = self.BR + 4 * (k % 8)
+                    off = (DOFF if which == 0 else 0) + ks * 16 * self.rowb + (db // 4) * 256
                     for hf in range(2):
-                        reads.append(f"ds_read_b64_tr_b16 {ar(slot + 2 * hf, 2)}, {v(TA + hf * 4 + db)} offset:{off}")
-                    acc = ar(which * 64 + db * 16, 16)
-                    bop = vr(base + (32 if which else 0) + 16 * rb + 4 * t2, 4)
-                    mf.append((f"{self.mf} {acc}, {ar(slot, 4)}, {bop}, {acc}", 2 * k + 1))
+                        reads.append(f"ds_read_b64_tr_b16 {self.fr(slot + 2 * hf, 2)}, "
+                                     f"{v(self.TA + hf * 4 + db % 4)} offset:{off}")
+                    acc = ar(which * (self.nacc // 2) + db * 16, 16)
+                    bop = vr(base + (16 * self.nrb if which else 0) + 16 * rb + 4 * t2, 4)
+                    mf.append((f"{self.mf} {acc}, {self.fr(slot, 4)}, {bop}, {acc}", 2 * k + 1))
                     k += 1
         return reads, mf
 
@@ -248,43 +268,69 @@ class Emitter:
         return [f"s_add_u32 s{ST0}, s{SJ}, {delta % NBUF}", f"s_and_b32 s{ST0}, s{ST0}, {NBUF - 1}",
                 f"s_lshl_b32 s{ST1}, s{ST0}, 9", f"s_lshl_b32 s{ST0}, s{ST0}, 15"]
 
+    def step_addr(self, delta, moves):
+        """Head dim 256: address registers moved on by one slot, to that of item i + delta
+        (`moves`: (bytes of a slot, registers))."""
+        ops = [f"s_add_u32 s{ST0}, s{SJ}, {delta % NBUF}", f"s_and_b32 s{ST0}, s{ST0}, {NBUF - 1}"]
+        for size, regs in moves:
+            ops += [f"s_movk_i32 s{ST1}, {size}" if size < 32768 else f"s_mov_b32 s{ST1}, {size}",
+                    f"s_cmp_eq_u32 s{ST0}, 0", f"s_cselect_b32 s{ST1}, {-(NBUF - 1) * size}, s{ST1}"]
+            ops += [f"v_add_u32 {v(r)}, s{ST1}, {v(r)}" for r in regs]
+        return ops
+
     def a_addr_ops(self):
         """QA/LA for the slot of item i+1"""
-        return (self.slot_addr(1) + [f"v_add_u32 {v(QA + t)}, s{ST0}, {op(f'qa{t}')}" for t in range(8)] +
-                [f"v_add_u32 {v(LA)}, s{ST1}, {op('la')}"])
+        if self.d == 256:
+            return self.step_addr(1, ((SLOT, range(self.QA, self.QA + 8)), (512, (self.LA,))))
+        op = self.op
+        return (self.slot_addr(1) + [f"v_add_u32 {v(self.QA + t)}, s{ST0}, {op(f'qa{t}')}" for t in range(8)] +
+                [f"v_add_u32 {v(self.LA)}, s{ST1}, {op('la')}"])
 
     def b_addr_ops(self):
         """TA for the slot of item i-1"""
-        return self.slot_addr(-1) + [f"v_add_u32 {v(TA + hf * 4 + db)}, s{ST0}, {op(f'ta{hf}{db}')}"
+        if self.d == 256:
+            return self.step_addr(-1, ((SLOT, range(self.TA, self.TA + 8)),))
+        op = self.op
+        return self.slot_addr(-1) + [f"v_add_u32 {v(self.TA + hf * 4 + db)}, s{ST0}, {op(f'ta{hf}{db}')}"
                                      for hf in range(2) for db in range(4)]
 
     def dma_groups(self):
         """Copy of item s94 (query tile s74) into slot s94 % 4: 4 + 4 Q/dO loads of 1 KB
         per wave, the Ls and Dn rows; then the copy state advances one item."""
+        op, bm = self.op, 32 * self.nrb
         g = [[
-            # record counts: the tile's rows inside the sequence (0..64) times the row
+            # record counts: the tile's rows inside the sequence (0..64, or 0..32) times the row
             # stride; items past the last one copy nothing (read as zeros)
-            f"s_lshl_b32 s{ST2}, s{SQF}, 6", f"s_sub_i32 s{ST2}, {op('nq')}, s{ST2}",
-            f"s_max_i32 s{ST2}, s{ST2}, 0", f"s_min_i32 s{ST2}, s{ST2}, 64",
+            f"s_lshl_b32 s{ST2}, s{SQF}, {bm.bit_length() - 1}", f"s_sub_i32 s{ST2}, {op('nq')}, s{ST2}",
+            f"s_max_i32 s{ST2}, s{ST2}, 0", f"s_min_i32 s{ST2}, s{ST2}, {bm}",
             f"s_cmp_lt_i32 s{SF}, {op('nitems')}",
-            f"s_cselect_b32 s{ST2}, s{ST2}, 0", f"s_cselect_b32 s{SL + 2}, 0x200, 0",
-            f"s_mul_i32 s{SQ + 2}, s{ST2}, {op('qrb')}", f"s_mul_i32 s{SD + 2}, s{ST2}, {op('drb')}",
+            f"s_cselect_b32 s{ST2}, s{ST2}, 0", f"s_cselect_b32 s{SL + 2}, {hex(self.ldb)}, 0",
+            f"s_mul_i32 s{SQ + 2}, s{ST2}, {op('qrb')}", f"s_mul_i32 s{SD + 2}, s{ST2}, {op('drb')}"] + ([
+            f"s_sub_i32 s{ST2}, s{ST2}, 16", f"s_max_i32 s{ST2}, s{ST2}, 0",
+            f"s_mul_i32 s{SQ2}, s{ST2}, {op('qrb')}", f"s_mul_i32 s{SD2}, s{ST2}, {op('drb')}"]
+                if self.d == 256 else []) + [
             f"s_and_b32 s{ST3}, s{SF}, {NBUF - 1}", f"s_lshl_b32 s{ST2}, s{ST3}, 15",
             f"s_add_u32 s{ST2}, s{ST2}, {op('lbase')}",
             f"s_lshl_b32 s{ST3}, s{ST3}, 9", f"s_add_u32 s{ST3}, s{ST3}, {op('ldbase')}"]]
         for part, rs, vo, base in (("q", SQ, "qo", 0), ("d", SD, "do", DOFF)):
             for i in range(4):
+                if self.d == 256 and i == 2:         # rows 16..31: same offsets, base 16 rows on
+                    rb, r2 = (op("qrb"), SQ2) if part == "q" else (op("drb"), SD2)
+                    g.append([f"s_lshl_b32 s{ST4}, {rb}, 4", f"s_add_u32 s{rs}, s{rs}, s{ST4}",
+                              f"s_addc_u32 s{rs + 1}, s{rs + 1}, 0", f"s_mov_b32 s{rs + 2}, s{r2}"])
+                o = op(f"{vo}{i if self.d == 128 else i % 2}")
                 g.append([f"s_add_u32 m0, s{ST2}, {base + i * 4096}", "s_nop 0"] + ([] if "nodma" in ABL else
-                          [f"buffer_load_dwordx4 {op(f'{vo}{i}')}, s[{rs}:{rs + 3}], 0 offen lds"]))
+                          [f"buffer_load_dwordx4 {o}, s[{rs}:{rs + 3}], 0 offen lds"]))
         g.append([f"s_mov_b32 m0, s{ST3}", "s_nop 0"] + ([] if "nodma" in ABL else
                  [f"buffer_load_dword {op('lo4')}, s[{SL}:{SL + 3}], 0 offen lds"]))
-        g.append([f"s_add_u32 m0, s{ST3}, 256", "s_nop 0"] + ([] if "nodma" in ABL else
-                 [f"buffer_load_dword {op('lo4b')}, s[{SL}:{SL + 3}], 0 offen lds"]))
+        if self.d == 128:
+            g.append([f"s_add_u32 m0, s{ST3}, 256", "s_nop 0"] + ([] if "nodma" in ABL else
+                     [f"buffer_load_dword {op('lo4b')}, s[{SL}:{SL + 3}], 0 offen lds"]))
         g.append([
             f"s_add_u32 s{SQF}, s{SQF}, 1", f"s_cmp_eq_u32 s{SQF}, {op('nqt')}",
             f"s_cselect_b32 s{ST0}, {op('qw_lo')}, {op('qs_lo')}", f"s_cselect_b32 s{ST1}, {op('qw_hi')}, {op('qs_hi')}",
             f"s_cselect_b32 s{ST2}, {op('dw_lo')}, {op('ds_lo')}", f"s_cselect_b32 s{ST3}, {op('dw_hi')}, {op('ds_hi')}",
-            f"s_cselect_b32 s{ST4}, {op('ldw')}, 0x200", f"s_cselect_b32 s{SQF}, {op('qt0')}, s{SQF}",
+            f"s_cselect_b32 s{ST4}, {op('ldw')}, {hex(self.ldb)}", f"s_cselect_b32 s{SQF}, {op('qt0')}, s{SQF}",
             f"s_add_u32 s{SQ}, s{SQ}, s{ST0}", f"s_addc_u32 s{SQ + 1}, s{SQ + 1}, s{ST1}",
             f"s_add_u32 s{SD}, s{SD}, s{ST2}", f"s_addc_u32 s{SD + 1}, s{SD + 1}, s{ST3}",
             f"s_add_u32 s{SL}, s{SL}, s{ST4}", f"s_addc_u32 s{SL + 1}, s{SL + 1}, 0",
@@ -299,24 +345,24 @@ class Emitter:
     def mask_block(self, par):
         """Scores of item i (SET[par]) set to negc where key > row, for each row block
         that straddles this wave's keys (kw0 + 31 > first row of the block)."""
-        e = self.e
-        e(f"s_lshl_b32 s{ST0}, s{SQC}, 6")
+        e, op, (t0, _, _, t3) = self.e, self.op, self.T
+        e(f"s_lshl_b32 s{ST0}, s{SQC}, {4 + self.nrb}")
         e(f"s_sub_i32 s{ST0}, {op('kw0')}, s{ST0}")              # kw0 - q0
         done = []
-        for rb in range(2):
+        for rb in range(self.nrb):
             skip = self.label(f"nomask{rb}_")
             e(f"s_sub_i32 s{ST1}, s{ST0}, {32 * rb}")
             e(f"s_cmp_gt_i32 s{ST1}, -31")
             e(f"s_cbranch_scc0 {skip}")
             e("s_nop 7")
-            e(f"v_mov_b32 {v(T3)}, {op('negc')}")
+            e(f"v_mov_b32 {v(t3)}, {op('negc')}")
             # element j: key - row = (kw0 - q0 - 32rb + l32 - 4hh) - (8*(j/4) + j%4)
-            e(f"v_add_u32 {v(T0)}, s{ST1}, {op('lk')}")
+            e(f"v_add_u32 {v(t0)}, s{ST1}, {op('lk')}")
             for j in range(16):
                 cst = 8 * (j // 4) + j % 4
-                r = SET[par] + 16 * rb + j
-                e(f"v_cmp_lt_i32 vcc, {cst}, {v(T0)}")
-                e(f"v_cndmask_b32 {v(r)}, {v(r)}, {v(T3)}, vcc")
+                r = self.SET[par] + 16 * rb + j
+                e(f"v_cmp_lt_i32 vcc, {cst}, {v(t0)}")
+                e(f"v_cndmask_b32 {v(r)}, {v(r)}, {v(t3)}, vcc")
             e(f"{skip}:")
             done.append(skip)
 
@@ -329,6 +375,9 @@ class Emitter:
         if has_a:
             self.es(self.a_addr_ops())
         v0 = self.grad_ops(par, 0) if has_v else []
+        v1 = self.grad_ops(par, 1) if has_v and self.nrb == 2 else []
+        if self.nrb == 1:                  # one row block: half beside either product
+            v0, v1 = v0[:len(v0) // 2], v0[len(v0) // 2:]
         if has_b:
             reads, mf = self.b_prod(par ^ 1)
             self.skip_mf = "nob" in ABL
@@ -337,10 +386,9 @@ class Emitter:
         else:
             self.dma()
             self.es(v0)
-        e("s_waitcnt vmcnt(10)")
+        e(f"s_waitcnt vmcnt({self.nload})")
         if "nobar" not in ABL:
             e("s_barrier")
-        v1 = self.grad_ops(par, 1) if has_v else []
         if has_a:
             reads, mf = self.a_prod(par ^ 1)
             self.skip_mf = "noa" in ABL
@@ -350,8 +398,13 @@ class Emitter:
             self.es(v1)
         e(f"s_branch {lbl_next}")
 
+    @property
+    def nload(self):
+        """buffer->LDS loads of one item"""
+        return 10 if self.d == 128 else 9
+
     def program(self):
-        e = self.e
+        e, op = self.e, self.op
         lbl_disp, lbl_next, lbl_out = "disp_%=", "next_%=", "out_%="
         e("s_nop 7")
         e(f"s_mov_b32 s{SM0}, m0")
@@ -364,17 +417,31 @@ class Emitter:
         e(f"s_mov_b32 s{SF}, 0")
         e(f"s_mov_b32 s{SQF}, {op('qt0')}")
         e(f"s_mov_b32 s{SQC}, {op('qt0')}")
-        for a in range(128):
+        for a in range(self.nacc):
             e(f"v_accvgpr_write_b32 a{a}, 0")
         self.dma()
         self.dma()
-        e("s_waitcnt vmcnt(10)")
+        e(f"s_waitcnt vmcnt({self.nload})")
         e("s_barrier")
         # A(0) into set 0 from slot 0
         e(f"s_mov_b32 s{ST0}, 0")
         e(f"s_mov_b32 s{ST1}, 0")
-        self.es([f"v_add_u32 {v(QA + t)}, s{ST0}, {op(f'qa{t}')}" for t in range(8)])
-        e(f"v_add_u32 {v(LA)}, s{ST1}, {op('la')}")
+        if self.d == 128:
+            self.es([f"v_add_u32 {v(self.QA + t)}, s{ST0}, {op(f'qa{t}')}" for t in range(8)])
+            e(f"v_add_u32 {v(self.LA)}, s{ST1}, {op('la')}")
+        else:
+            # chunk 2t + hh is an XOR of 32 t bytes away; TA starts at the slot before the first
+            # (row + 8 is 4096 bytes on, its swizzle an XOR of 32)
+            self.es([f"v_xor_b32 {v(self.QA + t)}, {32 * t}, {op('qa0')}" for t in range(8)])
+            e(f"v_mov_b32 {v(self.LA)}, {op('la')}")
+            e(f"s_mov_b32 s{ST0}, {(NBUF - 1) * SLOT}")
+            for hf in range(2):
+                for db in range(4):
+                    r = v(self.TA + hf * 4 + db)
+                    e(f"v_xor_b32 {r}, {64 * db + 32 * hf}, {op('ta0')}")
+                    e(f"v_add_u32 {r}, s{ST0}, {r}")
+                    if hf:
+                        e(f"v_add_u32 {r}, 4096, {r}")
         reads, mf = self.a_prod(0)
         self.interleave(reads, mf, ADIST)
 
@@ -427,18 +494,20 @@ class Emitter:
         e("s_nop 15")
         e("s_waitcnt vmcnt(0) lgkmcnt(0)")
         e("s_barrier")
+        t0, t1, t2, t3 = self.T
         for which in range(2):
-            for db in range(4):
+            for db in range(self.db):
                 for g4 in range(4):
-                    a0 = which * 64 + db * 16 + 4 * g4
+                    a0 = which * (self.nacc // 2) + db * 16 + 4 * g4
                     for x in range(4):
-                        e(f"v_accvgpr_read_b32 {v(T0 + x)}, a{a0 + x}")
+                        e(f"v_accvgpr_read_b32 {v(t0 + x)}, a{a0 + x}")
                     if which:
                         for x in range(4):
-                            e(f"v_mul_f32 {v(T0 + x)}, {op('scale')}, {v(T0 + x)}")
-                    e(f"{self.cvt} {v(T0)}, {v(T0)}, {v(T1)}")
-                    e(f"{self.cvt} {v(T1)}, {v(T2)}, {v(T3)}")
-                    e(f"ds_write_b64 {op('olds')}, {vr(T0, 2)} offset:{which * 16 * OSTR + (db * 4 + g4) * OSTR}")
+                            e(f"v_mul_f32 {v(t0 + x)}, {op('scale')}, {v(t0 + x)}")
+                    e(f"{self.cvt} {v(t0)}, {v(t0)}, {v(t1)}")
+                    e(f"{self.cvt} {v(t1)}, {v(t2)}, {v(t3)}")
+                    off = which * 4 * self.db * OSTR + (db * 4 + g4) * OSTR
+                    e(f"ds_write_b64 {op('olds')}, {vr(t0, 2)} offset:{off}")
         e("s_waitcnt lgkmcnt(0)")
         e(f"s_mov_b32 m0, s{SM0}")
         return self.lines
@@ -472,20 +541,22 @@ def render(knobs=None, measure=False):
 
 def _render():
     out = ["// Generated by gen_bwd_pipe.py; do not edit.", "#pragma once", ""]
-    for bf16, name in ((False, "FAL_BWDP_ASM_F16"), (True, "FAL_BWDP_ASM_BF16")):
-        lines = Emitter(bf16).program()
-        out.append(f"#define {name} \\")
-        for ln in lines:
-            out.append(f'  "{ln}\\n" \\')
+    for d, pre in ((128, "FAL_BWDP"), (256, "FAL_BWDP256")):
+        for bf16, name in ((False, "F16"), (True, "BF16")):
+            em = Emitter(d, bf16)
+            lines = em.program()
+            out.append(f"#define {pre}_ASM_{name} \\")
+            for ln in lines:
+                out.append(f'  "{ln}\\n" \\')
+            out.append("")
+        ins = ", ".join(f'"{c}"({x})' for _, c, x in operands(d))
+        clob = ", ".join([f'"v{i}"' for i in range(em.vlow, 256)] + [f'"a{i}"' for i in range(0, em.nacc)] +
+                         ([f'"a{i}"' for i in range(em.AR, 256)] if em.ring == "a" else []) +
+                         [f'"s{i}"' for i in range(72, 100)] + ['"vcc"', '"scc"', '"memory"'])
+        out.append(f"#define {pre}_OUTS")
+        out.append(f"#define {pre}_INS {ins}")
+        out.append(f"#define {pre}_CLOBBERS {clob}")
         out.append("")
-    ins = ", ".join(f'"{c}"({x})' for _, c, x in INS)
-    clob = ", ".join([f'"v{i}"' for i in range(104, 256)] + [f'"a{i}"' for i in range(0, 128)] +
-                     [f'"a{i}"' for i in range(AR, 256)] + [f'"s{i}"' for i in range(72, 100)] +
-                     ['"vcc"', '"scc"', '"memory"'])
-    out.append("#define FAL_BWDP_OUTS")
-    out.append(f"#define FAL_BWDP_INS {ins}")
-    out.append(f"#define FAL_BWDP_CLOBBERS {clob}")
-    out.append("")
     return "\n".join(out)
 
 

@@ -1,6 +1,7 @@
-"""Generates fal_dq_pipe.inc: the key-tile loop of the head_dim-128 dQ kernel
-(bwd_dq_kernel with PIPE) as a single inline-asm block, software-pipelined inside one
-wave at one wave per SIMD.
+"""Generates fal_dq_pipe.inc: the key-tile loop of the head_dim-128 and -256 dQ kernels
+(bwd_dq_kernel with PIPE) as a single inline-asm block each, software-pipelined inside one
+wave at one wave per SIMD.  Sizes below are head_dim 128's; head_dim 256 differs only in
+what the last paragraph of this text lists.
 
 A wave owns 32 query rows of one query head; their Q and dO fragments stay in
 registers (B operands), with the row's log2-domain LSE (as -L2) and D in one VGPR
@@ -33,6 +34,12 @@ Register plan (per lane; one wave per SIMD):
   s98/s99 temporaries
   v0..v91, a64..a191 and s0..s83 are left to the compiler (Q and dO arrive in AGPRs).
 
+Head dim 256: a tile is 32 keys (one key block), 16 KB per K or V tile again, and has the
+same 48 MFMAs with half the exponentials.  dQ^T takes a[0:127] and Q and dO the other 128
+AGPRs, so the rings are v[144:175] and v[112:143], the sets v[192:223] and v[224:255]
+(S^T, dP^T), -D v[176:191], the addresses v[104:111] and v[96:103], the temporaries
+v[92:95].  Chunks 16..31 of a row are 256 bytes on.
+
 The output is deterministic text, tracked under csrc/gen/; build.py checks the tracked
 file against render() and rewrites it only when asked (--regen).
 """
@@ -52,47 +59,27 @@ ADIST, QDIST = 4, 6
 MEASURE = False
 DEFAULT_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "gen", "fal_dq_pipe.inc")
 
-SET = (128, 192)
-DN = 92             # v[92:107]: -D in every register (the dP^T accumulators' start)
-KC = 112
-VC = 120
-T0, T1, T2, T3 = 108, 109, 110, 111
-AR = 192
-BR = 224
 SM, SM0, SR = 84, 86, 87
 SK, SV = 88, 92
 SJ, SD, ST, ST2 = 96, 97, 98, 99
 NEG_INF = "0xff800000"
 
-OUTS = []
-INS = []
-for t in range(8):
-    INS.append((f"Q{t}", "a", f"qreg[{t}]"))
-for t in range(8):
-    INS.append((f"O{t}", "a", f"doreg[{t}]"))
-for i in range(4):
-    INS.append((f"kvo{i}", "v", f"kvo[{i}]"))
-for i in range(4):
-    INS.append((f"vvo{i}", "v", f"vvo[{i}]"))
-for t in range(8):
-    INS.append((f"ka{t}", "v", f"p_ka[{t}]"))
-for hf in range(2):
-    for db in range(4):
-        INS.append((f"ta{hf}{db}", "v", f"p_ta[{hf}][{db}]"))
-INS += [("row", "v", "p_row"), ("hh4", "v", "p_hh4"), ("olds", "v", "p_olds"), ("nl", "v", "p_nl"),
-        ("dl", "v", "p_dl")]
-for i in range(4):
-    INS.append((f"kr{i}", "s", f"pk_rs[{i}]"))
-for i in range(4):
-    INS.append((f"vr{i}", "s", f"pv_rs[{i}]"))
-INS += [("c", "s", "p_c"), ("negc", "s", "p_negc"), ("jend", "s", "p_jend"), ("jl", "s", "p_jl"),
-        ("wrow", "s", "p_wrow"), ("nk", "s", "p_nk"), ("ktb", "s", "p_ktb"), ("vtb", "s", "p_vtb"),
-        ("krb", "s", "p_krb"), ("vrb", "s", "p_vrb"), ("rows", "s", "p_rows"), ("lbase", "s", "p_lbase")]
-IDX = {name: i for i, (name, _, _) in enumerate(OUTS + INS)}
 
-
-def op(name):
-    return f"%{IDX[name]}"
+def operands(d):
+    """(name, constraint, C++ expression) of the block's inputs."""
+    ins = [(f"Q{t}", "a", f"qreg[{t}]") for t in range(d // 16)]
+    ins += [(f"O{t}", "a", f"doreg[{t}]") for t in range(d // 16)]
+    ins += [(f"kvo{i}", "v", f"kvo[{i}]") for i in range(4)]
+    ins += [(f"vvo{i}", "v", f"vvo[{i}]") for i in range(4)]
+    ins += [(f"ka{t}", "v", f"p_ka[{t}]") for t in range(8)]
+    ins += [(f"ta{hf}{db}", "v", f"p_ta[{hf}][{db}]") for hf in range(2) for db in range(4)]
+    ins += [("row", "v", "p_row"), ("hh4", "v", "p_hh4"), ("olds", "v", "p_olds"), ("nl", "v", "p_nl"),
+            ("dl", "v", "p_dl")]
+    ins += [(f"kr{i}", "s", f"pk_rs[{i}]") for i in range(4)]
+    ins += [(f"vr{i}", "s", f"pv_rs[{i}]") for i in range(4)]
+    return ins + [("c", "s", "p_c"), ("negc", "s", "p_negc"), ("jend", "s", "p_jend"), ("jl", "s", "p_jl"),
+                  ("wrow", "s", "p_wrow"), ("nk", "s", "p_nk"), ("ktb", "s", "p_ktb"), ("vtb", "s", "p_vtb"),
+                  ("krb", "s", "p_krb"), ("vrb", "s", "p_vrb"), ("rows", "s", "p_rows"), ("lbase", "s", "p_lbase")]
 
 
 def v(n):
@@ -108,10 +95,29 @@ def ar(n, k):
 
 
 class Emitter:
-    def __init__(self, bf16):
+    def __init__(self, d, bf16):
         self.lines = []
+        self.ks, self.db = d // 16, d // 32
+        self.nkb = 256 // d                 # 32-key blocks per tile
+        self.bn = 32 * self.nkb
+        self.rowb = 2 * d                   # bytes of a tile row
+        self.nacc = d // 2
+        if d == 128:
+            self.SET, self.DN, self.KC, self.VC, self.T = (128, 192), 92, 112, 120, (108, 109, 110, 111)
+            self.AR, self.BR, self.ring, self.vlow = 192, 224, "a", 92
+        else:
+            self.SET, self.DN, self.KC, self.VC, self.T = (192, 224), 176, 104, 96, (92, 93, 94, 95)
+            self.AR, self.BR, self.ring, self.vlow = 144, 112, "v", 92
+        self.idx = {name: i for i, (name, _, _) in enumerate(operands(d))}
         self.mf = "v_mfma_f32_32x32x16_bf16" if bf16 else "v_mfma_f32_32x32x16_f16"
         self.cvt = "v_cvt_pk_bf16_f32" if bf16 else "v_cvt_pk_f16_f32"
+
+    def op(self, name):
+        return f"%{self.idx[name]}"
+
+    def fr(self, n, k):
+        """k registers of the fragment rings' file from n"""
+        return f"{self.ring}[{n}:{n + k - 1}]"
 
     def e(self, s):
         self.lines.append(s)
@@ -126,8 +132,9 @@ class Emitter:
         dS = P*(dP - D) (the dP^T accumulator started at -D), dS packed in place (pair k
         into register k).  Streamed so the exponentials spread between the MFMAs: the FMA runs two elements ahead,
         dS one element behind its exponential, a pair is packed after its second dS."""
-        s0 = SET[par] + 16 * kb
-        d0 = SET[par] + 32 + 16 * kb
+        op = self.op
+        s0 = self.SET[par] + 16 * kb
+        d0 = s0 + 16 * self.nkb
         fmas = [f"v_fma_f32 {v(s0 + j)}, {v(s0 + j)}, {op('c')}, {op('nl')}" for j in range(16)]
         ops = fmas[:2]
         for st in range(19):
@@ -149,17 +156,19 @@ class Emitter:
                 f"s_lshl_b32 {dst}, {dst}, 15"]
 
     def kcur_ops(self, sreg):
-        return [f"v_add_u32 {v(KC + t)}, {sreg}, {op(f'ka{t}')}" for t in range(8)]
+        return [f"v_add_u32 {v(self.KC + t)}, {sreg}, {self.op(f'ka{t}')}" for t in range(8)]
 
     def tcur_ops(self, sreg):
-        return [f"v_add_u32 {v(VC + hf * 4 + db)}, {sreg}, {op(f'ta{hf}{db}')}" for hf in range(2) for db in range(4)]
+        return [f"v_add_u32 {v(self.VC + hf * 4 + db)}, {sreg}, {self.op(f'ta{hf}{db}')}"
+                for hf in range(2) for db in range(4)]
 
     def dma_groups(self):
         """Copy of tile s97 into its slot (8 buffer->LDS loads), then the copy resources
         advance one tile (rows past the copy range read as zeros)."""
+        op = self.op
         groups = [[f"s_and_b32 s{ST}, s{SD}, {NBUF - 1}", f"s_lshl_b32 s{ST}, s{ST}, 15",
                    f"s_add_u32 s{ST}, s{ST}, {op('lbase')}",
-                   f"s_max_i32 s{SK + 2}, s{SR}, 0", f"s_min_i32 s{SK + 2}, s{SK + 2}, 64",
+                   f"s_max_i32 s{SK + 2}, s{SR}, 0", f"s_min_i32 s{SK + 2}, s{SK + 2}, {self.bn}",
                    f"s_mul_i32 s{SV + 2}, s{SK + 2}, {op('vrb')}", f"s_mul_i32 s{SK + 2}, s{SK + 2}, {op('krb')}"]]
         for part, rs, vo in (("k", SK, "kvo"), ("v", SV, "vvo")):
             for i in range(4):
@@ -169,7 +178,7 @@ class Emitter:
         groups.append([
             f"s_add_u32 s{SK}, s{SK}, {op('ktb')}", f"s_addc_u32 s{SK + 1}, s{SK + 1}, 0",
             f"s_add_u32 s{SV}, s{SV}, {op('vtb')}", f"s_addc_u32 s{SV + 1}, s{SV + 1}, 0",
-            f"s_sub_i32 s{SR}, s{SR}, 64",
+            f"s_sub_i32 s{SR}, s{SR}, {self.bn}",
             f"s_add_u32 s{SD}, s{SD}, 1"])
         return groups
 
@@ -182,15 +191,16 @@ class Emitter:
         into SET[par]."""
         reads, mf = [], []
         k = 0
-        for t in range(8):
-            for kb in range(2):
+        for t in range(self.ks):
+            for kb in range(self.nkb):
                 for which in range(2):          # S (K, Q), dP (V, dO)
-                    slot = AR + 4 * (k % 8)
-                    reads.append(f"ds_read_b128 {ar(slot, 4)}, {v(KC + t)} offset:{(VOFF if which else 0) + kb * 8192}")
-                    acc = vr(SET[par] + 32 * which + 16 * kb, 16)
-                    c = acc if t else (vr(DN, 16) if which else "0")
-                    bop = op(f"O{t}") if which else op(f"Q{t}")
-                    mf.append((f"{self.mf} {acc}, {ar(slot, 4)}, {bop}, {c}", k))
+                    slot = self.AR + 4 * (k % 8)
+                    off = (VOFF if which else 0) + kb * 8192 + (t // 8) * 256
+                    reads.append(f"ds_read_b128 {self.fr(slot, 4)}, {v(self.KC + t % 8)} offset:{off}")
+                    acc = vr(self.SET[par] + 16 * self.nkb * which + 16 * kb, 16)
+                    c = acc if t else (vr(self.DN, 16) if which else "0")
+                    bop = self.op(f"O{t}") if which else self.op(f"Q{t}")
+                    mf.append((f"{self.mf} {acc}, {self.fr(slot, 4)}, {bop}, {c}", k))
                     k += 1
         return reads, mf
 
@@ -198,15 +208,16 @@ class Emitter:
         """dQ^T += K^T dS^T of the tile whose dS^T is packed in SET[par], K^T addresses in VC."""
         reads, mf = [], []
         k = 0
-        for ks in range(4):
+        for ks in range(2 * self.nkb):
             kb, t2 = ks // 2, ks % 2
-            for db in range(4):
-                slot = BR + 4 * (k % 8)
+            for db in range(self.db):
+                slot = self.BR + 4 * (k % 8)
                 for hf in range(2):
-                    reads.append(f"ds_read_b64_tr_b16 {ar(slot + 2 * hf, 2)}, {v(VC + hf * 4 + db)} offset:{ks * 4096}")
+                    reads.append(f"ds_read_b64_tr_b16 {self.fr(slot + 2 * hf, 2)}, {v(self.VC + hf * 4 + db % 4)} "
+                                 f"offset:{ks * 16 * self.rowb + (db // 4) * 256}")
                 acc = ar(db * 16, 16)
-                bop = vr(SET[par] + 32 + 16 * kb + 4 * t2, 4)
-                mf.append((f"{self.mf} {acc}, {ar(slot, 4)}, {bop}, {acc}", 2 * k + 1))
+                bop = vr(self.SET[par] + 16 * self.nkb + 16 * kb + 4 * t2, 4)
+                mf.append((f"{self.mf} {acc}, {self.fr(slot, 4)}, {bop}, {acc}", 2 * k + 1))
                 k += 1
         return reads, mf
 
@@ -244,9 +255,9 @@ class Emitter:
         """Raw scores of tile j in SET[par] set to negc (c * negc = -inf) where
         key > row (causal) or key >= nk.  Skipped when no key of the tile can be masked
         for this wave."""
-        e = self.e
-        e(f"s_lshl_b32 s{ST}, s{SJ}, 6")                  # n0 = j * 64
-        e(f"s_add_u32 s{ST2}, s{ST}, 63")
+        e, op, (t0, t1, _, t3) = self.e, self.op, self.T
+        e(f"s_lshl_b32 s{ST}, s{SJ}, {4 + self.nkb}")                  # n0 = first key of tile j
+        e(f"s_add_u32 s{ST2}, s{ST}, {self.bn - 1}")
         e(f"s_cmp_gt_i32 s{ST2}, {op('wrow')}")
         e(f"s_cselect_b32 s{SM}, 1, 0")
         e(f"s_cmp_ge_i32 s{ST2}, {op('nk')}")
@@ -256,21 +267,21 @@ class Emitter:
         e(f"s_cbranch_scc1 {lbl}")
         e("s_nop 7")
         e("s_nop 7")
-        e(f"v_mov_b32 {v(T3)}, {op('negc')}")
+        e(f"v_mov_b32 {v(t3)}, {op('negc')}")
         e(f"s_sub_u32 s{ST2}, {op('nk')}, s{ST}")
         e(f"s_sub_u32 s{ST2}, s{ST2}, 1")                 # last valid key of the tile, local
         # thr = min(row - n0, nk - 1 - n0) - hh*4: key kb*32 + c_i (+ hh*4) is kept iff
         # c_i + kb*32 <= thr
-        e(f"v_subrev_u32 {v(T0)}, s{ST}, {op('row')}")
-        e(f"v_min_i32 {v(T0)}, s{ST2}, {v(T0)}")
-        e(f"v_sub_u32 {v(T0)}, {v(T0)}, {op('hh4')}")
-        for kb in range(2):
-            e(f"v_subrev_u32 {v(T1)}, {kb * 32}, {v(T0)}")
+        e(f"v_subrev_u32 {v(t0)}, s{ST}, {op('row')}")
+        e(f"v_min_i32 {v(t0)}, s{ST2}, {v(t0)}")
+        e(f"v_sub_u32 {v(t0)}, {v(t0)}, {op('hh4')}")
+        for kb in range(self.nkb):
+            e(f"v_subrev_u32 {v(t1)}, {kb * 32}, {v(t0)}")
             for i in range(16):
                 ci = (i // 4) * 8 + i % 4
-                r = SET[par] + kb * 16 + i
-                e(f"v_cmp_le_i32 vcc, {ci}, {v(T1)}")
-                e(f"v_cndmask_b32 {v(r)}, {v(T3)}, {v(r)}, vcc")
+                r = self.SET[par] + kb * 16 + i
+                e(f"v_cmp_le_i32 vcc, {ci}, {v(t1)}")
+                e(f"v_cndmask_b32 {v(r)}, {v(t3)}, {v(r)}, vcc")
         e(f"{lbl}:")
 
     def a_simple(self, par):
@@ -293,7 +304,7 @@ class Emitter:
             self.es(self.kcur_ops(f"s{ST2}"))
         # the gradient stream of the whole tile, split by issue cycles: about a third
         # beside the 16 dQ products, the rest beside the 32 S/dP products
-        gall = self.grad_ops(par, 0) + self.grad_ops(par, 1)
+        gall = [x for kb in range(self.nkb) for x in self.grad_ops(par, kb)]
         tot = sum(self.cost(x) for x in gall)
         cut, acc = 0, 0
         if has_q:
@@ -319,7 +330,7 @@ class Emitter:
         e(f"s_branch {L('next', shared=True)}")
 
     def program(self):
-        e = self.e
+        e, op, DN = self.e, self.op, self.DN
         labels = {}
         counter = [0]
 
@@ -342,7 +353,7 @@ class Emitter:
         e(f"v_sub_f32 {v(DN)}, 0, {op('dl')}")
         for r in range(DN + 1, DN + 16):
             e(f"v_mov_b32 {v(r)}, {v(DN)}")
-        for a in range(64):
+        for a in range(self.nacc):
             e(f"v_accvgpr_write_b32 a{a}, 0")
         self.dma()
         self.dma()
@@ -421,12 +432,12 @@ class Emitter:
             self.interleave(reads, mf, QDIST)
             e(f"s_branch {L('out', shared=True)}")
         e(f"{L('out', shared=True)}:")
-        # every wave is done with the ring: dQ^T goes to this wave's 16 blocks of LDS, OSTR apart
+        # every wave is done with the ring: dQ^T goes to this wave's blocks of LDS, OSTR apart
         for _ in range(2):
             e("s_nop 15")
         e("s_waitcnt vmcnt(0) lgkmcnt(0)")
         e("s_barrier")
-        for g in range(16):
+        for g in range(4 * self.db):
             e(f"ds_write_b128 {op('olds')}, {ar(4 * g, 4)} offset:{g * OSTR}")
         e("s_waitcnt lgkmcnt(0)")
         e(f"s_mov_b32 m0, s{SM0}")
@@ -461,20 +472,22 @@ def render(knobs=None, measure=False):
 
 def _render():
     out = ["// Generated by gen_dq_pipe.py; do not edit.", "#pragma once", ""]
-    for bf16, name in ((False, "FAL_DQP_ASM_F16"), (True, "FAL_DQP_ASM_BF16")):
-        lines = Emitter(bf16).program()
-        out.append(f"#define {name} \\")
-        for ln in lines:
-            out.append(f'  "{ln}\\n" \\')
+    for d, pre in ((128, "FAL_DQP"), (256, "FAL_DQP256")):
+        for bf16, name in ((False, "F16"), (True, "BF16")):
+            em = Emitter(d, bf16)
+            lines = em.program()
+            out.append(f"#define {pre}_ASM_{name} \\")
+            for ln in lines:
+                out.append(f'  "{ln}\\n" \\')
+            out.append("")
+        ins = ", ".join(f'"{c}"({x})' for _, c, x in operands(d))
+        clob = ", ".join([f'"v{i}"' for i in range(em.vlow, 256)] + [f'"a{i}"' for i in range(0, em.nacc)] +
+                         ([f'"a{i}"' for i in range(em.AR, 256)] if em.ring == "a" else []) +
+                         [f'"s{i}"' for i in range(84, 100)] + ['"vcc"', '"scc"', '"memory"'])
+        out.append(f"#define {pre}_OUTS")
+        out.append(f"#define {pre}_INS {ins}")
+        out.append(f"#define {pre}_CLOBBERS {clob}")
         out.append("")
-    ins = ", ".join(f'"{c}"({x})' for _, c, x in INS)
-    clob = ", ".join([f'"v{i}"' for i in range(DN, 256)] + [f'"a{i}"' for i in range(0, 64)] +
-                     [f'"a{i}"' for i in range(AR, 256)] + [f'"s{i}"' for i in range(84, 100)] +
-                     ['"vcc"', '"scc"', '"memory"'])
-    out.append("#define FAL_DQP_OUTS")
-    out.append(f"#define FAL_DQP_INS {ins}")
-    out.append(f"#define FAL_DQP_CLOBBERS {clob}")
-    out.append("")
     return "\n".join(out)
 
 

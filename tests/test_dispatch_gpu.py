@@ -4,7 +4,7 @@ that choose a kernel or a work order by problem size."""
 import pytest
 import torch
 
-from helpers import FWD_ATOL, max_abs, oracle_fwd, randn
+from helpers import FWD_ATOL, GRAD_RTOL, max_abs, oracle_bwd, oracle_fwd, randn, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -68,3 +68,33 @@ def test_head_dim_128_full_grid(B, Hq, Hkv, Nq, Nk, sign, causal):
     scale = sign * 128 ** -0.5
     o, lse = hip_ext.forward(q, k, v, scale, causal)
     check_groups(o, lse, q, k, v, scale, causal, [(b, g) for b in range(B) for g in range(Hkv)])
+
+
+def check_gradients(B, Hq, Hkv, Nq, Nk, d, causal, sign=1):
+    from flash_attn_legacy import hip_ext
+    q, k, v, do = (randn(s, i) for i, s in enumerate(
+        [(B, Hq, Nq, d), (B, Hkv, Nk, d), (B, Hkv, Nk, d), (B, Hq, Nq, d)]))
+    scale = sign * d ** -0.5
+    o, lse = hip_ext.forward(q, k, v, scale, causal)
+    got = hip_ext.backward(do, q, k, v, o, lse, scale, causal)
+    again = hip_ext.backward(do, q, k, v, o, lse, scale, causal)
+    for name, g, g2, ref in zip(("dq", "dk", "dv"), got, again, oracle_bwd(q, k, v, do, scale, causal)):
+        assert torch.isfinite(g).all(), name
+        assert rel_err(g, ref) <= GRAD_RTOL, name
+        assert torch.equal(g, g2), name + " differs between two runs"
+
+
+# head_dim 256 backward: edges of the 32-row items and key tiles, of the 128-key and
+# 128-row workgroups, of the causal pairing (odd and even tile counts), GQA, Nq != Nk with
+# key tiles that no query sees, a negative scale; bitwise equal over two runs.
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,Nq,Nk,sign", [
+    (1, 2, 2, 1, 1, 1),
+    (2, 4, 2, 31, 33, 1),
+    (1, 4, 4, 129, 127, 1),
+    (1, 4, 1, 300, 300, 1),
+    (2, 6, 2, 96, 417, -1),
+    (1, 2, 1, 545, 64, 1),
+])
+def test_head_dim_256_backward(B, Hq, Hkv, Nq, Nk, sign, causal):
+    check_gradients(B, Hq, Hkv, Nq, Nk, 256, causal, sign)
