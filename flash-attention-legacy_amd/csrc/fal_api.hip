@@ -344,7 +344,8 @@ int fal_fwd_varlen_bf16(const void* q, const void* k, const void* v, void* o, fl
 // ---------------------------------------------------------------------------
 // Backward
 // ---------------------------------------------------------------------------
-// Backward workspace: delta [rows] fp32, plus, for head dims without the query-outer
+// Backward workspace: delta [rows] fp32, the lsd array and the partial dK/dV sums of the
+// pipelined kernels (below), plus, for head dims without the query-outer
 // dQ kernel, the fp32 dQ accumulator [rows, d] in front of it.
 static size_t bwd_acc_bytes(size_t rows, int64_t head_dim, bool batched) {
   return bwd_split_dq(head_dim_ok(head_dim) ? (int)head_dim : 0, batched) ? 0 : align256(rows * head_dim * sizeof(float));
@@ -358,10 +359,32 @@ static size_t bwd_lsd_bytes(int64_t batch, int64_t heads_q, int64_t seqlen_q, in
   return align256((size_t)batch * heads_q * ((seqlen_q + bm - 1) / bm) * 2 * bm * sizeof(float));
 }
 
-size_t fal_bwd_workspace_size(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim) {
+// What a batched backward cannot do without.
+static size_t bwd_need(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim) {
   const size_t rows = (size_t)batch * heads_q * seqlen_q;
   return bwd_acc_bytes(rows, head_dim, true) + align256(rows * sizeof(float)) +
          bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim);
+}
+
+size_t fal_bwd_workspace_size(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim) {
+  // (head_dim 256: with room for partial dK/dV sums, one fp32 row per query row)
+  const size_t rows = (size_t)batch * heads_q * seqlen_q;
+  return bwd_need(batch, heads_q, seqlen_q, head_dim) +
+         (head_dim == 256 ? align256(rows * head_dim * sizeof(float)) : 0);
+}
+
+// At most this much goes to the partial dK/dV sums (512 key tiles at head_dim 256).
+constexpr size_t kKvPartMax = size_t(128) << 20;
+
+size_t fal_bwd_workspace_best(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t seqlen_q, int64_t seqlen_k,
+                              int64_t head_dim, int is_causal) {
+  const size_t need = bwd_need(batch, heads_q, seqlen_q, head_dim);
+  if (!head_dim_ok(head_dim) || batch <= 0 || heads_q <= 0 || heads_kv <= 0 || !dims_ok(seqlen_q) ||
+      !dims_ok(seqlen_k))
+    return need;
+  int run, runs;
+  return need + bwd_kv_plan(batch, heads_q, heads_kv, seqlen_q, seqlen_k, (int)head_dim, is_causal != 0,
+                            device_cu_count(), kKvPartMax, &run, &runs);
 }
 
 static int fill_bwd_common(BwdParams& p, const void* dout, const void* q, const void* k, const void* v,
@@ -434,7 +457,7 @@ static int fal_bwd_impl(const void* dout, const void* q, const void* k, const vo
   int rc = fill_bwd_common(p, dout, q, k, v, o, lse, dq, dk, dv, do_strides, q_strides, k_strides, v_strides,
                            o_strides, dq_strides, dk_strides, dv_strides, true);
   if (rc) return rc;
-  const size_t need = fal_bwd_workspace_size(batch, heads_q, seqlen_q, head_dim);
+  const size_t need = bwd_need(batch, heads_q, seqlen_q, head_dim);
   if (!workspace || workspace_bytes < need)
     return fail(FAL_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu", need, workspace_bytes);
   if (batch == 0 || (seqlen_k == 0 && seqlen_q == 0)) return ok();
@@ -442,8 +465,14 @@ static int fal_bwd_impl(const void* dout, const void* q, const void* k, const vo
   const size_t acc = bwd_acc_bytes(rows, head_dim, true);
   p.dq_acc = acc ? static_cast<float*>(workspace) : nullptr;
   p.delta = reinterpret_cast<float*>(static_cast<char*>(workspace) + acc);
-  if (bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim))
-    p.lsd = reinterpret_cast<float*>(static_cast<char*>(workspace) + acc + align256(rows * sizeof(float)));
+  const size_t lsd = bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim);
+  const size_t lsd_at = acc + align256(rows * sizeof(float));
+  if (lsd) {
+    p.lsd = reinterpret_cast<float*>(static_cast<char*>(workspace) + lsd_at);
+    p.kv_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + lsd_at + lsd);
+    bwd_kv_plan(batch, heads_q, heads_kv, seqlen_q, seqlen_k, (int)head_dim, is_causal != 0, device_cu_count(),
+                std::min(workspace_bytes - lsd_at - lsd, kKvPartMax), &p.kv_run, &p.kv_runs);
+  }
   p.dqa_sb = heads_q * seqlen_q * head_dim; p.dqa_sh = seqlen_q * head_dim; p.dqa_ss = head_dim;
   p.l_sb = heads_q * seqlen_q; p.l_sh = seqlen_q; p.l_ss = 1;
   p.B = (int)batch; p.Hq = (int)heads_q; p.Hkv = (int)heads_kv;

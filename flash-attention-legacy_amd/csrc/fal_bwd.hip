@@ -22,7 +22,9 @@
 //   (KV-outer, dS^T staged in LDS, dQ = dS K added with fp32 atomics; all 256 dK/dV
 //   columns accumulate in one pass, with K read from its LDS tile) and bwd_post_kernel
 //   (dQ cast to fp16).
+#include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "fal_kernels.h"
 #include "fal_bwd_pipe.inc"
@@ -839,7 +841,7 @@ constexpr int kKvOStr = 528;
 template <int D>
 constexpr int pipe_bm() { return D == 256 ? 32 : 64; }   // query rows per item
 
-template <class T, int D, bool CAUSAL>
+template <class T, int D, bool CAUSAL, bool SPLIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 bwd_kv_pipe_kernel(BwdParams p) {
   using V8 = vec8<T>;
@@ -857,19 +859,44 @@ bwd_kv_pipe_kernel(BwdParams p) {
   const int hh = lane >> 5;
 
   // work item: one or two 128-key tiles of one (batch, KV head); causal tiles are
-  // paired (kt, n-1-kt) so every workgroup has the same number of items
+  // paired (kt, n-1-kt) so every workgroup has the same number of items.  SPLIT (kv_run set):
+  // one run of one key tile's items.
   const int nkt = cdiv(p.Nk, kPipeBN);
   const int total = gridDim.x;
-  int id = blockIdx.x;
-  if ((total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
-  const int nk_items = CAUSAL ? (nkt + 1) / 2 : nkt;
-  const int kit = id % nk_items;
-  const int bh = id / nk_items;
+  int id = blockIdx.x, run = 0, kit, bh;
+  if (SPLIT) {
+    // the first key tiles of all heads first (an XCD keeps whole heads when they divide by 8):
+    // under a causal mask they have the most items
+    int units = p.B * p.Hkv, u = 0;
+    if ((units & 7) == 0) {
+      units >>= 3;
+      u = (id & 7) * units;
+      id >>= 3;
+    }
+    kit = id / (units * p.kv_runs);
+    id -= kit * units * p.kv_runs;
+    bh = u + id / p.kv_runs;
+    run = id % p.kv_runs;
+  } else {
+    if ((total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
+    const int nk_items = CAUSAL ? (nkt + 1) / 2 : nkt;
+    kit = id % nk_items;
+    bh = id / nk_items;
+  }
+  const int slot = (bh * nkt + kit) * p.kv_runs + run;   // (SPLIT) of this workgroup's sums
   const int b = bh / p.Hkv, hkv = bh % p.Hkv;
-  const int kt_b = (CAUSAL && nkt - 1 - kit != kit) ? nkt - 1 - kit : -1;
+  const int kt_b = (CAUSAL && !SPLIT && nkt - 1 - kit != kit) ? nkt - 1 - kit : -1;
   const int G = p.Hq / p.Hkv;
   const int nq = p.Nq, nk = p.Nk;
   const int nqt = cdiv(nq, kPipeBM);
+  int run_len = 0, nruns = 1;
+  if (SPLIT) {
+    kv_runs_of(G * max(nqt - (CAUSAL ? kit * kPipeBN / kPipeBM : 0), 0), p.kv_run, &run_len, &nruns);
+    // (uniform values: the pipelined loop takes them as scalar operands)
+    run_len = __builtin_amdgcn_readfirstlane(run_len);
+    nruns = __builtin_amdgcn_readfirstlane(nruns);
+    if (run >= nruns) return;
+  }
 
   typedef __attribute__((address_space(3))) char lds_t;
   const uint32_t lds0 = (uint32_t)(uintptr_t)((lds_t*)smem);
@@ -934,23 +961,31 @@ bwd_kv_pipe_kernel(BwdParams p) {
       vreg[t] = __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(vrs, vo + t * 32, 0, 0));
     }
   };
-  load_kv(kit);
-  for (int tile_i = 0; tile_i < 2; ++tile_i) {
+  // (head_dim 256: its 128 registers of K and V would be spilled around the epilogue, so
+  // each tile loads its own first)
+  constexpr bool AHEAD = D == 128;
+  if (AHEAD) load_kv(kit);
+  for (int tile_i = 0; tile_i < (SPLIT || !CAUSAL ? 1 : 2); ++tile_i) {
     const int kt = tile_i == 0 ? kit : kt_b;
     if (kt < 0) break;
     const int n0 = kt * kPipeBN;
     const int kw0 = n0 + ws * 32;
     const int qt0 = CAUSAL ? n0 / kPipeBM : 0;
     const int ntq = max(nqt - qt0, 0);
-    const int nitems = G * ntq;
+    if (!AHEAD) load_kv(kt);
+    // this workgroup's items: all of the key tile's, or a run of them from item i0 on
+    const bool part = SPLIT && nruns > 1;
+    const int i0 = part ? run * run_len : 0;
+    const int nitems = part ? min(run_len, G * ntq - i0) : G * ntq;
     __syncthreads();   // the previous tile's epilogue readers are done with the LDS
     if (nitems > 0) {
-      const int hq0 = hkv * G;
+      const int h0 = part ? __builtin_amdgcn_readfirstlane(i0 / ntq) : 0;
+      const int hq0 = hkv * G + h0, q0 = qt0 + i0 - h0 * ntq;
       const uint64_t qb = (uint64_t)(uintptr_t)((const T*)p.q + (int64_t)b * p.q_sb + (int64_t)hq0 * p.q_sh +
-                                                (int64_t)qt0 * kPipeBM * p.q_ss);
+                                                (int64_t)q0 * kPipeBM * p.q_ss);
       const uint64_t dob = (uint64_t)(uintptr_t)((const T*)p.dout + (int64_t)b * p.do_sb +
-                                                 (int64_t)hq0 * p.do_sh + (int64_t)qt0 * kPipeBM * p.do_ss);
-      const uint64_t lb = (uint64_t)(uintptr_t)(p.lsd + (((int64_t)b * p.Hq + hq0) * nqt + qt0) * 2 * kPipeBM);
+                                                 (int64_t)hq0 * p.do_sh + (int64_t)q0 * kPipeBM * p.do_ss);
+      const uint64_t lb = (uint64_t)(uintptr_t)(p.lsd + (((int64_t)b * p.Hq + hq0) * nqt + q0) * 2 * kPipeBM);
       const int64_t qwrap = p.q_sh * 2 - (int64_t)(ntq - 1) * qstep - qhalf;
       const int64_t dwrap = p.do_sh * 2 - (int64_t)(ntq - 1) * dstep - dhalf;
       const uint32_t p_qb_lo = (uint32_t)qb, p_qb_hi = (uint32_t)(qb >> 32) & 0xffffu;
@@ -961,7 +996,11 @@ bwd_kv_pipe_kernel(BwdParams p) {
       const uint32_t p_ds_lo = (uint32_t)(dstep - dhalf), p_ds_hi = (uint32_t)((uint64_t)(dstep - dhalf) >> 32);
       const uint32_t p_dw_lo = (uint32_t)dwrap, p_dw_hi = (uint32_t)((uint64_t)dwrap >> 32);
       const uint32_t p_ldw = (uint32_t)(1 + qt0) * 2 * kPipeBM * 4;   // last tile of a head -> first of the next
-      const int p_qt0 = qt0, p_nitems = nitems;
+      const int p_qt0 = qt0, p_qs0 = q0, p_nitems = nitems;
+      const int p_part = SPLIT ? __builtin_amdgcn_readfirstlane(nruns - 1) : 0;
+      // dV and dK sums of this wave's 32 keys
+      const uint64_t po = SPLIT ? (uint64_t)(uintptr_t)(p.kv_part + ((int64_t)slot * 4 + ws) * 64 * D) : 0;
+      const uint32_t p_po_lo = (uint32_t)po, p_po_hi = (uint32_t)(po >> 32) & 0xffffu;
       const int p_kw0 = CAUSAL ? kw0 : -(1 << 30);
       constexpr bool F16 = std::is_same<T, half_t>::value;
       if constexpr (D == 128 && F16)
@@ -973,7 +1012,8 @@ bwd_kv_pipe_kernel(BwdParams p) {
       if constexpr (D == 256 && !F16)
         asm volatile(FAL_BWDP256_ASM_BF16 : FAL_BWDP256_OUTS : FAL_BWDP256_INS : FAL_BWDP256_CLOBBERS);
     }
-    if (tile_i == 0 && kt_b >= 0) load_kv(kt_b);
+    if (part) return;
+    if (AHEAD && tile_i == 0 && kt_b >= 0) load_kv(kt_b);
     // dV then dK*scale of this wave's keys: piece pc = db*4 + g4 of lane (hh, l32) holds
     // columns 8*pc + hh*4 .. +3 of key kw0 + l32, at which*kKvOPart + pc*kKvOStr + lane*8.
     // Written back row-wise: each 16-byte store instruction covers whole rows.
@@ -1007,6 +1047,49 @@ bwd_kv_pipe_kernel(BwdParams p) {
 #pragma unroll
           for (int jj = 0; jj < 8; ++jj) buffer_store16(rs[which], vo[which] + (j0 + jj) * rstep[which], x[jj]);
         }
+    }
+  }
+}
+
+// Adds the runs of a split key tile (BwdParams::kv_run), in run order, and writes its dV and
+// dK * scale.  One workgroup per (batch, KV head, key tile, 32 keys, dV or dK); a run's sums
+// are blocks of 1 KB, block db*4 + g4 holding columns db*32 + g4*8 + hh*4 .. +3 of key l32 at
+// (hh*32 + l32) * 16.
+template <class T, int D, bool CAUSAL>
+__global__ void __launch_bounds__(256)
+bwd_kv_reduce_kernel(BwdParams p) {
+  constexpr int CPR = D / 8, RPI = 256 / CPR;
+  const int which = blockIdx.x & 1, w = (blockIdx.x >> 1) & 3;
+  const int nkt = cdiv(p.Nk, kPipeBN);
+  const int tile = blockIdx.x >> 3, kt = tile % nkt, bh = tile / nkt;
+  int len, runs;
+  const int nqt = cdiv(p.Nq, pipe_bm<D>());
+  kv_runs_of((p.Hq / p.Hkv) * max(nqt - (CAUSAL ? kt * kPipeBN / pipe_bm<D>() : 0), 0), p.kv_run, &len, &runs);
+  if (runs < 2) return;      // written by its workgroup
+  const int b = bh / p.Hkv, hkv = bh % p.Hkv;
+  const int cch = threadIdx.x % CPR, key0 = kt * kPipeBN + w * 32;
+  T* out = which ? (T*)p.dk + (int64_t)b * p.dk_sb + (int64_t)hkv * p.dk_sh
+                 : (T*)p.dv + (int64_t)b * p.dv_sb + (int64_t)hkv * p.dv_sh;
+  const int64_t ss = which ? p.dk_ss : p.dv_ss;
+  const float sc = which ? p.scale : 1.f;
+  const float* part = p.kv_part + ((int64_t)tile * p.kv_runs * 4 + w) * 64 * D + which * 32 * D + cch * 256;
+#pragma unroll
+  for (int r0 = 0; r0 < 32; r0 += RPI) {
+    const int r = r0 + threadIdx.x / CPR;
+    f32x4 lo = f32x4{0.f, 0.f, 0.f, 0.f}, hi = lo;
+    for (int i = 0; i < runs; ++i) {
+      const float* x = part + (int64_t)i * 4 * 64 * D + r * 4;
+      lo += *reinterpret_cast<const f32x4*>(x);
+      hi += *reinterpret_cast<const f32x4*>(x + 128);
+    }
+    if (key0 + r < p.Nk) {
+      vec8<T> h;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        h[e] = (T)(lo[e] * sc);
+        h[4 + e] = (T)(hi[e] * sc);
+      }
+      st_u4(out + (int64_t)(key0 + r) * ss + cch * 8, __builtin_bit_cast(u32x4, h));
     }
   }
 }
@@ -1414,16 +1497,88 @@ int bwd_block_n(int d) {
 bool bwd_pipe(int d) { return FAL_BWD_PIPE && (d == 128 || d == 256); }
 int bwd_pipe_bm(int d) { return d == 256 ? pipe_bm<256>() : pipe_bm<128>(); }
 
+// A dK/dV workgroup takes about 1.85 us per item and 8 us besides, so a grid smaller than the
+// GPU (few KV heads, short sequences) ends with its longest workgroup while CUs idle.
+// Cutting the key tiles' items into runs fills them; it costs the fp32 sums, written and
+// read again (about 2.5 and 4 TB/s), and the launch that adds them, about 6 us.  Tried are
+// 2 to 16 runs for the longest key tile, up to two workgroups per CU (longest first, so the
+// longest is followed by the shortest); the best is taken if it saves a tenth.
+// Backward us before -> after: 1 x 32/8 heads x 1024 x 128 causal 159 -> 86, x 2048 272 -> 163,
+// 1 x 28/4 x 333 x 128 83 -> 43, 1 x 16/4 x 4096 x 128 causal 500 -> 292,
+// 1 x 8/1 x 777 x 256 causal 371 -> 114.
+size_t bwd_kv_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int d, int causal, int ncu,
+                   size_t avail, int* run, int* runs) {
+  *run = *runs = 0;
+  constexpr int kMaxTiles = 256;
+  if (!bwd_pipe(d) || ncu <= 0 || Nq <= 0 || Nk <= 0) return 0;
+  const int64_t bm = bwd_pipe_bm(d), nqt = (Nq + bm - 1) / bm, nkt = (Nk + kPipeBN - 1) / kPipeBN;
+  const int64_t units = B * Hkv, G = Hq / Hkv, grid0 = units * (causal ? (nkt + 1) / 2 : nkt);
+  if (grid0 >= ncu || nkt > kMaxTiles || G * nqt > (1 << 20)) return 0;
+  auto items = [&](int64_t kt) { return (int)(G * std::max<int64_t>(nqt - (causal ? kt * kPipeBN / bm : 0), 0)); };
+  int64_t longest = items(0);
+  if (causal)
+    for (int64_t kt = 0; kt < (nkt + 1) / 2; ++kt)
+      longest = std::max<int64_t>(longest, items(kt) + (nkt - 1 - kt != kt ? items(nkt - 1 - kt) : 0));
+  const double slot = (double)kPipeBN * d * 2 * sizeof(float);
+  double best = 0.9 * (8 + 1.85 * longest);
+  size_t used = 0;
+  for (int r = 2; r <= 16 && r <= items(0); ++r) {
+    const int c = (items(0) + r - 1) / r;
+    int len, most;
+    kv_runs_of(items(0), c, &len, &most);
+    std::pair<int, int64_t> lens[kMaxTiles];      // (items, workgroups) of each key tile
+    int64_t grid = 0, split = 0;
+    for (int64_t kt = 0; kt < nkt; ++kt) {
+      int n;
+      kv_runs_of(items(kt), c, &len, &n);
+      lens[kt] = {len, n * units};
+      grid += n * units;
+      if (n > 1) split += n * units;
+    }
+    if (grid > 2 * (int64_t)ncu || most * nkt * units * slot > (double)avail) break;
+    std::sort(lens, lens + nkt, [](const auto& a, const auto& b) { return a.first > b.first; });
+    // the first ncu workgroups in order, the rest (shortest on the longest) behind them
+    int64_t span = lens[0].first, i = 0, j = nkt - 1, ni = lens[0].second, nj = lens[nkt - 1].second;
+    for (int64_t second = grid - ncu; second > 0;) {
+      const int64_t n = std::min({ni, nj, second});
+      span = std::max<int64_t>(span, (int64_t)lens[i].first + lens[j].first);
+      second -= n;
+      if ((ni -= n) == 0 && i + 1 < nkt) ni = lens[++i].second;
+      if ((nj -= n) == 0 && j > 0) nj = lens[--j].second;
+    }
+    const double us = (grid > ncu ? 16 : 8) + 1.85 * span + 6 + slot * split * (1 / 2.5e6 + 1 / 4e6);
+    if (us < best) {
+      best = us;
+      *run = c;
+      *runs = most;
+      used = (size_t)(most * nkt * units * slot);
+    }
+  }
+  return used;
+}
+
 template <class T, int D>
 static hipError_t launch_bwd_t(const BwdParams& p, int causal, dim3 grid, hipStream_t st) {
   if constexpr (D == 128 || D == 256) {
     if (!p.cu_q && p.lsd) {
-      const int nkt = cdiv(p.Nk, kPipeBN);
-      grid.x = (unsigned)((causal ? (nkt + 1) / 2 : nkt) * p.B * p.Hkv);
-      if (causal)
-        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, true>), grid, dim3(256), 0, st, p);
+      const int nkt = cdiv(p.Nk, kPipeBN), tiles = nkt * p.B * p.Hkv;
+      grid.x = p.kv_run ? (unsigned)(tiles * p.kv_runs) : (unsigned)((causal ? (nkt + 1) / 2 : nkt) * p.B * p.Hkv);
+      if (causal && !p.kv_run)
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, true, false>), grid, dim3(256), 0, st, p);
+      else if (causal)
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, true, true>), grid, dim3(256), 0, st, p);
+      else if (!p.kv_run)
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, false, false>), grid, dim3(256), 0, st, p);
       else
-        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, false>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, false, true>), grid, dim3(256), 0, st, p);
+      if (p.kv_run) {
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        if (causal)
+          hipLaunchKernelGGL((bwd_kv_reduce_kernel<T, D, true>), dim3((unsigned)tiles * 8), dim3(256), 0, st, p);
+        else
+          hipLaunchKernelGGL((bwd_kv_reduce_kernel<T, D, false>), dim3((unsigned)tiles * 8), dim3(256), 0, st, p);
+      }
       return hipGetLastError();
     }
   }

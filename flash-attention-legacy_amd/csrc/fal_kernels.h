@@ -93,7 +93,21 @@ struct BwdParams {
   int total_k;        // varlen: rows of the packed K/V
   int bf16;           // element type of every fp16/bf16 tensor: 0 fp16, 1 bf16
   float* lsd;         // batched head_dim 128 and 256: per query tile, -L*log2(e)/c then -D (null: unused)
+  // pipelined dK/dV kernel on small grids: each key tile's items are cut into runs of at most
+  // kv_run, one workgroup each, whose fp32 sums go to kv_part (slot (batch, KV head, key
+  // tile, run), kv_runs slots per key tile) and are added by bwd_kv_reduce_kernel; 0: one
+  // workgroup takes all items
+  int kv_run, kv_runs;
+  float* kv_part;
 };
+
+// Items of key tile kt (128 keys) cut into equal runs of at most p.kv_run: the run length,
+// and the number of runs.
+__host__ __device__ inline void kv_runs_of(int nitems, int kv_run, int* len, int* runs) {
+  const int r = nitems > kv_run ? (nitems + kv_run - 1) / kv_run : 1;
+  *len = (nitems + r - 1) / r;
+  *runs = *len > 0 ? (nitems + *len - 1) / *len : 1;
+}
 
 // KV-cache decode (one query token per sequence).
 struct DecodeParams {
@@ -168,6 +182,10 @@ int bwd_dq_block_m(int d);
 // batched head_dim d uses bwd_kv_pipe_kernel (workspace holds the lsd array)
 bool bwd_pipe(int d);
 int bwd_pipe_bm(int d);   // its query rows per item
+// Plan of BwdParams::kv_run / kv_runs for a batched call of head_dim d on `ncu` compute units
+// with `avail` bytes for the partial sums (0 / 0: no split); returns the bytes it uses.
+size_t bwd_kv_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int d, int causal, int ncu,
+                   size_t avail, int* run, int* runs);
 hipError_t launch_bwd_dq(const BwdParams& p, int d, int causal, dim3 grid, hipStream_t st);
 
 int decode_chunk(int d, int B, int Hkv, int max_seqlen);

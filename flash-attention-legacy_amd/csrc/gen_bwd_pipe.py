@@ -5,7 +5,8 @@ in what the last paragraph of this text lists.
 
 A workgroup owns 128 keys of one KV head; wave w owns keys kw0 = n0 + 32w .. +31 and
 keeps their K and V fragments in registers (B operands).  It walks the items (query
-head of the GQA group, 64-row query tile) in order.  For item i:
+head of the GQA group, 64-row query tile) in order, all of the key tile's or a run of them
+from query tile qs0 on.  For item i:
   A(i):  S = Q K^T + Ls and dP = dO V^T + Dn for the 64 rows x 32 keys (32 MFMAs,
          Q/dO fragments from LDS).  The accumulators start at Ls = -L*log2(e)/c and
          Dn = -D, read from LDS, so c*S is the exponent and dP is already dP - D;
@@ -101,7 +102,8 @@ def operands(d):
     ins += [("lk", "v", "p_lk"), ("olds", "v", "p_olds")]
     names = ("qb_lo", "qb_hi", "db_lo", "db_hi", "lb_lo", "lb_hi",
              "qs_lo", "qs_hi", "qw_lo", "qw_hi", "ds_lo", "ds_hi", "dw_lo", "dw_hi", "ldw",
-             "qrb", "drb", "nq", "nqt", "qt0", "nitems", "c", "negc", "kw0", "lbase", "ldbase", "scale")
+             "qrb", "drb", "nq", "nqt", "qt0", "qs0", "nitems", "c", "negc", "kw0", "lbase", "ldbase", "scale",
+             "part", "po_lo", "po_hi")
     return ins + [(n, "s", f"p_{n}") for n in names]
 
 
@@ -415,8 +417,8 @@ class Emitter:
             e(f"s_mov_b32 s{rs + 3}, {RSRC_W3}")
         e(f"s_mov_b32 s{SJ}, 0")
         e(f"s_mov_b32 s{SF}, 0")
-        e(f"s_mov_b32 s{SQF}, {op('qt0')}")
-        e(f"s_mov_b32 s{SQC}, {op('qt0')}")
+        e(f"s_mov_b32 s{SQF}, {op('qs0')}")
+        e(f"s_mov_b32 s{SQC}, {op('qs0')}")
         for a in range(self.nacc):
             e(f"v_accvgpr_write_b32 a{a}, 0")
         self.dma()
@@ -495,6 +497,19 @@ class Emitter:
         e("s_waitcnt vmcnt(0) lgkmcnt(0)")
         e("s_barrier")
         t0, t1, t2, t3 = self.T
+        # part: this workgroup has some of the key tile's items, so its sums go out in fp32 as
+        # they are, block (which, db, g4) of 1 KB after block, for bwd_kv_reduce_kernel
+        e(f"s_cmp_eq_u32 {op('part')}, 0")
+        e("s_cbranch_scc1 whole_%=")
+        e(f"s_mov_b32 s{SQ}, {op('po_lo')}")
+        e(f"s_mov_b32 s{SQ + 1}, {op('po_hi')}")
+        e(f"s_mov_b32 s{SQ + 2}, {8 * self.db * 1024}")
+        e(f"v_lshlrev_b32 {v(t0)}, 2, {op('lo4')}")
+        for g in range(8 * self.db):
+            e(f"s_mov_b32 s{ST0}, {g * 1024}")
+            e(f"buffer_store_dwordx4 {ar(4 * g, 4)}, {v(t0)}, s[{SQ}:{SQ + 3}], s{ST0} offen")
+        e("s_branch done_%=")
+        e("whole_%=:")
         for which in range(2):
             for db in range(self.db):
                 for g4 in range(4):
@@ -509,6 +524,7 @@ class Emitter:
                     off = which * 4 * self.db * OSTR + (db * 4 + g4) * OSTR
                     e(f"ds_write_b64 {op('olds')}, {vr(t0, 2)} offset:{off}")
         e("s_waitcnt lgkmcnt(0)")
+        e("done_%=:")
         e(f"s_mov_b32 m0, s{SM0}")
         return self.lines
 

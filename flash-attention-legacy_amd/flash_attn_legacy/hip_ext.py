@@ -58,6 +58,7 @@ def _load() -> ctypes.CDLL:
         "fal_fwd_varlen_workspace_size": (_SZ, [_I64] * 4),
         "fal_fwd_varlen": (_INT, [_VP] * 7 + [_I64] * 8 + [_STR] * 4 + [_F32, _INT, _VP, _SZ, _VP]),
         "fal_bwd_workspace_size": (_SZ, [_I64] * 4),
+        "fal_bwd_workspace_best": (_SZ, [_I64] * 6 + [_INT]),
         "fal_bwd": (_INT, [_VP] * 9 + [_I64] * 6 + [_STR] * 8 + [_F32, _INT, _VP, _SZ, _VP]),
         "fal_bwd_varlen_workspace_size": (_SZ, [_I64] * 5),
         "fal_bwd_varlen": (_INT, [_VP] * 11 + [_I64] * 8 + [_STR] * 8 + [_F32, _INT, _VP, _SZ, _VP]),
@@ -80,7 +81,7 @@ _lib = _load()
 SYMBOLS = (
     "fal_last_error", "fal_version", "fal_device_supported",
     "fal_fwd_workspace_size", "fal_fwd", "fal_fwd_varlen_workspace_size", "fal_fwd_varlen",
-    "fal_bwd_workspace_size", "fal_bwd", "fal_bwd_varlen_workspace_size", "fal_bwd_varlen",
+    "fal_bwd_workspace_size", "fal_bwd_workspace_best", "fal_bwd", "fal_bwd_varlen_workspace_size", "fal_bwd_varlen",
     "fal_decode_workspace_size", "fal_decode",
     "fal_fwd_bf16", "fal_fwd_varlen_bf16", "fal_bwd_bf16", "fal_bwd_varlen_bf16", "fal_decode_bf16",
     "fal_decode_noalloc",
@@ -303,8 +304,8 @@ def backward(dO, Q, K, V, O, L, softmax_scale: float, is_causal: bool = False) -
     dQ = torch.empty((B, Hq, N, d), dtype=Q.dtype, device=Q.device)
     dK = torch.empty((B, Hkv, Nk, d), dtype=Q.dtype, device=Q.device)
     dV = torch.empty((B, Hkv, Nk, d), dtype=Q.dtype, device=Q.device)
-    ws = _workspace(_lib.fal_bwd_workspace_size(B, Hq, N, d), Q.device)
     with torch.cuda.device(Q.device):
+        ws = _workspace(_lib.fal_bwd_workspace_best(B, Hq, Hkv, N, Nk, d, int(bool(is_causal))), Q.device)
         _check(_fn("fal_bwd", Q.dtype)(
             _ptr(dO), _ptr(Q), _ptr(K), _ptr(V), _ptr(O), _ptr(L), _ptr(dQ), _ptr(dK), _ptr(dV),
             B, Hq, Hkv, N, Nk, d,

@@ -105,13 +105,15 @@ int fal_fwd_varlen(const void* q, const void* k, const void* v, void* o, float* 
  * kernels it launches (precompute_D, flash_attn_bwd_*_launch).
  *   dout, q, o [B, Hq, Nq, d]; k, v [B, Hkv, Nk, d]; lse [B, Hq, Nq] from fal_fwd.
  *   Outputs dq [B, Hq, Nq, d], dk / dv [B, Hkv, Nk, d] (fp16), fully overwritten.
- * workspace: fal_bwd_workspace_size bytes: the row deltas D, plus an fp32 dQ
- * accumulator for head_dim 256 (the other head dims write dQ from their own kernel).
- * All gradients are bitwise deterministic, except dQ at head_dim 256: it is
- * accumulated with fp32 atomics, so its low bits can vary run to run (as in the
- * reference, flash_attn_bwd.cu:618).
+ * workspace: fal_bwd_workspace_size bytes hold the row deltas D and, at head_dim 128
+ * and 256, a second copy of them and of lse in tile order.  With fal_bwd_workspace_best
+ * bytes, always enough as well, head_dim 128 and 256 calls too small to fill the GPU split each key
+ * tile over several workgroups and add their fp32 sums; it depends on the current device.
+ * All gradients are bitwise deterministic (for the same workspace size).
  */
 size_t fal_bwd_workspace_size(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim);
+size_t fal_bwd_workspace_best(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t seqlen_q,
+                              int64_t seqlen_k, int64_t head_dim, int is_causal);
 int fal_bwd(const void* dout, const void* q, const void* k, const void* v, const void* o,
             const float* lse, void* dq, void* dk, void* dv,
             int64_t batch, int64_t heads_q, int64_t heads_kv,

@@ -98,3 +98,21 @@ def check_gradients(B, Hq, Hkv, Nq, Nk, d, causal, sign=1):
 ])
 def test_head_dim_256_backward(B, Hq, Hkv, Nq, Nk, sign, causal):
     check_gradients(B, Hq, Hkv, Nq, Nk, 256, causal, sign)
+
+
+# Pipelined backward on small grids, where each key tile's items are cut into runs whose sums a
+# second kernel adds: runs that start inside a head, key tiles of one run only (the last
+# causal ones), a last key tile of one key, MQA and GQA; and a call whose keys outnumber its
+# queries by so much that the workspace has no room for the sums.
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,Nq,Nk,d", [
+    (1, 8, 1, 257, 257, 128),
+    (1, 28, 4, 333, 333, 128),
+    (2, 16, 4, 512, 385, 128),
+    (1, 12, 3, 100, 200, 128),
+    (1, 8, 2, 260, 260, 256),
+    (1, 6, 1, 515, 129, 256),
+    (1, 4, 1, 64, 2000, 128),
+])
+def test_backward_runs(B, Hq, Hkv, Nq, Nk, d, causal):
+    check_gradients(B, Hq, Hkv, Nq, Nk, d, causal)
