@@ -1,11 +1,13 @@
-"""Build libfal_hip.so (the gfx950 attention library) in-tree with hipcc.
+"""Build libfal_hip.so (the gfx950 attention library) and its Python binding in-tree.
 
 Usage:  python flash-attention-legacy_amd/build.py [--jobs N] [--verbose] [--regen]
         python flash-attention-legacy_amd/build.py --out X.so [-D NAME=VALUE] [--knob fwd.KDIST=3] [--measure]
 
 Replaces the reference's nvcc ``CUDAExtension`` build (setup.py:48-82): every
 ``csrc/*.hip`` file is compiled for ``--offload-arch=gfx950`` and linked into
-``flash_attn_legacy/libfal_hip.so`` next to the Python package that loads it.
+``flash_attn_legacy/libfal_hip.so`` next to the Python package that loads it, and
+``csrc/fal_torch.cpp`` (host code: tensors in, library calls out) into
+``flash_attn_legacy/_fal_torch.so`` against the installed torch.
 """
 
 from __future__ import annotations
@@ -21,6 +23,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 OUT = os.path.join(HERE, "flash_attn_legacy", "libfal_hip.so")
+BINDING = os.path.join(HERE, "flash_attn_legacy", "_fal_torch.so")
 ARCH = "gfx950"
 
 COMMON_FLAGS = [
@@ -142,7 +145,31 @@ def build(jobs: int | None = None, verbose: bool = False, out: str = OUT, define
         raise RuntimeError(f"link failed:\n{r.stdout}{r.stderr}")
     _check_stubs(tmp)
     os.replace(tmp, out)
+    if not variant and os.path.abspath(out) == os.path.abspath(OUT):
+        build_binding(verbose)
     return out
+
+
+def build_binding(verbose: bool = False) -> str:
+    """Compile csrc/fal_torch.cpp with the host compiler; returns the module's path."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension as ext
+    inc = [*ext.include_paths("cuda"), sysconfig.get_paths()["include"]]
+    libdir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = BINDING + ".tmp"
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[a for p in inc for a in ("-isystem", p)], os.path.join(CSRC, "fal_torch.cpp"), "-o", tmp,
+           f"-L{libdir}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"binding build failed:\n{r.stdout}{r.stderr}")
+    os.replace(tmp, BINDING)
+    return BINDING
 
 
 def _check_stubs(lib: str) -> None:
