@@ -344,13 +344,8 @@ int fal_fwd_varlen_bf16(const void* q, const void* k, const void* v, void* o, fl
 // ---------------------------------------------------------------------------
 // Backward
 // ---------------------------------------------------------------------------
-// Backward workspace: delta [rows] fp32, the lsd array and the partial dK/dV sums of the
-// pipelined kernels (below), plus, for head dims without the query-outer
-// dQ kernel, the fp32 dQ accumulator [rows, d] in front of it.
-static size_t bwd_acc_bytes(size_t rows, int64_t head_dim, bool batched) {
-  return bwd_split_dq(head_dim_ok(head_dim) ? (int)head_dim : 0, batched) ? 0 : align256(rows * head_dim * sizeof(float));
-}
-
+// Backward workspace: D [rows] fp32, then the lsd array and the partial dK/dV sums of the
+// pipelined kernels (below).
 // Batched head_dim 128 and 256 also hold the lsd array: per (batch, query head, tile of 64
 // or 32 rows) a value of -L*log2(e)/c and one of -D per row.
 static size_t bwd_lsd_bytes(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim) {
@@ -362,8 +357,7 @@ static size_t bwd_lsd_bytes(int64_t batch, int64_t heads_q, int64_t seqlen_q, in
 // What a batched backward cannot do without.
 static size_t bwd_need(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim) {
   const size_t rows = (size_t)batch * heads_q * seqlen_q;
-  return bwd_acc_bytes(rows, head_dim, true) + align256(rows * sizeof(float)) +
-         bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim);
+  return align256(rows * sizeof(float)) + bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim);
 }
 
 size_t fal_bwd_workspace_size(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim) {
@@ -419,26 +413,15 @@ static int fill_bwd_common(BwdParams& p, const void* dout, const void* q, const 
   return FAL_OK;
 }
 
-static int run_bwd(BwdParams& p, int d, int causal, dim3 grid, dim3 dq_grid, bool batched, hipStream_t st) {
-  hipError_t e;
-  if (bwd_split_dq(d, batched)) {
-    // dQ kernel first: it also computes D = rowsum(dO * O), which the dK/dV kernel
-    // reads, so no preprocessing launch is needed
-    if (dq_grid.x > 0 && dq_grid.y > 0) {
-      e = launch_bwd_dq(p, d, causal, dq_grid, st);
-      if (e != hipSuccess) return launch_status(e, "bwd dq");
-    }
-    if (grid.x > 0 && grid.y > 0) return launch_status(launch_bwd(p, d, causal, grid, st), "bwd main");
-    return ok();
+static int run_bwd(BwdParams& p, int d, int causal, dim3 grid, dim3 dq_grid, hipStream_t st) {
+  // dQ kernel first: it also computes D = rowsum(dO * O), which the dK/dV kernel reads, so no
+  // preprocessing launch is needed
+  if (dq_grid.x > 0) {
+    hipError_t e = launch_bwd_dq(p, d, causal, dq_grid, st);
+    if (e != hipSuccess) return launch_status(e, "bwd dq");
   }
-  e = launch_bwd_pre(p, d, batched ? 1 : 0, st);
-  if (e != hipSuccess) return launch_status(e, "bwd preprocess");
-  if (grid.x > 0 && grid.y > 0) {
-    e = launch_bwd(p, d, causal, grid, st);
-    if (e != hipSuccess) return launch_status(e, "bwd main");
-  }
-  e = launch_bwd_post(p, d, st);
-  return launch_status(e, "bwd dq cast");
+  if (grid.x > 0) return launch_status(launch_bwd(p, d, causal, grid, st), "bwd main");
+  return ok();
 }
 
 static int fal_bwd_impl(const void* dout, const void* q, const void* k, const void* v, const void* o, const float* lse,
@@ -462,18 +445,16 @@ static int fal_bwd_impl(const void* dout, const void* q, const void* k, const vo
     return fail(FAL_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu", need, workspace_bytes);
   if (batch == 0 || (seqlen_k == 0 && seqlen_q == 0)) return ok();
   const size_t rows = (size_t)batch * heads_q * seqlen_q;
-  const size_t acc = bwd_acc_bytes(rows, head_dim, true);
-  p.dq_acc = acc ? static_cast<float*>(workspace) : nullptr;
-  p.delta = reinterpret_cast<float*>(static_cast<char*>(workspace) + acc);
+  p.delta = static_cast<float*>(workspace);
   const size_t lsd = bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim);
-  const size_t lsd_at = acc + align256(rows * sizeof(float));
+  const size_t lsd_at = align256(rows * sizeof(float));
   if (lsd) {
     p.lsd = reinterpret_cast<float*>(static_cast<char*>(workspace) + lsd_at);
+    p.lsd_tiles = cdiv((int)seqlen_q, bwd_pipe_bm((int)head_dim));
     p.kv_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + lsd_at + lsd);
     bwd_kv_plan(batch, heads_q, heads_kv, seqlen_q, seqlen_k, (int)head_dim, is_causal != 0, device_cu_count(),
                 std::min(workspace_bytes - lsd_at - lsd, kKvPartMax), &p.kv_run, &p.kv_runs);
   }
-  p.dqa_sb = heads_q * seqlen_q * head_dim; p.dqa_sh = seqlen_q * head_dim; p.dqa_ss = head_dim;
   p.l_sb = heads_q * seqlen_q; p.l_sh = seqlen_q; p.l_ss = 1;
   p.B = (int)batch; p.Hq = (int)heads_q; p.Hkv = (int)heads_kv;
   p.Nq = (int)seqlen_q; p.Nk = (int)seqlen_k;
@@ -485,7 +466,7 @@ static int fal_bwd_impl(const void* dout, const void* q, const void* k, const vo
   const int64_t dq_blocks = (int64_t)cdiv((int)seqlen_q, bwd_dq_block_m((int)head_dim)) * batch * heads_q;
   if (nblocks > 0x7fffffff || dq_blocks > 0x7fffffff)
     return fail(FAL_ERR_INVALID, "problem too large for one launch");
-  return run_bwd(p, (int)head_dim, is_causal != 0, dim3((unsigned)nblocks), dim3((unsigned)dq_blocks), true,
+  return run_bwd(p, (int)head_dim, is_causal != 0, dim3((unsigned)nblocks), dim3((unsigned)dq_blocks),
                  static_cast<hipStream_t>(stream));
 }
 int fal_bwd(const void* dout, const void* q, const void* k, const void* v, const void* o, const float* lse,
@@ -511,18 +492,33 @@ int fal_bwd_bf16(const void* dout, const void* q, const void* k, const void* v, 
                       1);
 }
 
+// Workspace of a packed backward: D [rows], the key-tile and query-tile lists and, for the
+// pipelined kernels, the first query tile of each sequence and the lsd array.
+struct BwdVarlenWs {
+  size_t work, qwork, first, lsd, bytes;   // offsets, total
+  int64_t cap, capq;                       // list capacities
+};
+static BwdVarlenWs bwd_varlen_ws(int64_t num_seqs, int64_t total_q, int64_t total_k, int64_t heads_q, int d, bool pipe) {
+  const int bn = pipe ? 128 : bwd_block_n(d), bm = bwd_dq_block_m(d);
+  BwdVarlenWs w{};
+  w.cap = (total_k + bn - 1) / bn + num_seqs;
+  w.capq = (total_q + bm - 1) / bm + num_seqs;
+  w.work = align256((size_t)total_q * heads_q * sizeof(float));
+  w.qwork = w.work + align256((size_t)w.cap * sizeof(int2));
+  w.bytes = w.first = w.qwork + align256((size_t)w.capq * sizeof(int2));
+  if (pipe) {
+    w.lsd = w.first + align256((size_t)num_seqs * sizeof(int));
+    w.bytes = w.lsd + align256((size_t)heads_q * w.capq * bm * 2 * sizeof(float));
+  }
+  return w;
+}
+
 size_t fal_bwd_varlen_workspace_size(int64_t num_seqs, int64_t total_q, int64_t total_k, int64_t heads_q,
                                      int64_t head_dim) {
-  const size_t rows = (size_t)total_q * heads_q;
   const int d = head_dim_ok(head_dim) ? (int)head_dim : 128;
-  const int bn = bwd_block_n(d);
-  const size_t cap = (size_t)((total_k + bn - 1) / bn + num_seqs);
-  size_t bytes = bwd_acc_bytes(rows, head_dim, false) + align256(rows * sizeof(float)) + align256(cap * sizeof(int2));
-  if (bwd_split_dq(d, false)) {
-    const int bm = bwd_dq_block_m(d);
-    bytes += align256((size_t)((total_q + bm - 1) / bm + num_seqs) * sizeof(int2));
-  }
-  return bytes;
+  // (heads_q bounds the KV heads)
+  const bool pipe = bwd_varlen_pipe(d, num_seqs, total_k, heads_q, device_cu_count());
+  return bwd_varlen_ws(num_seqs, total_q, total_k, heads_q, d, pipe).bytes;
 }
 
 static int fal_bwd_varlen_impl(const void* dout, const void* q, const void* k, const void* v, const void* o, const float* lse,
@@ -545,20 +541,27 @@ static int fal_bwd_varlen_impl(const void* dout, const void* q, const void* k, c
   int rc = fill_bwd_common(p, dout, q, k, v, o, lse, dq, dk, dv, do_strides, q_strides, k_strides, v_strides,
                            o_strides, dq_strides, dk_strides, dv_strides, false);
   if (rc) return rc;
-  const size_t need = fal_bwd_varlen_workspace_size(num_seqs, total_q, total_k, heads_q, head_dim);
-  if (!workspace || workspace_bytes < need)
-    return fail(FAL_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu", need, workspace_bytes);
+  const int d = (int)head_dim;
+  bool pipe = bwd_varlen_pipe(d, num_seqs, total_k, heads_kv, device_cu_count());
+  BwdVarlenWs w = bwd_varlen_ws(num_seqs, total_q, total_k, heads_q, d, pipe);
+  if (pipe && d != 256 && workspace_bytes < w.bytes) {   // (head_dim 256 has no other form)
+    pipe = false;
+    w = bwd_varlen_ws(num_seqs, total_q, total_k, heads_q, d, pipe);
+  }
+  if (!workspace || workspace_bytes < w.bytes)
+    return fail(FAL_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu", w.bytes, workspace_bytes);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (total_q == 0 && total_k == 0) return ok();
-  const size_t rows = (size_t)total_q * heads_q;
   char* ws = static_cast<char*>(workspace);
-  const size_t acc = bwd_acc_bytes(rows, head_dim, false);
-  p.dq_acc = acc ? reinterpret_cast<float*>(ws) : nullptr;
-  ws += acc;
   p.delta = reinterpret_cast<float*>(ws);
-  ws += align256(rows * sizeof(float));
-  int2* work = reinterpret_cast<int2*>(ws);
-  p.dqa_sb = 0; p.dqa_sh = head_dim; p.dqa_ss = heads_q * head_dim;
+  int2* work = reinterpret_cast<int2*>(ws + w.work);
+  int2* qwork = reinterpret_cast<int2*>(ws + w.qwork);
+  int* first = nullptr;
+  if (pipe) {
+    first = reinterpret_cast<int*>(ws + w.first);
+    p.lsd = reinterpret_cast<float*>(ws + w.lsd);
+    p.lsd_seq = first;
+  }
   p.l_sb = 0; p.l_sh = 1; p.l_ss = heads_q;
   p.B = 1; p.Hq = (int)heads_q; p.Hkv = (int)heads_kv;
   p.total_q = (int)total_q;
@@ -568,41 +571,40 @@ static int fal_bwd_varlen_impl(const void* dout, const void* q, const void* k, c
   p.cu_q = cu_seqlens_q;
   p.cu_k = cu_seqlens_k;
   p.work = work;
-  const int bn = bwd_block_n((int)head_dim);
-  const int cap = (int)((total_k + bn - 1) / bn + num_seqs);
+  // (the pipelined loop steps from one query head's lsd tiles to the next one's by 32 bits)
+  if (w.cap * heads_kv > 0x7fffffff || w.capq > 0x7fffffff || (pipe && w.capq >= (1 << 22)))
+    return fail(FAL_ERR_INVALID, "problem too large for one launch");
+  const int bn = pipe ? 128 : bwd_block_n(d), cap = (int)w.cap;
   int nb = cdiv((int)(max_seqlen_k > 0 ? max_seqlen_k : 1), bn);
   nb = nb < 1 ? 1 : (nb > 8192 ? 8192 : nb);
   // Every key row of every segment is covered by exactly one work item, which writes
   // its dK/dV rows (zeros when the segment has no query rows).  The schedule kernel
   // writes zeros to the rows outside all segments (dK/dV here; dQ in the query-tile
-  // schedule below, or the d 256 accumulator, zeroed for every row).
-  // key tiles grouped by sequence, the tile with the most query rows first
+  // schedule below).
+  // Key tiles grouped by sequence, longest sequence and first tile first.  Causal on the
+  // pipelined kernels, whose workgroups are few and long: the longest tiles of all sequences
+  // first (16 x 1024 rows, 32/8 heads x 128: 712 -> 639 us; not causal 851 -> 954, so there
+  // the sequences stay together).
   const ZeroRows zkv{dk, dv, dk_strides[2], dk_strides[1], dv_strides[2], dv_strides[1], (int)heads_kv,
                      (int)head_dim};
-  hipError_t e = launch_varlen_schedule(cu_seqlens_k, (int)num_seqs, (int)total_k, bn, nb, FAL_BWD_VARLEN_ORDER,
-                                        work, cap, st, &zkv);
+  hipError_t e = launch_varlen_schedule(cu_seqlens_k, (int)num_seqs, (int)total_k, bn, nb,
+                                        pipe && is_causal ? 5 : FAL_BWD_VARLEN_ORDER, work, cap, st, &zkv);
   if (e != hipSuccess) return launch_status(e, "fal_bwd_varlen schedule");
-  dim3 dq_grid(0, 0);
-  if (bwd_split_dq((int)head_dim, false)) {
-    // query tiles for the dQ kernel, grouped by sequence (as the forward's list)
-    const int bm = bwd_dq_block_m((int)head_dim);
-    const int capq = (int)((total_q + bm - 1) / bm + num_seqs);
-    int2* qwork = work + align256((size_t)cap * sizeof(int2)) / sizeof(int2);
-    int nbq = cdiv((int)(max_seqlen_q > 0 ? max_seqlen_q : 1), bm);
-    nbq = nbq < 1 ? 1 : (nbq > 8192 ? 8192 : nbq);
-    const ZeroRows zq{dq, nullptr, dq_strides[2], dq_strides[1], 0, 0, (int)heads_q, (int)head_dim};
-    e = launch_varlen_schedule(cu_seqlens_q, (int)num_seqs, (int)total_q, bm, nbq, FAL_BWD_DQ_VARLEN_ORDER, qwork,
-                               capq, st, &zq);
-    if (e != hipSuccess) return launch_status(e, "fal_bwd_varlen dq schedule");
-    p.qwork = qwork;
-    p.n_qitems = capq;
-    const int64_t groups8 = ((int64_t)capq * heads_kv + 7) / 8 * 8;
-    const int64_t nblocks = groups8 * (heads_q / heads_kv);
-    if (nblocks > 0x7fffffff) return fail(FAL_ERR_INVALID, "problem too large for one launch");
-    dq_grid = dim3((unsigned)nblocks);
-  }
-  if ((int64_t)cap * heads_kv > 0x7fffffff) return fail(FAL_ERR_INVALID, "problem too large for one launch");
-  return run_bwd(p, (int)head_dim, is_causal != 0, dim3((unsigned)(cap * heads_kv)), dq_grid, false, st);
+  // query tiles for the dQ kernel, grouped by sequence (as the forward's list)
+  const int bm = bwd_dq_block_m(d), capq = (int)w.capq;
+  int nbq = cdiv((int)(max_seqlen_q > 0 ? max_seqlen_q : 1), bm);
+  nbq = nbq < 1 ? 1 : (nbq > 8192 ? 8192 : nbq);
+  const ZeroRows zq{dq, nullptr, dq_strides[2], dq_strides[1], 0, 0, (int)heads_q, (int)head_dim};
+  e = launch_varlen_schedule(cu_seqlens_q, (int)num_seqs, (int)total_q, bm, nbq, FAL_BWD_DQ_VARLEN_ORDER, qwork,
+                             capq, st, &zq, first);
+  if (e != hipSuccess) return launch_status(e, "fal_bwd_varlen dq schedule");
+  p.qwork = qwork;
+  p.n_qitems = capq;
+  if (pipe) p.lsd_tiles = capq * (bm / bwd_pipe_bm(d));
+  const int64_t groups8 = ((int64_t)capq * heads_kv + 7) / 8 * 8;
+  const int64_t nblocks = groups8 * (heads_q / heads_kv);
+  if (nblocks > 0x7fffffff) return fail(FAL_ERR_INVALID, "problem too large for one launch");
+  return run_bwd(p, d, is_causal != 0, dim3((unsigned)(cap * heads_kv)), dim3((unsigned)nblocks), st);
 }
 int fal_bwd_varlen(const void* dout, const void* q, const void* k, const void* v, const void* o, const float* lse,
                    void* dq, void* dk, void* dv, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,

@@ -3,11 +3,11 @@
 // Math follows the reference backward (csrc/kernels/flash_attn_bwd.cu:76-107 for the
 // preprocess, :425-647 for the KV-outer kernel): D = rowsum(dO * O);
 // P = exp(S*scale - L); dV += P^T dO; dP = dO V^T; dS = P (dP - D) * scale;
-// dK += dS^T Q; dQ += dS K accumulated in fp32 and cast at the end; dK/dV of a KV
-// head sum over all query heads of its GQA group inside one workgroup.
+// dK += dS^T Q; dQ = dS K; dK/dV of a KV head sum over all query heads of its GQA group.
+// Every sum is in a fixed order, in fp32.
 //
 // Kernels:
-// * head_dim 32/64/96/128 (FA2's split form, no atomics, deterministic):
+// * FA2's split form (no atomics):
 //   - bwd_dq_kernel (query-outer, runs first): a workgroup owns 128 query rows;
 //     Q and dO stay in VGPRs, K/V tiles stream through LDS; it computes D for its
 //     rows, P, dS and dQ = dS K, written once in fp16;
@@ -16,12 +16,8 @@
 //     accumulators straight into the B operands of dV^T += dO^T P and
 //     dK^T += Q^T dS (dO^T and Q^T from the Q/dO tiles via ds_read_b64_tr_b16);
 //     dK/dV stay in registers until the end.
-//   Batched head_dim 128 and 256 run both as software-pipelined asm loops
-//   (bwd_kv_pipe_kernel, bwd_dq_kernel with PIPE).
-// * packed head_dim 256: bwd_pre_kernel (D, zeroed fp32 dQ accumulator), bwd_kernel
-//   (KV-outer, dS^T staged in LDS, dQ = dS K added with fp32 atomics; all 256 dK/dV
-//   columns accumulate in one pass, with K read from its LDS tile) and bwd_post_kernel
-//   (dQ cast to fp16).
+// * head_dim 128 and 256 (packed head_dim 128: of longer sequences) run both as
+//   software-pipelined asm loops (bwd_kv_pipe_kernel, bwd_dq_kernel with PIPE).
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -32,348 +28,9 @@
 
 namespace fal {
 
-// --------------------------------------------------------------------------
-// Preprocess: delta = rowsum(dO * O) (fp32) and zero the fp32 dQ accumulator when
-// the atomic dQ path is used.
-// One group of D/8 lanes per row (16-byte loads), reduced with xor shuffles.
-// --------------------------------------------------------------------------
-template <int D>
-constexpr int row_group() { return D / 8 <= 4 ? 4 : D / 8 <= 8 ? 8 : D / 8 <= 16 ? 16 : 32; }
-
-template <class T, int D>
-__global__ void __launch_bounds__(256)
-bwd_pre_kernel(BwdParams p, int rows, int batched) {
-  using V8 = vec8<T>;
-  constexpr int G = row_group<D>();   // lanes per row (power of two; lanes past D idle)
-  const int r = blockIdx.x * (256 / G) + threadIdx.x / G;
-  const int c = (threadIdx.x % G) * 8;
-  if (r >= rows) return;   // whole group exits together (G divides 64)
-  int64_t o_off, do_off, l_off, qa_off;
-  if (batched) {
-    const int n = r % p.Nq;
-    const int h = (r / p.Nq) % p.Hq;
-    const int b = r / (p.Nq * p.Hq);
-    o_off = b * p.o_sb + h * p.o_sh + (int64_t)n * p.o_ss;
-    do_off = b * p.do_sb + h * p.do_sh + (int64_t)n * p.do_ss;
-    l_off = b * p.l_sb + h * p.l_sh + (int64_t)n * p.l_ss;
-    qa_off = b * p.dqa_sb + h * p.dqa_sh + (int64_t)n * p.dqa_ss;
-  } else {
-    const int tok = r / p.Hq;
-    const int h = r % p.Hq;
-    o_off = (int64_t)tok * p.o_ss + h * p.o_sh;
-    do_off = (int64_t)tok * p.do_ss + h * p.do_sh;
-    l_off = (int64_t)tok * p.l_ss + h * p.l_sh;
-    qa_off = (int64_t)tok * p.dqa_ss + h * p.dqa_sh;
-  }
-  float s = 0.f;
-  if (c < D) {
-    const V8 a = ld8((const T*)p.o + o_off + c);
-    const V8 g = ld8((const T*)p.dout + do_off + c);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s = fmaf((float)a[j], (float)g[j], s);
-  }
-#pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  if (threadIdx.x % G == 0) p.delta[l_off] = s;
-  if (c >= D || !p.dq_acc) return;
-  float* qa = p.dq_acc + qa_off + c;
-  *reinterpret_cast<f32x4*>(qa) = f32x4{0.f, 0.f, 0.f, 0.f};
-  *reinterpret_cast<f32x4*>(qa + 4) = f32x4{0.f, 0.f, 0.f, 0.f};
-}
-
-// dQ = fp16(dq_acc * scale)
-template <class T, int D>
-__global__ void __launch_bounds__(256)
-bwd_post_kernel(BwdParams p, int rows, int batched) {
-  using V8 = vec8<T>;
-  constexpr int G = row_group<D>();
-  const int r = blockIdx.x * (256 / G) + threadIdx.x / G;
-  const int c = (threadIdx.x % G) * 8;
-  if (r >= rows || c >= D) return;
-  int64_t qa_off, dq_off;
-  if (batched) {
-    const int n = r % p.Nq;
-    const int h = (r / p.Nq) % p.Hq;
-    const int b = r / (p.Nq * p.Hq);
-    qa_off = b * p.dqa_sb + h * p.dqa_sh + (int64_t)n * p.dqa_ss;
-    dq_off = b * p.dq_sb + h * p.dq_sh + (int64_t)n * p.dq_ss;
-  } else {
-    const int tok = r / p.Hq;
-    const int h = r % p.Hq;
-    qa_off = (int64_t)tok * p.dqa_ss + h * p.dqa_sh;
-    dq_off = (int64_t)tok * p.dq_ss + h * p.dq_sh;
-  }
-  const f32x4 x0 = *reinterpret_cast<const f32x4*>(p.dq_acc + qa_off + c);
-  const f32x4 x1 = *reinterpret_cast<const f32x4*>(p.dq_acc + qa_off + c + 4);
-  V8 h;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    h[j] = (T)(x0[j] * p.scale);
-    h[j + 4] = (T)(x1[j] * p.scale);
-  }
-  st_u4((T*)p.dq + dq_off + c, __builtin_bit_cast(u32x4, h));
-}
-
 #ifndef FAL_PRESCALE_FP16
 #define FAL_PRESCALE_FP16 0
 #endif
-#ifndef FAL_BWD_KLDS
-#define FAL_BWD_KLDS 1   // head_dim 256: K fragments from the LDS K tile (+20%: no K registers to spill)
-#endif
-#ifndef FAL_BWD_DW
-#define FAL_BWD_DW 256   // head_dim 256: dK/dV columns held per pass (256: one pass, +11% over two passes of 128)
-#endif
-
-// --------------------------------------------------------------------------
-// Main KV-outer kernel
-// --------------------------------------------------------------------------
-template <class T, int D, int NW, int BMQ, bool CAUSAL>
-__global__ void __launch_bounds__(NW * 64)
-bwd_kernel(BwdParams p) {
-  using V8 = vec8<T>;
-  using V4 = vec4<T>;
-  static_assert(BMQ == 32, "query tile is one 32-row MFMA block");
-  constexpr int BN = NW * 32;
-  constexpr int KS = D / 16;
-  constexpr int DW = D > FAL_BWD_DW ? FAL_BWD_DW : D;   // dK/dV columns accumulated per pass
-  constexpr int NPASS = D / DW;
-  constexpr int DWB = DW / 32;
-  constexpr int DQB = D / 32;
-  constexpr int LDK = D + 8;
-  constexpr int LDQ = BMQ + 8;
-  constexpr int QCH = BMQ * D / 8;                   // 16B chunks per Q (or dO) tile
-  constexpr int QCPT = (QCH + NW * 64 - 1) / (NW * 64);
-  constexpr int CPR = D / 8;
-
-  __shared__ __attribute__((aligned(16))) T ks_s[BN * LDK];
-  __shared__ __attribute__((aligned(16))) T q_s[BMQ * LDK];
-  __shared__ __attribute__((aligned(16))) T do_s[BMQ * LDK];
-  __shared__ __attribute__((aligned(16))) T dst_s[BN * LDQ];
-  __shared__ __attribute__((aligned(16))) float l_s[BMQ];
-  __shared__ __attribute__((aligned(16))) float d_s[BMQ];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int w = tid >> 6;
-  const int l32 = lane & 31;
-  const int hh = lane >> 5;
-
-  int b, hkv, kt, q_off, k_off, nq, nk;
-  if (p.cu_q) {
-    // 1-D grid, KV head fastest: block i runs on XCD i % 8, so for a multiple of 8 KV
-    // heads each XCD walks one KV head's items in list order (grouped by sequence) and
-    // the query tiles they all read stay in its L2
-    const int2 wk = p.work[blockIdx.x / p.Hkv];
-    if (wk.x < 0) return;
-    hkv = blockIdx.x % p.Hkv;
-    b = 0;
-    kt = wk.y;
-    seg_bounds(p.cu_q, wk.x, p.total_q, q_off, nq);
-    seg_bounds(p.cu_k, wk.x, p.total_k, k_off, nk);
-  } else {
-    const int total = gridDim.x;
-    int id = blockIdx.x;
-    if ((total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
-    kt = id % p.n_ktiles;      // causal: low key tiles see the most query rows; run first
-    const int bh = id / p.n_ktiles;
-    b = bh / p.Hkv;
-    hkv = bh % p.Hkv;
-    q_off = 0;
-    k_off = 0;
-    nq = p.Nq;
-    nk = p.Nk;
-  }
-  const int n0 = kt * BN;
-  if (n0 >= nk) return;
-  const int G = p.Hq / p.Hkv;
-  const float c = p.scale_log2;
-
-  const T* kbase = (const T*)p.k + (int64_t)b * p.k_sb + (int64_t)hkv * p.k_sh + (int64_t)k_off * p.k_ss;
-  const T* vbase = (const T*)p.v + (int64_t)b * p.v_sb + (int64_t)hkv * p.v_sh + (int64_t)k_off * p.v_ss;
-
-  // K/V rows of this wave (B operands: n = key, k = head dim)
-  const int kw0 = n0 + w * 32;
-  const int key = kw0 + l32;
-  // K of this wave's keys is read from the K tile in LDS (FAL_BWD_KLDS), which leaves
-  // the registers to V and the dK/dV accumulators
-  V8 kreg[FAL_BWD_KLDS ? 1 : KS], vreg[KS];
-#pragma unroll
-  for (int t = 0; t < KS; ++t) {
-    if (!FAL_BWD_KLDS) kreg[t] = key < nk ? ld8(kbase + (int64_t)key * p.k_ss + t * 16 + hh * 8) : zero8<T>();
-    vreg[t] = key < nk ? ld8(vbase + (int64_t)key * p.v_ss + t * 16 + hh * 8) : zero8<T>();
-  }
-  // K tile, row-major, for dQ = dS K
-  for (int ch = tid; ch < BN * CPR; ch += NW * 64) {
-    const int r = ch / CPR, cc = (ch % CPR) * 8;
-    const u32x4 x = (n0 + r < nk) ? ld_u4(kbase + (int64_t)(n0 + r) * p.k_ss + cc) : u32x4{0, 0, 0, 0};
-    st_u4(ks_s + r * LDK + cc, x);
-  }
-
-  const int nqt = cdiv(nq, BMQ);
-  const int qt0 = CAUSAL ? (n0 / BMQ) : 0;
-  const int tofs_q = tr_offset(lane, LDK);
-  const int tofs_s = tr_offset(lane, LDQ);
-
-  for (int pass = 0; pass < NPASS; ++pass) {
-    const int dbase = pass * DW;
-    f32x16 dk_acc[DWB], dv_acc[DWB];
-#pragma unroll
-    for (int i = 0; i < DWB; ++i) {
-      dk_acc[i] = zero_f16();
-      dv_acc[i] = zero_f16();
-    }
-
-    for (int g = 0; g < G; ++g) {
-      const int hq = hkv * G + g;
-      const T* qbase = (const T*)p.q + (int64_t)b * p.q_sb + (int64_t)hq * p.q_sh + (int64_t)q_off * p.q_ss;
-      const T* dobase = (const T*)p.dout + (int64_t)b * p.do_sb + (int64_t)hq * p.do_sh + (int64_t)q_off * p.do_ss;
-      const float* lbase = p.lse + (int64_t)b * p.l_sb + (int64_t)hq * p.l_sh + (int64_t)q_off * p.l_ss;
-      const float* dbase_p = p.delta + (int64_t)b * p.l_sb + (int64_t)hq * p.l_sh + (int64_t)q_off * p.l_ss;
-      float* qabase = p.dq_acc + (int64_t)b * p.dqa_sb + (int64_t)hq * p.dqa_sh + (int64_t)q_off * p.dqa_ss;
-
-      u32x4 qpre[QCPT], dopre[QCPT];
-      float lpre = 0.f, dpre = 0.f;
-      auto fetch = [&](int qt) {
-        const int q0 = qt * BMQ;
-#pragma unroll
-        for (int i = 0; i < QCPT; ++i) {
-          const int ch = tid + i * NW * 64;
-          const int r = ch / CPR, cc = (ch % CPR) * 8;
-          const bool ok = (QCH % (NW * 64) == 0 || ch < QCH) && (q0 + r < nq);
-          qpre[i] = ok ? ld_u4(qbase + (int64_t)(q0 + r) * p.q_ss + cc) : u32x4{0, 0, 0, 0};
-          dopre[i] = ok ? ld_u4(dobase + (int64_t)(q0 + r) * p.do_ss + cc) : u32x4{0, 0, 0, 0};
-        }
-        if (tid < BMQ) {
-          const int r = q0 + tid;
-          float lv = INFINITY, dv = 0.f;
-          if (r < nq) {
-            const float L = lbase[(int64_t)r * p.l_ss];
-            lv = (L == -INFINITY) ? INFINITY : L * kLog2e;
-            dv = dbase_p[(int64_t)r * p.l_ss];
-          }
-          lpre = lv;
-          dpre = dv;
-        }
-      };
-      auto stash = [&]() {
-#pragma unroll
-        for (int i = 0; i < QCPT; ++i) {
-          const int ch = tid + i * NW * 64;
-          if (QCH % (NW * 64) == 0 || ch < QCH) {
-            const int r = ch / CPR, cc = (ch % CPR) * 8;
-            st_u4(q_s + r * LDK + cc, qpre[i]);
-            st_u4(do_s + r * LDK + cc, dopre[i]);
-          }
-        }
-        if (tid < BMQ) {
-          l_s[tid] = lpre;
-          d_s[tid] = dpre;
-        }
-      };
-
-      if (qt0 < nqt) {
-        fetch(qt0);
-        __syncthreads();   // previous users of q_s/do_s are done
-        stash();
-      }
-      __syncthreads();
-
-      for (int qt = qt0; qt < nqt; ++qt) {
-        const int q0 = qt * BMQ;
-        if (qt + 1 < nqt) fetch(qt + 1);
-        const bool active = !CAUSAL || (q0 + BMQ - 1 >= kw0);
-        if (active) {
-          f32x16 s = zero_f16(), dp = zero_f16();
-#pragma unroll
-          for (int t = 0; t < KS; ++t) {
-            s = mfma32(ld8(q_s + l32 * LDK + t * 16 + hh * 8),
-                       FAL_BWD_KLDS ? ld8(ks_s + (w * 32 + l32) * LDK + t * 16 + hh * 8) : kreg[t], s);
-            dp = mfma32(ld8(do_s + l32 * LDK + t * 16 + hh * 8), vreg[t], dp);
-          }
-          // P and dS (element i: query q0 + (i/4)*8 + hh*4 + i%4, key `key`)
-#pragma unroll
-          for (int g4 = 0; g4 < 4; ++g4) {
-            const f32x4 lv = *reinterpret_cast<const f32x4*>(l_s + g4 * 8 + hh * 4);
-            const f32x4 dv = *reinterpret_cast<const f32x4*>(d_s + g4 * 8 + hh * 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int i = g4 * 4 + e;
-              const int qrow = q0 + g4 * 8 + hh * 4 + e;
-              float pv = fast_exp2(fmaf(s[i], c, -lv[e]));
-              if (key >= nk || (CAUSAL && key > qrow)) pv = 0.f;
-              s[i] = pv;
-              dp[i] = pv * (dp[i] - dv[e]);
-            }
-          }
-          // dV^T += dO^T P ; dK^T += Q^T dS  (this pass's head-dim columns)
-#pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            const V8 pb = cvt8t<T>(s, ks);
-            const V8 sb = cvt8t<T>(dp, ks);
-#pragma unroll
-            for (int db = 0; db < DWB; ++db) {
-              const int col = dbase + db * 32;
-              dv_acc[db] = mfma32(kslab_tr(do_s + tofs_q + col, ks * 16, hh, LDK), pb, dv_acc[db]);
-              dk_acc[db] = mfma32(kslab_tr(q_s + tofs_q + col, ks * 16, hh, LDK), sb, dk_acc[db]);
-            }
-          }
-          if (pass == 0) {
-            // dS^T (fp16) into LDS: row = key (local), columns = query rows
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-              V4 h;
-#pragma unroll
-              for (int e = 0; e < 4; ++e) h[e] = (T)dp[g4 * 4 + e];
-              *reinterpret_cast<V4*>(dst_s + (w * 32 + l32) * LDQ + g4 * 8 + hh * 4) = h;
-            }
-          }
-        }
-        __syncthreads();   // dS^T complete; q_s/do_s reads done
-
-        if (pass == 0) {
-          // dQ[q0:q0+32, db*32:+32] += dS K over the key blocks that are active
-          for (int db = w; db < DQB; db += NW) {
-            f32x16 acc = zero_f16();
-            for (int ks = 0; ks < BN / 16; ++ks) {
-              const int kwave0 = n0 + (ks >> 1) * 32;   // first key of the owning wave
-              if (CAUSAL && q0 + BMQ - 1 < kwave0) break;
-              acc = mfma32(kslab_tr(dst_s + tofs_s, ks * 16, hh, LDQ),
-                           kslab_tr(ks_s + tofs_q + db * 32, ks * 16, hh, LDK), acc);
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int qrow = q0 + (i >> 2) * 8 + hh * 4 + (i & 3);
-              if (qrow < nq)
-                unsafeAtomicAdd(qabase + (int64_t)qrow * p.dqa_ss + db * 32 + l32, acc[i]);
-            }
-          }
-        }
-        if (qt + 1 < nqt) stash();
-        __syncthreads();
-      }
-    }
-
-    // write dK (scaled) and dV for this pass's columns
-    if (key < nk) {
-      T* dkrow = (T*)p.dk + (int64_t)b * p.dk_sb + (int64_t)hkv * p.dk_sh + (int64_t)(k_off + key) * p.dk_ss;
-      T* dvrow = (T*)p.dv + (int64_t)b * p.dv_sb + (int64_t)hkv * p.dv_sh + (int64_t)(k_off + key) * p.dv_ss;
-#pragma unroll
-      for (int db = 0; db < DWB; ++db)
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          V4 hk, hv;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            hk[e] = (T)(dk_acc[db][g4 * 4 + e] * p.scale);
-            hv[e] = (T)dv_acc[db][g4 * 4 + e];
-          }
-          const int col = dbase + db * 32 + g4 * 8 + hh * 4;
-          *reinterpret_cast<V4*>(dkrow + col) = hk;
-          *reinterpret_cast<V4*>(dvrow + col) = hv;
-        }
-    }
-  }
-}
 
 // Scheduling fence between MFMA steps of the head_dim-128 kernel: keeps the compiler
 // from hoisting every operand read of a phase at once (which overflows the 256-register
@@ -412,7 +69,7 @@ bwd_kernel(BwdParams p) {
 #ifndef FAL_BWD2_NW
 #define FAL_BWD2_NW 4   // waves per workgroup: 4 (64 keys, 2 workgroups per CU) or 8 (128 keys, double-buffered Q/dO)
 #endif
-template <class T, int D, bool CAUSAL, bool FUSED>
+template <class T, int D, bool CAUSAL>
 __global__ void __launch_bounds__(FAL_BWD2_NW * 64) __attribute__((amdgpu_waves_per_eu(2, 8)))
 bwd2_kernel(BwdParams p) {
   using V8 = vec8<T>;
@@ -435,17 +92,12 @@ bwd2_kernel(BwdParams p) {
   constexpr int QIPT = BMQ * CPR / (NW * 64);
   static_assert(BMQ * CPR % (NW * 64) == 0, "Q tile must split evenly over the waves");
   static_assert((DBUF ? 2 : 1) * 2 * QPART * 2 >= NKG * 32 * D * 4, "dK/dV reduction reuses the Q/dO buffers");
-  static_assert(!(FUSED && PRESCALE), "the fused dQ product needs the unscaled K tile");
-  static_assert(!FUSED || NW == 4, "the fused dQ product splits 64 rows x D over four waves");
-  constexpr int LDQ = BMQ + 8;            // dS^T tile row stride (fused): 64 query rows + pad
 
   __shared__ __attribute__((aligned(1024))) T ks_s[KPART];
   __shared__ __attribute__((aligned(1024))) T vs_s[KPART];
   __shared__ __attribute__((aligned(1024))) T qd_s[(DBUF ? 2 : 1) * 2 * QPART];   // [buffer][Q, dO]
   __shared__ float l_s[2][BMQ];
   __shared__ float d_s[2][BMQ];
-  // fused: dS^T of the current item, row = key of the tile, column = query row of the item
-  __shared__ __attribute__((aligned(16))) T dst_s[FUSED ? BN * LDQ : 8];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -725,52 +377,6 @@ bwd2_kernel(BwdParams p) {
             }
           }
           __builtin_amdgcn_s_setprio(0);
-          if constexpr (FUSED) {
-            // this wave's dS^T block (32 keys x 32 query rows) into the tile
-            T* drow = dst_s + (kg * 32 + l32) * LDQ + qh * 32 + hh * 4;
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-              V4 h;
-#pragma unroll
-              for (int e = 0; e < 4; ++e) h[e] = (T)dp[g4 * 4 + e];
-              *reinterpret_cast<V4*>(drow + g4 * 8) = h;
-            }
-          }
-        } else if constexpr (FUSED) {
-          // every key of this wave is past every query row of its half: dS = 0
-          T* drow = dst_s + (kg * 32 + l32) * LDQ + qh * 32 + hh * 4;
-#pragma unroll
-          for (int g4 = 0; g4 < 4; ++g4) *reinterpret_cast<u32x2*>(drow + g4 * 8) = u32x2{0, 0};
-        }
-        if constexpr (FUSED) {
-          // dQ[q, :] += dS[q, keys] K[keys, :] over the tile's 64 keys, added to the fp32
-          // accumulator with atomics (the reference's scheme, flash_attn_bwd.cu:602-620).
-          // Wave (kg, qh) takes query half qh and head-dim columns kg*D/2 .. +D/2.
-          __syncthreads();                // barrier C: the dS^T tile is complete
-          constexpr int QDB = D / 64;     // 32-wide head-dim blocks per wave
-          const int tofs_s = tr_offset(lane, LDQ) + qh * 32;
-          // one buffer resource over the item's accumulator rows: adds to rows past the
-          // end of the sequence fall outside it and are dropped
-          const float* qa = p.dq_acc + (int64_t)b * p.dqa_sb + (int64_t)(hkv * G + cur_hq) * p.dqa_sh +
-                            (int64_t)(q_off + q0) * p.dqa_ss;
-          const __amdgpu_buffer_rsrc_t qrs =
-              make_rsrc(qa, (uint32_t)min((int64_t)max(nq - q0, 0) * p.dqa_ss * 4, (int64_t)0x7fffffff));
-          // lane part of the byte offset in a VGPR, the row step of element i in the
-          // instruction's scalar offset
-          const int qrow_bytes = __builtin_amdgcn_readfirstlane((int)p.dqa_ss * 4);
-          const int qoff = ((qh * 32 + hh * 4) * (int)p.dqa_ss + kg * QDB * 32 + l32) * 4;
-#pragma unroll
-          for (int j = 0; j < QDB; ++j) {
-            // one 32-column block at a time (16 accumulator registers)
-            f32x16 qacc = zero_f16();
-#pragma unroll
-            for (int ks = 0; ks < BN / 16; ++ks)
-              qacc = mfma32(kslab_tr(dst_s + tofs_s, ks * 16, hh, LDQ), trk(ks_s, kg * QDB + j, ks * 16), qacc);
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-              __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(qacc[i], qrs, qoff + j * 128,
-                                                              ((i >> 2) * 8 + (i & 3)) * qrow_bytes, 0);
-          }
         }
         if (!DBUF && item + 1 < nitems_q) {
           __syncthreads();                // barrier B: every wave is done with this item's tile
@@ -831,9 +437,6 @@ bwd2_kernel(BwdParams p) {
 // B2 x 16/8 heads x 2048 causal 957 -> 322 us, B2 x 16 x 4096 2147 -> 942 (non-causal
 // 4053 -> 1709).
 // --------------------------------------------------------------------------
-#ifndef FAL_BWD_PIPE
-#define FAL_BWD_PIPE 1
-#endif
 constexpr int kPipeBN = 128;    // keys per workgroup
 // dK/dV hand-off in LDS after the loop: per wave, dV then dK*scale, D/8 pieces of 512
 // bytes each, kKvOStr apart so the row-wise reads of the epilogue spread over the banks
@@ -841,9 +444,11 @@ constexpr int kKvOStr = 528;
 template <int D>
 constexpr int pipe_bm() { return D == 256 ? 32 : 64; }   // query rows per item
 
-template <class T, int D, bool CAUSAL, bool SPLIT>
+enum KvForm { kKvWhole, kKvSplit, kKvPacked };
+template <class T, int D, bool CAUSAL, KvForm FORM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 bwd_kv_pipe_kernel(BwdParams p) {
+  constexpr bool SPLIT = FORM == kKvSplit, PACKED = FORM == kKvPacked;
   using V8 = vec8<T>;
   using TL = SwizzledTile<D>;
   constexpr int CPR = TL::CPR, KS = D / 16, kPipeBM = pipe_bm<D>();
@@ -860,11 +465,21 @@ bwd_kv_pipe_kernel(BwdParams p) {
 
   // work item: one or two 128-key tiles of one (batch, KV head); causal tiles are
   // paired (kt, n-1-kt) so every workgroup has the same number of items.  SPLIT (kv_run set):
-  // one run of one key tile's items.
+  // one run of one key tile's items.  PACKED: one key tile of one sequence; KV heads fastest,
+  // so for a multiple of 8 of them an XCD walks one head's list, grouped by sequence, and the
+  // query tiles it reads stay in its L2.
   const int nkt = cdiv(p.Nk, kPipeBN);
   const int total = gridDim.x;
-  int id = blockIdx.x, run = 0, kit, bh;
-  if (SPLIT) {
+  int id = blockIdx.x, run = 0, kit, bh, q_off = 0, k_off = 0, nq = p.Nq, nk = p.Nk, lsd0 = 0;
+  if (PACKED) {
+    const int2 wk = p.work[id / p.Hkv];
+    if (wk.x < 0) return;
+    bh = id % p.Hkv;
+    kit = wk.y;
+    seg_bounds(p.cu_q, wk.x, p.total_q, q_off, nq);
+    seg_bounds(p.cu_k, wk.x, p.total_k, k_off, nk);
+    lsd0 = p.lsd_seq[wk.x] * (128 / kPipeBM);
+  } else if (SPLIT) {
     // the first key tiles of all heads first (an XCD keeps whole heads when they divide by 8):
     // under a causal mask they have the most items
     int units = p.B * p.Hkv, u = 0;
@@ -885,9 +500,8 @@ bwd_kv_pipe_kernel(BwdParams p) {
   }
   const int slot = (bh * nkt + kit) * p.kv_runs + run;   // (SPLIT) of this workgroup's sums
   const int b = bh / p.Hkv, hkv = bh % p.Hkv;
-  const int kt_b = (CAUSAL && !SPLIT && nkt - 1 - kit != kit) ? nkt - 1 - kit : -1;
+  const int kt_b = (CAUSAL && FORM == kKvWhole && nkt - 1 - kit != kit) ? nkt - 1 - kit : -1;
   const int G = p.Hq / p.Hkv;
-  const int nq = p.Nq, nk = p.Nk;
   const int nqt = cdiv(nq, kPipeBM);
   int run_len = 0, nruns = 1;
   if (SPLIT) {
@@ -946,12 +560,12 @@ bwd_kv_pipe_kernel(BwdParams p) {
   auto load_kv = [&](int kt) {
     // one resource per key tile: its rows inside the sequence, offsets from its first row
     const int n0 = kt * kPipeBN;
-    const int64_t rows = min(max((int64_t)p.Nk - n0, (int64_t)0), (int64_t)kPipeBN);
+    const int64_t rows = min(max((int64_t)nk - n0, (int64_t)0), (int64_t)kPipeBN);
     const __amdgpu_buffer_rsrc_t krs =
-        make_rsrc((const T*)p.k + (int64_t)b * p.k_sb + (int64_t)hkv * p.k_sh + (int64_t)n0 * p.k_ss,
+        make_rsrc((const T*)p.k + (int64_t)b * p.k_sb + (int64_t)hkv * p.k_sh + (int64_t)(k_off + n0) * p.k_ss,
                   (uint32_t)(rows * p.k_ss * 2));
     const __amdgpu_buffer_rsrc_t vrs =
-        make_rsrc((const T*)p.v + (int64_t)b * p.v_sb + (int64_t)hkv * p.v_sh + (int64_t)n0 * p.v_ss,
+        make_rsrc((const T*)p.v + (int64_t)b * p.v_sb + (int64_t)hkv * p.v_sh + (int64_t)(k_off + n0) * p.v_ss,
                   (uint32_t)(rows * p.v_ss * 2));
     const int r = ws * 32 + l32;
     const int ko = (int)(r * p.k_ss * 2) + hh * 16, vo = (int)(r * p.v_ss * 2) + hh * 16;
@@ -965,7 +579,7 @@ bwd_kv_pipe_kernel(BwdParams p) {
   // each tile loads its own first)
   constexpr bool AHEAD = D == 128;
   if (AHEAD) load_kv(kit);
-  for (int tile_i = 0; tile_i < (SPLIT || !CAUSAL ? 1 : 2); ++tile_i) {
+  for (int tile_i = 0; tile_i < (FORM != kKvWhole || !CAUSAL ? 1 : 2); ++tile_i) {
     const int kt = tile_i == 0 ? kit : kt_b;
     if (kt < 0) break;
     const int n0 = kt * kPipeBN;
@@ -982,10 +596,11 @@ bwd_kv_pipe_kernel(BwdParams p) {
       const int h0 = part ? __builtin_amdgcn_readfirstlane(i0 / ntq) : 0;
       const int hq0 = hkv * G + h0, q0 = qt0 + i0 - h0 * ntq;
       const uint64_t qb = (uint64_t)(uintptr_t)((const T*)p.q + (int64_t)b * p.q_sb + (int64_t)hq0 * p.q_sh +
-                                                (int64_t)q0 * kPipeBM * p.q_ss);
+                                                ((int64_t)q0 * kPipeBM + q_off) * p.q_ss);
       const uint64_t dob = (uint64_t)(uintptr_t)((const T*)p.dout + (int64_t)b * p.do_sb +
-                                                 (int64_t)hq0 * p.do_sh + (int64_t)q0 * kPipeBM * p.do_ss);
-      const uint64_t lb = (uint64_t)(uintptr_t)(p.lsd + (((int64_t)b * p.Hq + hq0) * nqt + q0) * 2 * kPipeBM);
+                                                 (int64_t)hq0 * p.do_sh + ((int64_t)q0 * kPipeBM + q_off) * p.do_ss);
+      const uint64_t lb =
+          (uint64_t)(uintptr_t)(p.lsd + (((int64_t)b * p.Hq + hq0) * p.lsd_tiles + lsd0 + q0) * 2 * kPipeBM);
       const int64_t qwrap = p.q_sh * 2 - (int64_t)(ntq - 1) * qstep - qhalf;
       const int64_t dwrap = p.do_sh * 2 - (int64_t)(ntq - 1) * dstep - dhalf;
       const uint32_t p_qb_lo = (uint32_t)qb, p_qb_hi = (uint32_t)(qb >> 32) & 0xffffu;
@@ -995,7 +610,8 @@ bwd_kv_pipe_kernel(BwdParams p) {
       const uint32_t p_qw_lo = (uint32_t)qwrap, p_qw_hi = (uint32_t)((uint64_t)qwrap >> 32);
       const uint32_t p_ds_lo = (uint32_t)(dstep - dhalf), p_ds_hi = (uint32_t)((uint64_t)(dstep - dhalf) >> 32);
       const uint32_t p_dw_lo = (uint32_t)dwrap, p_dw_hi = (uint32_t)((uint64_t)dwrap >> 32);
-      const uint32_t p_ldw = (uint32_t)(1 + qt0) * 2 * kPipeBM * 4;   // last tile of a head -> first of the next
+      // last tile of a head -> first of the next
+      const uint32_t p_ldw = (uint32_t)(p.lsd_tiles - nqt + 1 + qt0) * 2 * kPipeBM * 4;
       const int p_qt0 = qt0, p_qs0 = q0, p_nitems = nitems;
       const int p_part = SPLIT ? __builtin_amdgcn_readfirstlane(nruns - 1) : 0;
       // dV and dK sums of this wave's 32 keys
@@ -1025,9 +641,9 @@ bwd_kv_pipe_kernel(BwdParams p) {
       // are dropped (no branch, no 64-bit address per store)
       const int nkw = max(min(nk - kw0, 32), 0);
       const __amdgpu_buffer_rsrc_t rs[2] = {
-          make_rsrc((T*)p.dv + (int64_t)b * p.dv_sb + (int64_t)hkv * p.dv_sh + (int64_t)kw0 * p.dv_ss,
+          make_rsrc((T*)p.dv + (int64_t)b * p.dv_sb + (int64_t)hkv * p.dv_sh + (int64_t)(k_off + kw0) * p.dv_ss,
                     (uint32_t)((int64_t)nkw * p.dv_ss * 2)),
-          make_rsrc((T*)p.dk + (int64_t)b * p.dk_sb + (int64_t)hkv * p.dk_sh + (int64_t)kw0 * p.dk_ss,
+          make_rsrc((T*)p.dk + (int64_t)b * p.dk_sb + (int64_t)hkv * p.dk_sh + (int64_t)(k_off + kw0) * p.dk_ss,
                     (uint32_t)((int64_t)nkw * p.dk_ss * 2))};
       const int vo[2] = {((lane / CPR) * (int)p.dv_ss + cch * 8) * 2, ((lane / CPR) * (int)p.dk_ss + cch * 8) * 2};
       const int rstep[2] = {(int)p.dv_ss * 2 * RPI, (int)p.dk_ss * 2 * RPI};   // rows of an instruction, in bytes
@@ -1114,9 +730,6 @@ constexpr int kDqOStr = 1040;
 #ifndef FAL_BWD_DQ_WPE
 #define FAL_BWD_DQ_WPE 2
 #endif
-#ifndef FAL_BWD_DQ_PIPE
-#define FAL_BWD_DQ_PIPE 1   // batched head_dim 128 (and 256): software-pipelined key-tile loop (fal_dq_pipe.inc)
-#endif
 template <class T, int D, int NW, int BN, bool CAUSAL, bool PIPE = false>
 __global__ void __launch_bounds__(NW * 64)
 __attribute__((amdgpu_waves_per_eu(PIPE ? 1 : FAL_BWD_DQ_WPE, PIPE ? 1 : 8)))
@@ -1147,7 +760,7 @@ bwd_dq_kernel(BwdParams p) {
   const int l32 = lane & 31;
   const int hh = lane >> 5;
 
-  int b, hq, qt_a, qt_b = -1, q_off, k_off, nq, nk;
+  int b, hq, qt_a, qt_b = -1, q_off, k_off, nq, nk, lsd0 = 0;
   if (p.cu_q) {
     // 1-D grid: (work item, KV head) groups dealt round-robin to the 8 XCDs in list
     // order, the query heads of a group back to back on one XCD (they read the same
@@ -1164,6 +777,7 @@ bwd_dq_kernel(BwdParams p) {
     qt_a = wk.y;
     seg_bounds(p.cu_q, wk.x, p.total_q, q_off, nq);
     seg_bounds(p.cu_k, wk.x, p.total_k, k_off, nk);
+    if (PIPE && p.lsd) lsd0 = p.lsd_seq[wk.x] * (BM / kPipeBM);
   } else {
     // heads of one KV head and the query tiles of a head are dealt to one XCD together
     const int total = gridDim.x;
@@ -1231,7 +845,7 @@ bwd_dq_kernel(BwdParams p) {
     // whose exponent c * x is -inf, and -D = 0.
     const int nt = cdiv(nq, kPipeBM);
     if (row < nt * kPipeBM) {
-      float* t = p.lsd + (((int64_t)b * p.Hq + hq) * nt + row / kPipeBM) * 2 * kPipeBM + row % kPipeBM;
+      float* t = p.lsd + (((int64_t)b * p.Hq + hq) * p.lsd_tiles + lsd0 + row / kPipeBM) * 2 * kPipeBM + row % kPipeBM;
       const bool live = row < nq && lrow2 != INFINITY;
       t[0] = live ? -lrow2 / c : (c > 0.f ? -INFINITY : INFINITY);
       t[kPipeBM] = row < nq ? -drow : 0.f;
@@ -1478,23 +1092,24 @@ bwd_dq_kernel(BwdParams p) {
 // --------------------------------------------------------------------------
 // Launchers
 // --------------------------------------------------------------------------
-constexpr int kBwdNW = 4;
-
-// head dims on the split path (dQ kernel + dK/dV kernel); 256 keeps the atomic kernel,
-// whose dK/dV accumulators would not fit the split kernel's registers
+// head dims of bwd2_kernel (256 has the pipelined kernels only)
 constexpr bool split_d(int d) { return d == 32 || d == 64 || d == 96 || d == 128; }
-// head dims whose KV-outer kernel also forms dQ = dS K (fp32 atomics into an accumulator,
-// five products instead of the split form's seven)
-#ifndef FAL_BWD_FUSED
-#define FAL_BWD_FUSED 0
-#endif
-constexpr bool fused_d(int d) { return FAL_BWD_FUSED && (d == 64 || d == 128); }
 
 int bwd_block_n(int d) {
-  return split_d(d) ? FAL_BWD2_NW * 16 : kBwdNW * 32;
+  return split_d(d) ? FAL_BWD2_NW * 16 : kPipeBN;
 }
 
-bool bwd_pipe(int d) { return FAL_BWD_PIPE && (d == 128 || d == 256); }
+bool bwd_pipe(int d) { return d == 128 || d == 256; }
+// Packed head_dim 256 has no other form (its fp32-atomic one took 2.5 to 3.7 times as long: 16
+// sequences of up to 2048, 16/4 heads, causal 1909 -> 639 us, 4 of 300, 8/1 heads 556 -> 150).
+// At head_dim 128 bwd2_kernel keeps two workgroups of 64 keys per CU, which hide each other's
+// start and end; the pipelined kernel's one of 128 keys needs sequences of many items and a
+// grid of several rounds.  us, bwd2_kernel -> this, 32/8 heads causal: 16 x 1024 697 -> 648,
+// 32 x 512 497 -> 452, 16 of 64 to 2048 564 -> 553 (not causal 905 -> 862); but 32 of 16 to 512
+// 214 -> 229, and 4 of 64 to 2048 (264 key tiles) 130 -> 135.
+bool bwd_varlen_pipe(int d, int64_t num_seqs, int64_t total_k, int64_t heads_kv, int ncu) {
+  return d == 256 || (d == 128 && total_k >= 512 * num_seqs && total_k / kPipeBN * heads_kv >= 3 * (int64_t)ncu);
+}
 int bwd_pipe_bm(int d) { return d == 256 ? pipe_bm<256>() : pipe_bm<128>(); }
 
 // A dK/dV workgroup takes about 1.85 us per item and 8 us besides, so a grid smaller than the
@@ -1560,17 +1175,24 @@ size_t bwd_kv_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, i
 template <class T, int D>
 static hipError_t launch_bwd_t(const BwdParams& p, int causal, dim3 grid, hipStream_t st) {
   if constexpr (D == 128 || D == 256) {
-    if (!p.cu_q && p.lsd) {
+    if (p.cu_q && p.lsd) {
+      if (causal)
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, true, kKvPacked>), grid, dim3(256), 0, st, p);
+      else
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, false, kKvPacked>), grid, dim3(256), 0, st, p);
+      return hipGetLastError();
+    }
+    if (p.lsd) {
       const int nkt = cdiv(p.Nk, kPipeBN), tiles = nkt * p.B * p.Hkv;
       grid.x = p.kv_run ? (unsigned)(tiles * p.kv_runs) : (unsigned)((causal ? (nkt + 1) / 2 : nkt) * p.B * p.Hkv);
       if (causal && !p.kv_run)
-        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, true, false>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, true, kKvWhole>), grid, dim3(256), 0, st, p);
       else if (causal)
-        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, true, true>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, true, kKvSplit>), grid, dim3(256), 0, st, p);
       else if (!p.kv_run)
-        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, false, false>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, false, kKvWhole>), grid, dim3(256), 0, st, p);
       else
-        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, false, true>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((bwd_kv_pipe_kernel<T, D, false, kKvSplit>), grid, dim3(256), 0, st, p);
       if (p.kv_run) {
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -1583,20 +1205,15 @@ static hipError_t launch_bwd_t(const BwdParams& p, int causal, dim3 grid, hipStr
     }
   }
   if constexpr (split_d(D)) {
-    constexpr bool kFused = fused_d(D);
     // batched causal: one workgroup per pair of key tiles
     if (!p.cu_q && causal) grid.x = (unsigned)((p.n_ktiles + 1) / 2) * p.B * p.Hkv;
     if (causal)
-      hipLaunchKernelGGL((bwd2_kernel<T, D, true, kFused>), grid, dim3(FAL_BWD2_NW * 64), 0, st, p);
+      hipLaunchKernelGGL((bwd2_kernel<T, D, true>), grid, dim3(FAL_BWD2_NW * 64), 0, st, p);
     else
-      hipLaunchKernelGGL((bwd2_kernel<T, D, false, kFused>), grid, dim3(FAL_BWD2_NW * 64), 0, st, p);
-  } else {
-    if (causal)
-      hipLaunchKernelGGL((bwd_kernel<T, D, kBwdNW, 32, true>), grid, dim3(kBwdNW * 64), 0, st, p);
-    else
-      hipLaunchKernelGGL((bwd_kernel<T, D, kBwdNW, 32, false>), grid, dim3(kBwdNW * 64), 0, st, p);
+      hipLaunchKernelGGL((bwd2_kernel<T, D, false>), grid, dim3(FAL_BWD2_NW * 64), 0, st, p);
+    return hipGetLastError();
   }
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 template <int D>
 static hipError_t launch_bwd_d(const BwdParams& p, int causal, dim3 grid, hipStream_t st) {
@@ -1608,7 +1225,6 @@ static hipError_t launch_bwd_d(const BwdParams& p, int causal, dim3 grid, hipStr
 #endif
 constexpr int kDqNW = 4;
 
-bool bwd_split_dq(int d, bool batched) { return (split_d(d) && !fused_d(d)) || (batched && bwd_pipe(d)); }
 int bwd_dq_block_m(int d) {
   (void)d;
   return kDqNW * 32;
@@ -1619,7 +1235,7 @@ static hipError_t launch_bwd_dq_t(const BwdParams& p, int causal, dim3 grid, hip
   if (!p.cu_q && causal && FAL_BWD_DQ_PAIR)
     grid.x = (unsigned)((cdiv(p.Nq, kDqNW * 32) + 1) / 2) * p.B * p.Hq;
   if constexpr (D == 128 || D == 256) {
-    if (!p.cu_q && FAL_BWD_DQ_PIPE) {
+    if (p.lsd) {
       constexpr int BN = 8192 / D;
       if (causal)
         hipLaunchKernelGGL((bwd_dq_kernel<T, D, kDqNW, BN, true, true>), grid, dim3(kDqNW * 64), 0, st, p);
@@ -1661,47 +1277,6 @@ hipError_t launch_bwd(const BwdParams& p, int d, int causal, dim3 grid, hipStrea
     case 96: return launch_bwd_d<96>(p, causal, grid, st);
     case 128: return launch_bwd_d<128>(p, causal, grid, st);
     case 256: return launch_bwd_d<256>(p, causal, grid, st);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-template <class T, int D, bool PRE>
-static hipError_t launch_rowwise_t(const BwdParams& p, int batched, hipStream_t st) {
-  const int rows = batched ? p.B * p.Hq * p.Nq : p.total_q * p.Hq;
-  if (rows == 0) return hipSuccess;
-  constexpr int RPB = 256 / row_group<D>();
-  dim3 grid(cdiv(rows, RPB));
-  if (PRE)
-    hipLaunchKernelGGL((bwd_pre_kernel<T, D>), grid, dim3(256), 0, st, p, rows, batched);
-  else
-    hipLaunchKernelGGL((bwd_post_kernel<T, D>), grid, dim3(256), 0, st, p, rows, batched);
-  return hipGetLastError();
-}
-
-template <int D, bool PRE>
-static hipError_t launch_rowwise(const BwdParams& p, int batched, hipStream_t st) {
-  return p.bf16 ? launch_rowwise_t<bf16_t, D, PRE>(p, batched, st) : launch_rowwise_t<half_t, D, PRE>(p, batched, st);
-}
-
-hipError_t launch_bwd_pre(const BwdParams& p, int d, int batched, hipStream_t st) {
-  switch (d) {
-    case 32: return launch_rowwise<32, true>(p, batched, st);
-    case 64: return launch_rowwise<64, true>(p, batched, st);
-    case 96: return launch_rowwise<96, true>(p, batched, st);
-    case 128: return launch_rowwise<128, true>(p, batched, st);
-    case 256: return launch_rowwise<256, true>(p, batched, st);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch_bwd_post(const BwdParams& p, int d, hipStream_t st) {
-  const int batched = p.cu_q == nullptr;
-  switch (d) {
-    case 32: return launch_rowwise<32, false>(p, batched, st);
-    case 64: return launch_rowwise<64, false>(p, batched, st);
-    case 96: return launch_rowwise<96, false>(p, batched, st);
-    case 128: return launch_rowwise<128, false>(p, batched, st);
-    case 256: return launch_rowwise<256, false>(p, batched, st);
     default: return hipErrorInvalidValue;
   }
 }

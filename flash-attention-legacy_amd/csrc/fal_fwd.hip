@@ -940,18 +940,28 @@ fwd_combine_kernel(FwdParams p) {
 // that, for causal attention, the most expensive tiles start first
 // (descending=1: tile t costs ~t+1 KV tiles in the forward) or, for the KV-outer
 // backward, the tiles with the most query rows below them start first
-// (descending=0).  Unused trailing slots get (-1, -1).
+// (descending=0), or by the tiles from this one to the sequence's end, most first
+// (descending=5: the same for sequences of unequal length).  Unused trailing slots get
+// (-1, -1).  `first` (optional) receives an offset per sequence such that the sequences'
+// tiles, counted from it, do not overlap.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(1024)
 varlen_schedule_kernel(const int* __restrict__ cu, int num_seqs, int rows, int tile, int nbuckets,
-                       int descending, int2* __restrict__ work, int capacity, ZeroRows zero) {
+                       int descending, int2* __restrict__ work, int capacity, ZeroRows zero, int* __restrict__ first) {
   extern __shared__ int sh[];            // [nbuckets] counts, then [nbuckets] cursors
   int* cnt = sh;
   int* cur = sh + nbuckets;
-  __shared__ int seg_end;
+  __shared__ int seg_end, ntiles;
   for (int i = threadIdx.x; i < nbuckets; i += blockDim.x) cnt[i] = 0;
-  if (threadIdx.x == 0) seg_end = 0;
+  if (threadIdx.x == 0) seg_end = ntiles = 0;
   __syncthreads();
+  if (first)
+    for (int s = threadIdx.x; s < num_seqs; s += blockDim.x) {
+      int off, len;
+      seg_bounds(cu, s, rows, off, len);
+      const int nt = cdiv(len, tile);
+      first[s] = min(atomicAdd(&ntiles, nt), capacity - nt);
+    }
   if (zero.a) {
     // rows [0, start of segment 0) and [end of the last segment, rows) are in no segment
     // (for a monotone cu_seqlens): write zeros there, as the reference's per-sequence
@@ -962,15 +972,15 @@ varlen_schedule_kernel(const int* __restrict__ cu, int num_seqs, int rows, int t
       atomicMax(&seg_end, off + len);
     }
     __syncthreads();
-    int first = rows, flen = 0;
-    if (num_seqs > 0) seg_bounds(cu, 0, rows, first, flen);
+    int begin = rows, flen = 0;
+    if (num_seqs > 0) seg_bounds(cu, 0, rows, begin, flen);
     const int last = seg_end;
     const int cpr = zero.heads * (zero.d / 8);   // 16-byte chunks per row
-    const int nlo = first, nhi = rows - max(last, first);
+    const int nlo = begin, nhi = rows - max(last, begin);
     const int64_t nchunks = (int64_t)(nlo + nhi) * cpr;
     for (int64_t i = threadIdx.x; i < nchunks; i += blockDim.x) {
       const int rr = (int)(i / cpr);
-      const int r = rr < nlo ? rr : max(last, first) + (rr - nlo);
+      const int r = rr < nlo ? rr : max(last, begin) + (rr - nlo);
       const int ch = (int)(i % cpr);
       const int h = ch / (zero.d / 8), c8 = (ch % (zero.d / 8)) * 8;
       st_u4(static_cast<half_t*>(zero.a) + (int64_t)r * zero.a_row + (int64_t)h * zero.a_head + c8,
@@ -980,7 +990,8 @@ varlen_schedule_kernel(const int* __restrict__ cu, int num_seqs, int rows, int t
               u32x4{0, 0, 0, 0});
     }
   }
-  if (descending >= 2) {
+  const bool remain = descending == 5;
+  if (descending >= 2 && !remain) {
     // Grouped by sequence: longest sequences first (bucketed by tile count), each
     // sequence's tiles contiguous; 2: last tile first (query-outer causal work grows
     // with the tile index), 3: first tile first (KV-outer causal work shrinks with it),
@@ -1020,7 +1031,7 @@ varlen_schedule_kernel(const int* __restrict__ cu, int num_seqs, int rows, int t
     int off, len;
     seg_bounds(cu, s, rows, off, len);
     const int nt = cdiv(len, tile);
-    for (int t = 0; t < nt; ++t) atomicAdd(&cnt[min(t, nbuckets - 1)], 1);
+    for (int t = 0; t < nt; ++t) atomicAdd(&cnt[min(remain ? nt - 1 - t : t, nbuckets - 1)], 1);
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -1039,7 +1050,7 @@ varlen_schedule_kernel(const int* __restrict__ cu, int num_seqs, int rows, int t
     seg_bounds(cu, s, rows, off, len);
     const int nt = cdiv(len, tile);
     for (int t = 0; t < nt; ++t) {
-      const int pos = atomicAdd(&cur[min(t, nbuckets - 1)], 1);
+      const int pos = atomicAdd(&cur[min(remain ? nt - 1 - t : t, nbuckets - 1)], 1);
       if (pos < capacity) work[pos] = make_int2(s, t);
     }
   }
@@ -1294,12 +1305,12 @@ hipError_t launch_fwd(const FwdParams& p, int d, int causal, dim3 grid, hipStrea
 }
 
 hipError_t launch_varlen_schedule(const int* cu, int num_seqs, int rows, int tile, int nbuckets, int descending,
-                                  int2* work, int capacity, hipStream_t st, const ZeroRows* zero) {
+                                  int2* work, int capacity, hipStream_t st, const ZeroRows* zero, int* first) {
   const size_t shmem = 2 * sizeof(int) * (size_t)nbuckets;
   ZeroRows z{};
   if (zero) z = *zero;
   hipLaunchKernelGGL(varlen_schedule_kernel, dim3(1), dim3(1024), shmem, st, cu, num_seqs, rows, tile,
-                     nbuckets, descending, work, capacity, z);
+                     nbuckets, descending, work, capacity, z, first);
   return hipGetLastError();
 }
 

@@ -55,9 +55,8 @@ struct FwdParams {
   int persist;
 };
 
-// Backward.  Same addressing as FwdParams, plus dO (do_*), the fp32 dQ
-// accumulator (dqa_*, same layout as Q but float), dK/dV outputs and the
-// per-row delta = rowsum(dO * O) (same layout as lse).
+// Backward.  Same addressing as FwdParams, plus dO (do_*), the dQ, dK and dV outputs and
+// the per-row delta = rowsum(dO * O) (same layout as lse).
 struct BwdParams {
   const half_t* q;
   const half_t* k;
@@ -66,7 +65,6 @@ struct BwdParams {
   const half_t* dout;
   const float* lse;
   float* delta;
-  float* dq_acc;
   half_t* dq;
   half_t* dk;
   half_t* dv;
@@ -76,7 +74,6 @@ struct BwdParams {
   int64_t o_sb, o_sh, o_ss;
   int64_t do_sb, do_sh, do_ss;
   int64_t l_sb, l_sh, l_ss;
-  int64_t dqa_sb, dqa_sh, dqa_ss;
   int64_t dq_sb, dq_sh, dq_ss;
   int64_t dk_sb, dk_sh, dk_ss;
   int64_t dv_sb, dv_sh, dv_ss;
@@ -92,7 +89,11 @@ struct BwdParams {
   int total_q;        // varlen: rows of the packed Q (row-wise kernels)
   int total_k;        // varlen: rows of the packed K/V
   int bf16;           // element type of every fp16/bf16 tensor: 0 fp16, 1 bf16
-  float* lsd;         // batched head_dim 128 and 256: per query tile, -L*log2(e)/c then -D (null: unused)
+  // pipelined dK/dV kernel (head_dim 128 and 256; null: not used): per (batch, query head,
+  // query tile), -L*log2(e)/c then -D of the tile's rows
+  float* lsd;
+  const int* lsd_seq; // varlen: first tile of each sequence, in tiles of the dQ kernel
+  int lsd_tiles;      // tiles per query head
   // pipelined dK/dV kernel on small grids: each key tile's items are cut into runs of at most
   // kv_run, one workgroup each, whose fp32 sums go to kv_part (slot (batch, KV head, key
   // tile, run), kv_runs slots per key tile) and are added by bwd_kv_reduce_kernel; 0: one
@@ -170,17 +171,16 @@ struct ZeroRows {
 constexpr int kVarlenSmallSeqs = FAL_VARLEN_SMALL_SEQS;
 constexpr int kVarlenSmallTokens = FAL_VARLEN_SMALL_TOKENS;
 hipError_t launch_varlen_schedule(const int* cu, int num_seqs, int rows, int tile, int nbuckets, int descending,
-                                  int2* work, int capacity, hipStream_t st, const ZeroRows* zero = nullptr);
+                                  int2* work, int capacity, hipStream_t st, const ZeroRows* zero = nullptr,
+                                  int* first = nullptr);
 
 int bwd_block_n(int d);
 hipError_t launch_bwd(const BwdParams& p, int d, int causal, dim3 grid, hipStream_t st);
-hipError_t launch_bwd_pre(const BwdParams& p, int d, int rows_batched, hipStream_t st);
-hipError_t launch_bwd_post(const BwdParams& p, int d, hipStream_t st);
-// head dims whose dQ comes from the query-outer kernel (no fp32 accumulator)
-bool bwd_split_dq(int d, bool batched);
 int bwd_dq_block_m(int d);
-// batched head_dim d uses bwd_kv_pipe_kernel (workspace holds the lsd array)
+// batched calls of head dim d run the pipelined kernels (the workspace holds the lsd array)
 bool bwd_pipe(int d);
+// a packed call of head dim d runs them (num_seqs sequences of total_k keys in all)
+bool bwd_varlen_pipe(int d, int64_t num_seqs, int64_t total_k, int64_t heads_kv, int ncu);
 int bwd_pipe_bm(int d);   // its query rows per item
 // Plan of BwdParams::kv_run / kv_runs for a batched call of head_dim d on `ncu` compute units
 // with `avail` bytes for the partial sums (0 / 0: no split); returns the bytes it uses.

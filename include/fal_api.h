@@ -130,6 +130,8 @@ int fal_bwd(const void* dout, const void* q, const void* k, const void* v, const
  * FlashAttnVarlenFunc.backward (flash_attn_legacy/flash_attn.py:133-157), which
  * calls the batched backward once per sequence with host syncs in between.
  *   Layouts as fal_fwd_varlen; lse [total_q, Hq] from fal_fwd_varlen.
+ * workspace: the row deltas D, the work lists and, where the pipelined kernels run, D and
+ * lse in tile order.  The size depends on the current device, as fal_bwd_workspace_best does.
  */
 size_t fal_bwd_varlen_workspace_size(int64_t num_seqs, int64_t total_q, int64_t total_k,
                                      int64_t heads_q, int64_t head_dim);

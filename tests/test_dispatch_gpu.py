@@ -116,3 +116,19 @@ def test_head_dim_256_backward(B, Hq, Hkv, Nq, Nk, sign, causal):
 ])
 def test_backward_runs(B, Hq, Hkv, Nq, Nk, d, causal):
     check_gradients(B, Hq, Hkv, Nq, Nk, d, causal)
+
+
+# Packed backward on the pipelined kernels: head_dim 256 always, head_dim 128 from 768 key
+# tiles (times KV heads) of sequences of 512 keys on average.  Sequences that end inside a
+# query item or key tile, of one row, without queries or keys, in an order that the work
+# lists change; GQA, where one head's rows of the row-value array are followed by the next's.
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("lens_q,lens_k,hq,hkv,d", [
+    ([1, 33, 300, 129], [1, 33, 300, 129], 4, 2, 256),
+    ([70, 0, 130, 515, 31], [140, 33, 0, 257, 128], 4, 1, 256),
+    ([515, 1201, 64, 700, 641], [515, 1201, 64, 700, 641], 32, 32, 128),
+    ([600, 0, 1100, 70], [1, 900, 2200, 3100], 32, 16, 128),
+])
+def test_packed_backward_pipelined(lens_q, lens_k, hq, hkv, d, causal):
+    from test_varlen_gpu import bwd_check
+    bwd_check(lens_q, lens_k, hq, hkv, d, causal)
