@@ -814,6 +814,41 @@ bwd_dq_kernel(BwdParams p) {
   const T* vbase = (const T*)p.v + (int64_t)b * p.v_sb + (int64_t)hkv * p.v_sh + (int64_t)k_off * p.v_ss;
   const int64_t lrow = (int64_t)b * p.l_sb + (int64_t)hq * p.l_sh + (int64_t)q_off * p.l_ss;
 
+  const int kend = CAUSAL ? min(nk, m0 + BM) : nk;
+  const int ntiles = cdiv(kend, BN);
+  const int nfull = CAUSAL ? min(nk / BN, (m0 + 1) / BN) : nk / BN;
+
+  const int ws = __builtin_amdgcn_readfirstlane(w);
+  int kvo[IPT], vvo[IPT];
+#pragma unroll
+  for (int i = 0; i < IPT; ++i) {
+    const int I = i * NW + ws;
+    const int pch = I * 64 + lane;
+    const int r = pch / CPR;
+    const int cc = TL::logical_chunk(r, pch % CPR);
+    kvo[i] = (int)(r * p.k_ss + cc * 8) * 2;   // from the tile's first row
+    vvo[i] = (int)(r * p.v_ss + cc * 8) * 2;
+  }
+  if (PIPE && ntiles > 0) {
+    // the pipelined loop's first two K/V tiles (rows past the end read as zeros): on their
+    // way while the rows of Q, dO and O arrive.  Head_dim 256 also keeps fewer values alive
+    // across the loop (no scratch left when causal, 48 bytes before): backward of 1 x 16 x
+    // 1024 causal 110.6 -> 105.1 us, packed 16 x up to 2048, 16/4 heads 640 -> 618;
+    // head_dim 128 level.
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int64_t rows = min(max((int64_t)nk - j * BN, (int64_t)0), (int64_t)BN);
+      const __amdgpu_buffer_rsrc_t krs = make_rsrc(kbase + (int64_t)j * BN * p.k_ss, (uint32_t)(rows * p.k_ss * 2));
+      const __amdgpu_buffer_rsrc_t vrs = make_rsrc(vbase + (int64_t)j * BN * p.v_ss, (uint32_t)(rows * p.v_ss * 2));
+      T* slot = smem + j * 2 * PART + ws * 512;
+#pragma unroll
+      for (int i = 0; i < IPT; ++i) {
+        buffer_to_lds16(krs, kvo[i], slot + i * NW * 512);
+        buffer_to_lds16(vrs, vvo[i], slot + PART + i * NW * 512);
+      }
+    }
+  }
+
   // Q and dO slices of this wave (B operands: n = query row, k = head dim), the row's
   // log-sum-exp (log2 domain) and D = rowsum(dO * O).  The two lanes of a row hold one
   // half of the head dim each.  D is also stored for the dK/dV kernel, which runs after
@@ -852,21 +887,6 @@ bwd_dq_kernel(BwdParams p) {
     }
   }
 
-  const int kend = CAUSAL ? min(nk, m0 + BM) : nk;
-  const int ntiles = cdiv(kend, BN);
-  const int nfull = CAUSAL ? min(nk / BN, (m0 + 1) / BN) : nk / BN;
-
-  const int ws = __builtin_amdgcn_readfirstlane(w);
-  int kvo[IPT], vvo[IPT];
-#pragma unroll
-  for (int i = 0; i < IPT; ++i) {
-    const int I = i * NW + ws;
-    const int pch = I * 64 + lane;
-    const int r = pch / CPR;
-    const int cc = TL::logical_chunk(r, pch % CPR);
-    kvo[i] = (int)(r * p.k_ss + cc * 8) * 2;   // from the tile's first row
-    vvo[i] = (int)(r * p.v_ss + cc * 8) * 2;
-  }
   int kaddr[KS];   // fragment (row l32, chunk 2t+hh) of 32-key block 0
 #pragma unroll
   for (int t = 0; t < KS; ++t) kaddr[t] = TL::offset(l32, 2 * t + hh);
@@ -900,8 +920,9 @@ bwd_dq_kernel(BwdParams p) {
     const int p_hh4 = hh * 4;
     const float p_nl = -lrow2, p_dl = drow;
     const float p_c = c, p_negc = c > 0.f ? -INFINITY : INFINITY;   // c * negc = -inf
-    const int64_t rows_left = max((int64_t)nk, (int64_t)0);
-    const uint64_t ka0 = (uint64_t)(uintptr_t)kbase, va0 = (uint64_t)(uintptr_t)vbase;
+    const int64_t rows_left = max((int64_t)nk - 2 * BN, (int64_t)0);   // from the third tile on
+    const uint64_t ka0 = (uint64_t)(uintptr_t)(kbase + (int64_t)2 * BN * p.k_ss);
+    const uint64_t va0 = (uint64_t)(uintptr_t)(vbase + (int64_t)2 * BN * p.v_ss);
     const uint32_t pk_rs[4] = {(uint32_t)ka0, (uint32_t)(ka0 >> 32) & 0xffffu,
                                (uint32_t)min(rows_left * p.k_ss * 2, (int64_t)0x7fffffff), 0x00020000u};
     const uint32_t pv_rs[4] = {(uint32_t)va0, (uint32_t)(va0 >> 32) & 0xffffu,

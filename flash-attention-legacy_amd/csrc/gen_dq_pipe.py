@@ -349,14 +349,12 @@ class Emitter:
             e(f"s_mov_b32 s{SV + i}, {op(f'vr{i}')}")
         e(f"s_mov_b32 s{SJ}, 0")
         e(f"s_mov_b32 s{SR}, {op('rows')}")
-        e(f"s_mov_b32 s{SD}, 0")
+        e(f"s_mov_b32 s{SD}, 2")   # (tiles 0 and 1 are copied by the caller)
         e(f"v_sub_f32 {v(DN)}, 0, {op('dl')}")
         for r in range(DN + 1, DN + 16):
             e(f"v_mov_b32 {v(r)}, {v(DN)}")
         for a in range(self.nacc):
             e(f"v_accvgpr_write_b32 a{a}, 0")
-        self.dma()
-        self.dma()
         e("s_waitcnt vmcnt(8)")
         e("s_barrier")
         # A of the first tile (if this wave has any tile)
