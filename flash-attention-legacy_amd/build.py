@@ -61,8 +61,8 @@ def _compile(src: str, verbose: bool, objdir: str = OBJ, flags=()) -> str:
     return obj
 
 
-GENERATORS = (("gen_fwd_pipe", "fal_fwd_pipe.inc"), ("gen_bwd_pipe", "fal_bwd_pipe.inc"),
-              ("gen_dq_pipe", "fal_dq_pipe.inc"))
+GENERATORS = (("gen_fwd_pipe", "fal_fwd_pipe.inc"), ("gen_fwd64_pipe", "fal_fwd64_pipe.inc"),
+              ("gen_bwd_pipe", "fal_bwd_pipe.inc"), ("gen_dq_pipe", "fal_dq_pipe.inc"))
 GEN_DIR = os.path.join(CSRC, "gen")     # the tracked generated asm loops
 
 
@@ -95,12 +95,12 @@ def check_generated(regen: bool = False) -> None:
 def _parse_knobs(knobs) -> dict:
     """['fwd.KDIST=3', 'bwd.ABL=nob'] -> {'gen_fwd_pipe': {'KDIST': '3'}, ...}"""
     out: dict = {}
-    short = {"fwd": "gen_fwd_pipe", "bwd": "gen_bwd_pipe", "dq": "gen_dq_pipe"}
+    short = {"fwd": "gen_fwd_pipe", "fwd64": "gen_fwd64_pipe", "bwd": "gen_bwd_pipe", "dq": "gen_dq_pipe"}
     for kv in knobs:
         key, _, val = kv.partition("=")
         gen, _, name = key.partition(".")
         if gen not in short or not name or not _:
-            raise ValueError(f"knob {kv!r}: expected fwd.NAME=VALUE, bwd.NAME=VALUE or dq.NAME=VALUE")
+            raise ValueError(f"knob {kv!r}: expected fwd.NAME=VALUE, fwd64.NAME=VALUE, bwd.NAME=VALUE or dq.NAME=VALUE")
         out.setdefault(short[gen], {})[name] = val
     return out
 
@@ -192,7 +192,7 @@ def main() -> int:
     ap.add_argument("--out", default=OUT, help="library path to write")
     ap.add_argument("-D", dest="defines", action="append", default=[], help="NAME=VALUE tunable macro")
     ap.add_argument("--knob", dest="knobs", action="append", default=[],
-                    help="generator knob: fwd.NAME=VALUE, bwd.NAME=VALUE or dq.NAME=VALUE")
+                    help="generator knob: fwd.NAME=VALUE, fwd64.NAME=VALUE, bwd.NAME=VALUE or dq.NAME=VALUE")
     ap.add_argument("--measure", action="store_true",
                     help="admit ablation knobs (timing-only builds whose results are wrong)")
     ap.add_argument("--regen", action="store_true",

@@ -193,6 +193,7 @@ static int fal_fwd_impl(const void* q, const void* k, const void* v, void* o, fl
   }
   if (is_causal && !p.kchunk && !p.persist && !p.gqa4)
     p.lpt = fwd_causal_order((int)head_dim, nblocks, batch * heads_q, ncu);
+  p.small = !p.kchunk && fwd_small_pipe((int)head_dim, nblocks, seqlen_q, seqlen_k, is_causal != 0, ncu);
   if (nblocks > 0x7fffffff) return fail(FAL_ERR_INVALID, "problem too large for one launch");
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e = launch_fwd(p, (int)head_dim, is_causal != 0, dim3((unsigned)nblocks), st);

@@ -26,6 +26,7 @@
 
 #include "fal_kernels.h"
 #include "fal_fwd_pipe.inc"
+#include "fal_fwd64_pipe.inc"
 
 namespace fal {
 
@@ -49,6 +50,15 @@ namespace fal {
 #ifndef FAL_FWD_PIPE
 #define FAL_FWD_PIPE 1   // head_dim 128 at two row blocks per wave: software-pipelined tile loop
 #endif
+// The configurations whose key-tile loop is a software-pipelined asm block: head_dim 128
+// with 64 query rows per wave (fal_fwd_pipe.inc); head_dim 64 with 32, where the launch asks
+// for it (SMALL, fal_fwd64_pipe.inc).
+template <int D, int NW, int BN, int RB, bool SMALL>
+struct FwdPipe {
+  static constexpr bool wide = FAL_FWD_PIPE && D == 128 && RB == 2 && NW == 4 && BN == 64 && !FAL_PRESCALE_FP16;
+  static constexpr bool narrow = SMALL && D == 64 && RB == 1 && NW == 4 && BN == 64 && !FAL_PRESCALE_FP16;
+  static constexpr bool any = wide || narrow;
+};
 
 // A workgroup's (batch or sequence, query head, query tile) and its row ranges.
 struct FwdItem {
@@ -170,17 +180,18 @@ __device__ __forceinline__ bool fwd_item(const FwdParams& p, FwdItem& it, int bm
   return true;
 }
 
-// Pipelined loop's O hand-off in LDS: 32 blocks of 1 KB per wave, 1040 bytes apart so the
-// row-wise reads of the epilogue spread over the banks.
+// Pipelined loops' O hand-off in LDS: RB * D/8 blocks of 1 KB per wave, 1040 bytes apart so
+// the row-wise reads of the epilogue spread over the banks.
 constexpr int kPipeOStr = 1040;
-constexpr int kPipeOWave = 32 * kPipeOStr;
+template <int D, int RB>
+constexpr int pipe_owave() { return RB * (D / 8) * kPipeOStr; }
 
 // One work item (query tile of one head, or of four heads under gqa4) of fwd_kernel.
 // Every wave of the workgroup takes the same early returns.
 // Persistent schedule (`next` valid when has_next): returns pre | (qpre << 2) for the next
 // item -- pre = 2 when this item issued the copies of its first two K/V tiles, qpre = 1
 // when it loaded its Q slices into qio (the Q registers, free once the tile loop is done).
-template <class T, int D, int NW, int BN, bool CAUSAL, int RB>
+template <class T, int D, int NW, int BN, bool CAUSAL, int RB, bool SMALL>
 __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T* smem, const FwdItem& next,
                                         bool has_next, vec8<T> (&qio)[RB][D / 16]) {
   using TL = SwizzledTile<D>;
@@ -190,10 +201,11 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
   // instead pre-multiplies an fp16 Q by scale*log2(e), rounded once to fp16: that saves
   // the FMA but shifts large scores by up to ~1e-2 in log2 units, so it is off.
   constexpr bool PRESCALE = FAL_PRESCALE_FP16 && std::is_same<T, half_t>::value;
-  // PIPE: the key-tile loop is the software-pipelined asm block (head_dim 128, 64 query
-  // rows per wave, one wave per SIMD) with a ring of 4 K/V tiles copied two tiles ahead.
-  constexpr bool PIPE = FAL_FWD_PIPE && D == 128 && RB == 2 && NW == 4 && BN == 64 && !FAL_PRESCALE_FP16;
+  // PIPE: the key-tile loop is a software-pipelined asm block with a ring of 4 K/V tiles
+  // copied two tiles ahead (WIDE: head_dim 128, 64 query rows per wave, one wave per SIMD).
+  constexpr bool PIPE = FwdPipe<D, NW, BN, RB, SMALL>::any, WIDE = FwdPipe<D, NW, BN, RB, SMALL>::wide;
   constexpr bool PIPE_SIGN = PIPE;
+  constexpr int kPipeOWave = pipe_owave<D, RB>();
   constexpr int BM = NW * 32 * RB;  // query rows per workgroup (RB 32-row blocks per wave)
   constexpr int KS = D / 16;        // MFMA k-steps over the head dim
   constexpr int NKB = BN / 32;      // 32-key blocks per tile
@@ -219,7 +231,7 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
   const int b = it.b, hq = it.hq, qt = it.qt, q_off = it.q_off, k_off = it.k_off, nq = it.nq, nk = it.nk;
   const int hkv = hq / (p.Hq / p.Hkv);
   // gqa4 (pipelined loop only): the waves share 64 query rows of different heads
-  const bool gqa4 = PIPE && p.gqa4;
+  const bool gqa4 = WIDE && p.gqa4;
   const int BMW = gqa4 ? 32 * RB : BM;      // query rows per workgroup and head
   const int m0 = qt * BMW;
   if (m0 >= nq) return 0;
@@ -269,12 +281,11 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
       const __amdgpu_buffer_rsrc_t vrs =
           make_rsrc(xvb + (int64_t)t * BN * p.v_ss, (uint32_t)min(rt * p.v_ss * 2, (int64_t)0x7fffffff));
       T* kdst = smem + t * 2 * PART;
+      // (K before V: the narrow loop's first wait counts on the order)
 #pragma unroll
-      for (int i = 0; i < IPT; ++i) {
-        const int I = i * NW + ws;
-        buffer_to_lds16(krs, kvo[i], kdst + I * 64 * 8);
-        buffer_to_lds16(vrs, vvo[i], kdst + PART + I * 64 * 8);
-      }
+      for (int i = 0; i < IPT; ++i) buffer_to_lds16(krs, kvo[i], kdst + (i * NW + ws) * 64 * 8);
+#pragma unroll
+      for (int i = 0; i < IPT; ++i) buffer_to_lds16(vrs, vvo[i], kdst + PART + (i * NW + ws) * 64 * 8);
     }
     return 2;
   };
@@ -519,8 +530,8 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
 
   const int wrow_hi = m0 + (w * RB + RB - 1) * 32 + 31;   // last query row of this wave
   if constexpr (PIPE) {
-    // The whole key-tile loop is one software-pipelined asm block (fal_fwd_pipe.inc,
-    // generated by gen_fwd_pipe.py): a 4-slot K/V ring copied two tiles ahead, PV of
+    // The whole key-tile loop is one software-pipelined asm block (generated by
+    // gen_fwd_pipe.py and gen_fwd64_pipe.py): a 4-slot K/V ring copied two tiles ahead, PV of
     // tile j-1 and S of tile j+1 interleaved with the softmax of tile j, masking of the
     // diagonal and last tiles, and the row-max fix-up.  It leaves m and l in registers
     // and this wave's O in LDS.
@@ -564,14 +575,22 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
     const int p_jl = __builtin_amdgcn_readfirstlane(jl);
     const int p_jbeg = jbeg, p_jend = jend, p_nk = nk;
     const int p_wrow = CAUSAL ? wrow0 : 0x3fffffff;
-    if constexpr (std::is_same<T, half_t>::value)
-      asm volatile(FAL_PIPE_ASM_F16 : FAL_PIPE_OUTS : FAL_PIPE_INS : FAL_PIPE_CLOBBERS);
-    else
-      asm volatile(FAL_PIPE_ASM_BF16 : FAL_PIPE_OUTS : FAL_PIPE_INS : FAL_PIPE_CLOBBERS);
+    // narrow loop: the tiles below this index need no mask for the wave, are not its last
+    // one, and the tiles they copy (up to three on) are whole
+    const int p_jf = __builtin_amdgcn_readfirstlane(
+        min(min(jl, CAUSAL ? min(nk / BN, (wrow0 + 1) / BN) : nk / BN), min(nk, jend * BN) / BN - 3));
+    (void)p_jf;
+    constexpr bool F16 = std::is_same<T, half_t>::value;
+#define FAL_PIPE_RUN(ASM, P) asm volatile(ASM : P##_OUTS : P##_INS : P##_CLOBBERS)
+    if constexpr (D == 128 && F16) FAL_PIPE_RUN(FAL_PIPE_ASM_F16, FAL_PIPE);
+    if constexpr (D == 128 && !F16) FAL_PIPE_RUN(FAL_PIPE_ASM_BF16, FAL_PIPE);
+    if constexpr (D == 64 && F16) FAL_PIPE_RUN(FAL_PIPE64_ASM_F16, FAL_PIPE64);
+    if constexpr (D == 64 && !F16) FAL_PIPE_RUN(FAL_PIPE64_ASM_BF16, FAL_PIPE64);
+#undef FAL_PIPE_RUN
     // persistent schedule: the next item's Q slices load while this item's O goes out
     // (buffer loads: rows past the sequence read as zeros; a negative scale, folded into
     // Q, keeps the loads at the item's start)
-    if (p.persist && has_next && !negq && next.qt * BMW < next.nq) {
+    if (WIDE && p.persist && has_next && !negq && next.qt * BMW < next.nq) {
       // one resource over the item's rows (offsets from its first row stay small)
       const int nm0 = next.qt * BMW;
       const T* nqb = (const T*)p.q + (int64_t)next.b * p.q_sb + (int64_t)next.hq * p.q_sh +
@@ -606,8 +625,8 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
             for (int e = 0; e < 4; ++e) oacc[rb][db][g4 * 4 + e] = x[e];
           }
     } else {
-      // O and L straight from LDS: each store instruction writes 4 whole rows (16 lanes
-      // x 16 bytes per row), where stores from the accumulator layout would write 16
+      // O and L straight from LDS: each store instruction writes whole rows (D/8 lanes x
+      // 16 bytes per row), where stores from the accumulator layout would write 16
       // bytes into each of 32 rows
       float inv[RB];
 #pragma unroll
@@ -617,7 +636,9 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
         if (hh == 0 && row[rb] < nq)
           lbase[(int64_t)row[rb] * p.l_ss] = l_tot > 0.f ? (m_run[rb] + fast_log2(l_tot)) * kLn2 : -INFINITY;
       }
-      const int cch = lane & 15;               // 16-byte chunk of the row
+      constexpr int RPI = 64 / CPR;            // rows per store instruction
+      constexpr int JJ = 16 / RPI;             // store instructions per 16 rows
+      const int cch = lane % CPR;              // 16-byte chunk of the row
       const int wr0 = m0 + (gqa4 ? 0 : ws) * RB * 32;   // (ws: the wave index as a scalar)
       // one buffer resource over this wave's rows inside the sequence: stores past its
       // end are dropped, so a store needs no branch and no 64-bit address (at most 64
@@ -625,37 +646,37 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
       const __amdgpu_buffer_rsrc_t ors =
           make_rsrc(obase + (int64_t)wr0 * p.o_ss,
                     (uint32_t)min((int64_t)max(min(nq - wr0, RB * 32), 0) * p.o_ss * 2, (int64_t)0x7fffffff));
-      const int ovo = ((lane >> 4) * (int)p.o_ss + cch * 8) * 2;
+      const int ovo = ((lane / CPR) * (int)p.o_ss + cch * 8) * 2;
       // per 16 rows: all LDS reads and row factors first, then the stores (one wait, not
       // one per row)
 #pragma unroll
       for (int hb = 0; hb < 2 * RB; ++hb) {
         const int rb = hb >> 1;
-        f32x4 a0[4], a1[4];
-        float iv[4];
+        f32x4 a0[JJ], a1[JJ];
+        float iv[JJ];
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int l32w = (hb & 1) * 16 + jj * 4 + (lane >> 4);
-          const int g = rb * 16 + cch;
+        for (int jj = 0; jj < JJ; ++jj) {
+          const int l32w = (hb & 1) * 16 + jj * RPI + lane / CPR;
+          const int g = rb * CPR + cch;
           a0[jj] = *reinterpret_cast<const f32x4*>(wbase + l32w * 16 + g * kPipeOStr);
           a1[jj] = *reinterpret_cast<const f32x4*>(wbase + (32 + l32w) * 16 + g * kPipeOStr);
           iv[jj] = __shfl(inv[rb], l32w);
         }
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int r = hb * 16 + jj * 4 + (lane >> 4);   // row of the wave, 0..63
+        for (int jj = 0; jj < JJ; ++jj) {
+          const int r = hb * 16 + jj * RPI;               // first of the instruction's rows, 0..63
           V8 h;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             h[e] = (T)(a0[jj][e] * iv[jj]);
             h[4 + e] = (T)(a1[jj][e] * iv[jj]);
           }
-          buffer_store16(ors, ovo + (r - (lane >> 4)) * (int)p.o_ss * 2, __builtin_bit_cast(u32x4, h));
+          buffer_store16(ors, ovo + r * (int)p.o_ss * 2, __builtin_bit_cast(u32x4, h));
         }
       }
       stored = true;
     }
-    if (p.persist) __syncthreads();   // every wave has its O out of LDS (the next item reuses it)
+    if (WIDE && p.persist) __syncthreads();   // every wave has its O out of LDS (the next item reuses it)
   } else {
   if (jbeg < jend) load_tile(jbeg, 0);
   // Tiles that need no mask for any row of the workgroup: straight-line, unrolled by
@@ -765,7 +786,7 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
   }
   // Persistent schedule: the next item's first two K/V tiles are copied after this item's
   // O stores, so their latency overlaps those stores and the next item's Q loads.
-  if (PIPE && p.persist && has_next) pre_next = issue_first2(next);
+  if (WIDE && p.persist && has_next) pre_next = issue_first2(next);
   return pre_next | (qpre_next << 2);
 }
 
@@ -844,18 +865,19 @@ __device__ __forceinline__ bool fwd_item_vpair(const FwdParams& p, FwdItem& it, 
 // VPAIR: packed sequences, each workgroup walking the two items of one pair of the
 // work list (fwd_item_vpair); a separate instantiation, so the batched kernel keeps
 // its own register allocation.
-template <class T, int D, int NW, int BN, bool CAUSAL, int RB, bool VPAIR = false>
+template <class T, int D, int NW, int BN, bool CAUSAL, int RB, bool VPAIR = false, bool SMALL = false>
 __global__ void __launch_bounds__(NW * 64)
 __attribute__((amdgpu_waves_per_eu((RB == 2 && D >= 128) ? 1 : (D <= 128 ? FAL_FWD_WPE : 1), 8)))
 fwd_kernel(FwdParams p) {
-  constexpr bool PIPE = FAL_FWD_PIPE && D == 128 && RB == 2 && NW == 4 && BN == 64 && !FAL_PRESCALE_FP16;
+  constexpr bool PIPE = FwdPipe<D, NW, BN, RB, SMALL>::any, WIDE = FwdPipe<D, NW, BN, RB, SMALL>::wide;
   constexpr int PART = BN * SwizzledTile<D>::CPR * 8;
   constexpr int NSLOT = PIPE ? 4 : 2;
-  // the pipelined loop's O hand-off (4 x kPipeOWave bytes) reaches past the 128 KB ring
-  constexpr int NSMEM = PIPE ? (4 * kPipeOWave) / 2 : NSLOT * 2 * PART;
+  // (the O hand-off of the pipelined head_dim-128 and -32 loops reaches past the ring)
+  constexpr int NOUT = PIPE ? NW * pipe_owave<D, RB>() / 2 : 0;
+  constexpr int NSMEM = NSLOT * 2 * PART > NOUT ? NSLOT * 2 * PART : NOUT;
   __shared__ __attribute__((aligned(1024))) T smem[NSMEM];
   FwdItem it;
-  if (PIPE && p.persist) {
+  if (WIDE && p.persist) {
     // items past the tile count (qt >= n_qtiles) are skipped inside fwd_body; each item
     // ends with a barrier after its O left LDS and may issue the next item's first copies
     FwdItem nx;
@@ -869,7 +891,7 @@ fwd_kernel(FwdParams p) {
     bool have = item(it, 0);
     for (int i = 0; have; ++i) {
       const bool more = item(nx, i + 1);
-      const int r = fwd_body<T, D, NW, BN, CAUSAL, RB>(p, it, smem, nx, more, qio);
+      const int r = fwd_body<T, D, NW, BN, CAUSAL, RB, SMALL>(p, it, smem, nx, more, qio);
       nx.pre = r & 3;
       nx.qpre = r >> 2;
       it = nx;
@@ -880,7 +902,7 @@ fwd_kernel(FwdParams p) {
   // ---- resolve this workgroup's (batch/sequence, head, query tile) ----
   if (!fwd_item<CAUSAL>(p, it, p.gqa4 ? 64 : NW * 32 * RB)) return;
   vec8<T> qio[RB][D / 16];
-  fwd_body<T, D, NW, BN, CAUSAL, RB>(p, it, smem, it, false, qio);
+  fwd_body<T, D, NW, BN, CAUSAL, RB, SMALL>(p, it, smem, it, false, qio);
 }
 
 // ---------------------------------------------------------------------------
@@ -1102,6 +1124,15 @@ static hipError_t launch_fwd_t(const FwdParams& p, int causal, dim3 grid, hipStr
       return hipGetLastError();
     }
   }
+  if constexpr (!VARLEN && D == 64) {
+    if (p.small) {
+      if (causal)
+        hipLaunchKernelGGL((fwd_kernel<T, D, 4, 64, true, 1, false, true>), grid, dim3(256), 0, st, p);
+      else
+        hipLaunchKernelGGL((fwd_kernel<T, D, 4, 64, false, 1, false, true>), grid, dim3(256), 0, st, p);
+      return hipGetLastError();
+    }
+  }
   if (causal)
     hipLaunchKernelGGL((fwd_kernel<T, D, NW, BN, true, RB>), grid, dim3(NW * 64), 0, st, p);
   else
@@ -1176,6 +1207,20 @@ size_t fwd_split_plan(int64_t B, int64_t Hq, int64_t Nq, int64_t Nk, int d, int 
   }
   if (!*kchunk) return 0;
   return (size_t)(B * Hq * *nsplit * Nq) * (size_t)(d + 2) * sizeof(float) + 256;
+}
+
+// Head dim 64's pipelined loop overlaps the products and the softmax inside a wave, where the
+// C++ loop leaves that to the waves of a SIMD: a 64-key tile takes a lone wave 840 cycles
+// instead of 1150.  That pays while a grid of at most two workgroups per CU (what their
+// registers allow) ends with its longest chain of tiles, and from 16 tiles on; a shorter one
+// is lost in the loop's start and end, and a larger grid runs at the board's power limit,
+// where fewer cycles come back as a lower clock.  us, C++ loop -> this: 2 x 8 heads x 1024
+// causal 16.5 -> 14.9, non-causal 16.0 -> 14.8, 4 x 12 x 1000 causal 18.4 -> 17.3, 2 x 16 x
+// 2048 causal 32.1 -> 30.1; but 8 x 12 x 512 non-causal 14.4 -> 15.7, 1 x 8 x 128 6.1 -> 6.6,
+// and 4 x 16 x 2048 non-causal 87.4 -> 87.2.
+bool fwd_small_pipe(int d, int64_t nblocks, int64_t Nq, int64_t Nk, int causal, int ncu) {
+  const int64_t keys = causal ? std::min(Nq, Nk) : Nk;
+  return d == 64 && !FAL_PRESCALE_FP16 && nblocks <= 2 * (int64_t)ncu && keys > 15 * 64;
 }
 
 // Order of a causal grid.  Head by head puts query tile t of every head on the same CU

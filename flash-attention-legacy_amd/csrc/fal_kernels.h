@@ -51,6 +51,7 @@ struct FwdParams {
   // Causal batched grid of one query tile per workgroup: 0 = head by head; otherwise longest
   // tiles first over all heads, reversed from this rank on (fwd_item; fwd_causal_order).
   int lpt;
+  int small;   // head_dim 64: the pipelined loop of fal_fwd64_pipe.inc (fwd_small_pipe)
   // pipelined kernel: persistent grid (one workgroup per CU walking pairs of query tiles)
   int persist;
 };
@@ -144,6 +145,9 @@ int fwd_block_n(int d);
 // returns the workspace bytes the split needs (0 without a split).
 // True when the pipelined kernel is the faster of head_dim 128's two for this batched call.
 bool fwd_wide_pays(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int causal, int ncu);
+// FwdParams::small of a batched grid of `nblocks` workgroups (no split) on a GPU of `ncu`
+// compute units
+bool fwd_small_pipe(int d, int64_t nblocks, int64_t Nq, int64_t Nk, int causal, int ncu);
 // FwdParams::lpt of a causal grid of `nblocks` workgroups over `units` heads (batch x query
 // head) on a GPU of `ncu` compute units.
 int fwd_causal_order(int d, int64_t nblocks, int64_t units, int ncu);
