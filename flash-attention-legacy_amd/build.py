@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import argparse
 import concurrent.futures as cf
+import json
 import os
 import shutil
 import subprocess
@@ -150,17 +151,34 @@ def build(jobs: int | None = None, verbose: bool = False, out: str = OUT, define
     return out
 
 
+_TORCH_QUERY = """
+import json, os, sysconfig, torch
+from torch.utils import cpp_extension as ext
+print(json.dumps([[*ext.include_paths("cuda"), sysconfig.get_paths()["include"]],
+                  os.path.join(os.path.dirname(torch.__file__), "lib"), int(torch._C._GLIBCXX_USE_CXX11_ABI)]))
+"""
+
+
+def _torch_paths():
+    """(include folders, library folder, C++ ABI flag) of the installed torch.  Asked of another
+    interpreter, the second time without PYTHONPATH, by way of which pip's isolated builds
+    hide the installed packages."""
+    errors = ""
+    for flags in ([], ["-E"]):
+        r = subprocess.run([sys.executable, *flags, "-c", _TORCH_QUERY], capture_output=True, text=True)
+        if r.returncode == 0:
+            return json.loads(r.stdout.strip().splitlines()[-1])
+        errors = r.stderr
+    raise RuntimeError(f"torch is needed to build the Python binding:\n{errors}")
+
+
 def build_binding(verbose: bool = False) -> str:
     """Compile csrc/fal_torch.cpp with the host compiler; returns the module's path."""
-    import sysconfig
-    import torch
-    from torch.utils import cpp_extension as ext
-    inc = [*ext.include_paths("cuda"), sysconfig.get_paths()["include"]]
-    libdir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    inc, libdir, abi = _torch_paths()
     tmp = BINDING + ".tmp"
     cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
            *[a for p in inc for a in ("-isystem", p)], os.path.join(CSRC, "fal_torch.cpp"), "-o", tmp,
            f"-L{libdir}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
     if verbose:
