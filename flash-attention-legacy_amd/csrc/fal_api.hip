@@ -41,9 +41,11 @@ bool head_dim_ok(int64_t d) { return d == 32 || d == 64 || d == 96 || d == 128 |
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// A strided operand: 16-byte aligned base and every used stride a multiple of 8
-// elements, so each 8-element row chunk is one aligned 16-byte access.
-int check_operand(const char* name, const void* p, const int64_t* st, bool use_batch) {
+// A strided operand of `rows` rows: 16-byte aligned base and every used stride a multiple of
+// 8 elements, so each 8-element row chunk is one aligned 16-byte access, and rows at least
+// `apart` elements apart: most kernels bound a tile by rows * stride bytes, so the end of a
+// row longer than its stride would read as zeros, or not be stored.
+int check_operand(const char* name, const void* p, const int64_t* st, bool use_batch, int64_t rows, int64_t apart) {
   if (!p) return fail(FAL_ERR_INVALID, "%s: null pointer", name);
   if (!st) return fail(FAL_ERR_INVALID, "%s: null strides", name);
   if (!aligned16(p)) return fail(FAL_ERR_INVALID, "%s: base pointer must be 16-byte aligned", name);
@@ -55,8 +57,14 @@ int check_operand(const char* name, const void* p, const int64_t* st, bool use_b
   if (st[2] >= (int64_t(1) << 22))
     return fail(FAL_ERR_UNSUPPORTED, "%s: sequence stride %lld elements is too large (limit 4194304)", name,
                 (long long)st[2]);
+  if (rows > 1 && st[2] < apart)
+    return fail(FAL_ERR_UNSUPPORTED, "%s: sequence stride %lld is shorter than a row of %lld elements", name,
+                (long long)st[2], (long long)apart);
   return FAL_OK;
 }
+
+// The sequence stride of `rows` rows of `d` elements (a single row's may be anything).
+int64_t row_stride(const int64_t* st, int64_t rows, int64_t d) { return rows > 1 ? st[2] : std::max(st[2], d); }
 
 int launch_status(hipError_t e, const char* what) {
   if (e != hipSuccess) return fail(FAL_ERR_LAUNCH, "%s: %s", what, hipGetErrorString(e));
@@ -138,8 +146,10 @@ static int fal_fwd_impl(const void* q, const void* k, const void* v, void* o, fl
     return fail(FAL_ERR_INVALID, "num_heads_q (%lld) must be divisible by num_heads_kv (%lld)",
                 (long long)heads_q, (long long)heads_kv);
   int rc;
-  if ((rc = check_operand("q", q, q_strides, true)) || (rc = check_operand("k", k, k_strides, true)) ||
-      (rc = check_operand("v", v, v_strides, true)) || (rc = check_operand("o", o, o_strides, true)))
+  if ((rc = check_operand("q", q, q_strides, true, seqlen_q, head_dim)) ||
+      (rc = check_operand("k", k, k_strides, true, seqlen_k, head_dim)) ||
+      (rc = check_operand("v", v, v_strides, true, seqlen_k, head_dim)) ||
+      (rc = check_operand("o", o, o_strides, true, seqlen_q, head_dim)))
     return rc;
   if (!lse) return fail(FAL_ERR_INVALID, "lse: null pointer");
   if (batch == 0 || seqlen_q == 0) return ok();
@@ -151,10 +161,10 @@ static int fal_fwd_impl(const void* q, const void* k, const void* v, void* o, fl
   p.v = static_cast<const half_t*>(v);
   p.o = static_cast<half_t*>(o);
   p.lse = lse;
-  p.q_sb = q_strides[0]; p.q_sh = q_strides[1]; p.q_ss = q_strides[2];
-  p.k_sb = k_strides[0]; p.k_sh = k_strides[1]; p.k_ss = k_strides[2];
-  p.v_sb = v_strides[0]; p.v_sh = v_strides[1]; p.v_ss = v_strides[2];
-  p.o_sb = o_strides[0]; p.o_sh = o_strides[1]; p.o_ss = o_strides[2];
+  p.q_sb = q_strides[0]; p.q_sh = q_strides[1]; p.q_ss = row_stride(q_strides, seqlen_q, head_dim);
+  p.k_sb = k_strides[0]; p.k_sh = k_strides[1]; p.k_ss = row_stride(k_strides, seqlen_k, head_dim);
+  p.v_sb = v_strides[0]; p.v_sh = v_strides[1]; p.v_ss = row_stride(v_strides, seqlen_k, head_dim);
+  p.o_sb = o_strides[0]; p.o_sh = o_strides[1]; p.o_ss = row_stride(o_strides, seqlen_q, head_dim);
   p.l_sb = heads_q * seqlen_q; p.l_sh = seqlen_q; p.l_ss = 1;
   p.B = (int)batch; p.Hq = (int)heads_q; p.Hkv = (int)heads_kv;
   p.Nq = (int)seqlen_q; p.Nk = (int)seqlen_k;
@@ -261,8 +271,10 @@ static int fal_fwd_varlen_impl(const void* q, const void* k, const void* v, void
                 (long long)heads_kv);
   if (!cu_seqlens_q || !cu_seqlens_k) return fail(FAL_ERR_INVALID, "cu_seqlens: null pointer");
   int rc;
-  if ((rc = check_operand("q", q, q_strides, false)) || (rc = check_operand("k", k, k_strides, false)) ||
-      (rc = check_operand("v", v, v_strides, false)) || (rc = check_operand("o", o, o_strides, false)))
+  if ((rc = check_operand("q", q, q_strides, false, total_q, head_dim)) ||
+      (rc = check_operand("k", k, k_strides, false, total_k, head_dim)) ||
+      (rc = check_operand("v", v, v_strides, false, total_k, head_dim)) ||
+      (rc = check_operand("o", o, o_strides, false, total_q, head_dim)))
     return rc;
   if (!lse) return fail(FAL_ERR_INVALID, "lse: null pointer");
   const size_t need = fal_fwd_varlen_workspace_size(num_seqs, total_q, max_seqlen_q, head_dim);
@@ -299,10 +311,10 @@ static int fal_fwd_varlen_impl(const void* q, const void* k, const void* v, void
   p.v = static_cast<const half_t*>(v);
   p.o = static_cast<half_t*>(o);
   p.lse = lse;
-  p.q_sh = q_strides[1]; p.q_ss = q_strides[2];
-  p.k_sh = k_strides[1]; p.k_ss = k_strides[2];
-  p.v_sh = v_strides[1]; p.v_ss = v_strides[2];
-  p.o_sh = o_strides[1]; p.o_ss = o_strides[2];
+  p.q_sh = q_strides[1]; p.q_ss = row_stride(q_strides, total_q, head_dim);
+  p.k_sh = k_strides[1]; p.k_ss = row_stride(k_strides, total_k, head_dim);
+  p.v_sh = v_strides[1]; p.v_ss = row_stride(v_strides, total_k, head_dim);
+  p.o_sh = o_strides[1]; p.o_ss = row_stride(o_strides, total_q, head_dim);
   p.l_sb = 0; p.l_sh = 1; p.l_ss = heads_q;
   p.B = 1; p.Hq = (int)heads_q; p.Hkv = (int)heads_kv;
   p.scale_log2 = signed_scale_log2(softmax_scale);
@@ -386,12 +398,17 @@ static int fill_bwd_common(BwdParams& p, const void* dout, const void* q, const 
                            const void* o, const float* lse, void* dq, void* dk, void* dv,
                            const int64_t* do_s, const int64_t* q_s, const int64_t* k_s, const int64_t* v_s,
                            const int64_t* o_s, const int64_t* dq_s, const int64_t* dk_s, const int64_t* dv_s,
-                           bool batched) {
+                           bool batched, int64_t rows_q, int64_t rows_k, int64_t d) {
   int rc;
-  if ((rc = check_operand("dout", dout, do_s, batched)) || (rc = check_operand("q", q, q_s, batched)) ||
-      (rc = check_operand("k", k, k_s, batched)) || (rc = check_operand("v", v, v_s, batched)) ||
-      (rc = check_operand("o", o, o_s, batched)) || (rc = check_operand("dq", dq, dq_s, batched)) ||
-      (rc = check_operand("dk", dk, dk_s, batched)) || (rc = check_operand("dv", dv, dv_s, batched)))
+  const int64_t in = d == 256 ? 0 : d;   // (head_dim 256's kernels bound a tile by its last row)
+  if ((rc = check_operand("dout", dout, do_s, batched, rows_q, in)) ||
+      (rc = check_operand("q", q, q_s, batched, rows_q, in)) ||
+      (rc = check_operand("k", k, k_s, batched, rows_k, in)) ||
+      (rc = check_operand("v", v, v_s, batched, rows_k, in)) ||
+      (rc = check_operand("o", o, o_s, batched, rows_q, in)) ||
+      (rc = check_operand("dq", dq, dq_s, batched, rows_q, d)) ||
+      (rc = check_operand("dk", dk, dk_s, batched, rows_k, d)) ||
+      (rc = check_operand("dv", dv, dv_s, batched, rows_k, d)))
     return rc;
   if (!lse) return fail(FAL_ERR_INVALID, "lse: null pointer");
   p.dout = static_cast<const half_t*>(dout);
@@ -403,14 +420,14 @@ static int fill_bwd_common(BwdParams& p, const void* dout, const void* q, const 
   p.dq = static_cast<half_t*>(dq);
   p.dk = static_cast<half_t*>(dk);
   p.dv = static_cast<half_t*>(dv);
-  p.do_sb = batched ? do_s[0] : 0; p.do_sh = do_s[1]; p.do_ss = do_s[2];
-  p.q_sb = batched ? q_s[0] : 0; p.q_sh = q_s[1]; p.q_ss = q_s[2];
-  p.k_sb = batched ? k_s[0] : 0; p.k_sh = k_s[1]; p.k_ss = k_s[2];
-  p.v_sb = batched ? v_s[0] : 0; p.v_sh = v_s[1]; p.v_ss = v_s[2];
-  p.o_sb = batched ? o_s[0] : 0; p.o_sh = o_s[1]; p.o_ss = o_s[2];
-  p.dq_sb = batched ? dq_s[0] : 0; p.dq_sh = dq_s[1]; p.dq_ss = dq_s[2];
-  p.dk_sb = batched ? dk_s[0] : 0; p.dk_sh = dk_s[1]; p.dk_ss = dk_s[2];
-  p.dv_sb = batched ? dv_s[0] : 0; p.dv_sh = dv_s[1]; p.dv_ss = dv_s[2];
+  p.do_sb = batched ? do_s[0] : 0; p.do_sh = do_s[1]; p.do_ss = row_stride(do_s, rows_q, d);
+  p.q_sb = batched ? q_s[0] : 0; p.q_sh = q_s[1]; p.q_ss = row_stride(q_s, rows_q, d);
+  p.k_sb = batched ? k_s[0] : 0; p.k_sh = k_s[1]; p.k_ss = row_stride(k_s, rows_k, d);
+  p.v_sb = batched ? v_s[0] : 0; p.v_sh = v_s[1]; p.v_ss = row_stride(v_s, rows_k, d);
+  p.o_sb = batched ? o_s[0] : 0; p.o_sh = o_s[1]; p.o_ss = row_stride(o_s, rows_q, d);
+  p.dq_sb = batched ? dq_s[0] : 0; p.dq_sh = dq_s[1]; p.dq_ss = row_stride(dq_s, rows_q, d);
+  p.dk_sb = batched ? dk_s[0] : 0; p.dk_sh = dk_s[1]; p.dk_ss = row_stride(dk_s, rows_k, d);
+  p.dv_sb = batched ? dv_s[0] : 0; p.dv_sh = dv_s[1]; p.dv_ss = row_stride(dv_s, rows_k, d);
   return FAL_OK;
 }
 
@@ -439,7 +456,7 @@ static int fal_bwd_impl(const void* dout, const void* q, const void* k, const vo
   BwdParams p{};
   p.bf16 = bf16;
   int rc = fill_bwd_common(p, dout, q, k, v, o, lse, dq, dk, dv, do_strides, q_strides, k_strides, v_strides,
-                           o_strides, dq_strides, dk_strides, dv_strides, true);
+                           o_strides, dq_strides, dk_strides, dv_strides, true, seqlen_q, seqlen_k, head_dim);
   if (rc) return rc;
   const size_t need = bwd_need(batch, heads_q, seqlen_q, head_dim);
   if (!workspace || workspace_bytes < need)
@@ -540,7 +557,7 @@ static int fal_bwd_varlen_impl(const void* dout, const void* q, const void* k, c
   BwdParams p{};
   p.bf16 = bf16;
   int rc = fill_bwd_common(p, dout, q, k, v, o, lse, dq, dk, dv, do_strides, q_strides, k_strides, v_strides,
-                           o_strides, dq_strides, dk_strides, dv_strides, false);
+                           o_strides, dq_strides, dk_strides, dv_strides, false, total_q, total_k, head_dim);
   if (rc) return rc;
   const int d = (int)head_dim;
   bool pipe = bwd_varlen_pipe(d, num_seqs, total_k, heads_kv, device_cu_count());
@@ -664,8 +681,10 @@ static int fal_decode_impl(const void* q, const void* k_cache, const void* v_cac
                 (long long)(heads_q / heads_kv));
   if (!cache_seqlens) return fail(FAL_ERR_INVALID, "cache_seqlens: null pointer");
   int rc;
-  if ((rc = check_operand("q", q, q_strides, true)) || (rc = check_operand("k_cache", k_cache, k_strides, true)) ||
-      (rc = check_operand("v_cache", v_cache, v_strides, true)) || (rc = check_operand("o", o, o_strides, true)))
+  if ((rc = check_operand("q", q, q_strides, true, 1, 0)) ||
+      (rc = check_operand("k_cache", k_cache, k_strides, true, max_seqlen_k, head_dim)) ||
+      (rc = check_operand("v_cache", v_cache, v_strides, true, max_seqlen_k, head_dim)) ||
+      (rc = check_operand("o", o, o_strides, true, 1, 0)))
     return rc;
   const size_t need = fal_decode_workspace_size(batch, heads_q, heads_kv, max_seqlen_k, head_dim);
   if (!workspace || workspace_bytes < need)
@@ -682,8 +701,8 @@ static int fal_decode_impl(const void* q, const void* k_cache, const void* v_cac
   p.o = static_cast<half_t*>(o);
   p.lse = lse;
   p.q_sb = q_strides[0]; p.q_sh = q_strides[1];
-  p.k_sb = k_strides[0]; p.k_sh = k_strides[1]; p.k_ss = k_strides[2];
-  p.v_sb = v_strides[0]; p.v_sh = v_strides[1]; p.v_ss = v_strides[2];
+  p.k_sb = k_strides[0]; p.k_sh = k_strides[1]; p.k_ss = row_stride(k_strides, max_seqlen_k, head_dim);
+  p.v_sb = v_strides[0]; p.v_sh = v_strides[1]; p.v_ss = row_stride(v_strides, max_seqlen_k, head_dim);
   p.o_sb = o_strides[0]; p.o_sh = o_strides[1];
   p.B = (int)batch; p.Hq = (int)heads_q; p.Hkv = (int)heads_kv;
   p.max_seqlen = (int)max_seqlen_k;

@@ -548,6 +548,9 @@ bwd_kv_pipe_kernel(BwdParams p) {
   const float p_negc = p.scale_log2 > 0.f ? -INFINITY : INFINITY;   // c * negc = -inf
   const float p_scale = p.scale;
   const uint32_t p_qrb = (uint32_t)(p.q_ss * 2), p_drb = (uint32_t)(p.do_ss * 2);
+  // (head_dim 256) how far a tile's last row reaches past rows * stride
+  const int p_qx = 2 * D - (int)p_qrb, p_dx = 2 * D - (int)p_drb;
+  (void)p_qx, (void)p_dx;
   const int p_nq = nq, p_nqt = nqt;
   const int64_t qstep = (int64_t)kPipeBM * p.q_ss * 2, dstep = (int64_t)kPipeBM * p.do_ss * 2;
   // head_dim 256: an item's copies leave the resources 16 rows on
@@ -563,10 +566,10 @@ bwd_kv_pipe_kernel(BwdParams p) {
     const int64_t rows = min(max((int64_t)nk - n0, (int64_t)0), (int64_t)kPipeBN);
     const __amdgpu_buffer_rsrc_t krs =
         make_rsrc((const T*)p.k + (int64_t)b * p.k_sb + (int64_t)hkv * p.k_sh + (int64_t)(k_off + n0) * p.k_ss,
-                  (uint32_t)(rows * p.k_ss * 2));
+                  rows_bytes<D>(rows, p.k_ss));
     const __amdgpu_buffer_rsrc_t vrs =
         make_rsrc((const T*)p.v + (int64_t)b * p.v_sb + (int64_t)hkv * p.v_sh + (int64_t)(k_off + n0) * p.v_ss,
-                  (uint32_t)(rows * p.v_ss * 2));
+                  rows_bytes<D>(rows, p.v_ss));
     const int r = ws * 32 + l32;
     const int ko = (int)(r * p.k_ss * 2) + hh * 16, vo = (int)(r * p.v_ss * 2) + hh * 16;
 #pragma unroll
@@ -838,8 +841,8 @@ bwd_dq_kernel(BwdParams p) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int64_t rows = min(max((int64_t)nk - j * BN, (int64_t)0), (int64_t)BN);
-      const __amdgpu_buffer_rsrc_t krs = make_rsrc(kbase + (int64_t)j * BN * p.k_ss, (uint32_t)(rows * p.k_ss * 2));
-      const __amdgpu_buffer_rsrc_t vrs = make_rsrc(vbase + (int64_t)j * BN * p.v_ss, (uint32_t)(rows * p.v_ss * 2));
+      const __amdgpu_buffer_rsrc_t krs = make_rsrc(kbase + (int64_t)j * BN * p.k_ss, rows_bytes<D>(rows, p.k_ss));
+      const __amdgpu_buffer_rsrc_t vrs = make_rsrc(vbase + (int64_t)j * BN * p.v_ss, rows_bytes<D>(rows, p.v_ss));
       T* slot = smem + j * 2 * PART + ws * 512;
 #pragma unroll
       for (int i = 0; i < IPT; ++i) {
@@ -929,6 +932,9 @@ bwd_dq_kernel(BwdParams p) {
                                (uint32_t)min(rows_left * p.v_ss * 2, (int64_t)0x7fffffff), 0x00020000u};
     const uint32_t p_ktb = (uint32_t)(BN * p.k_ss * 2), p_vtb = (uint32_t)(BN * p.v_ss * 2);
     const uint32_t p_krb = (uint32_t)(p.k_ss * 2), p_vrb = (uint32_t)(p.v_ss * 2);
+    // (head_dim 256) how far a tile's last row reaches past rows * stride
+    const int p_kx = 2 * D - (int)p_krb, p_vx = 2 * D - (int)p_vrb;
+    (void)p_kx, (void)p_vx;
     const int p_rows = (int)min(rows_left, (int64_t)0x7fffffff);
     // tiles of this wave: [0, jl]; causal waves stop at their diagonal tile, waves whose
     // rows are all past the end have none

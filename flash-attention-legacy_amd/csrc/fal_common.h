@@ -214,6 +214,12 @@ __device__ __forceinline__ void global_to_lds16(const void* src, void* lds_wave_
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t nbytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)nbytes, 0x00020000);
 }
+// Bytes from the first to the end of the last of `rows` rows of D 16-bit elements, `ss` elements
+// apart (less than D: rows that overlap, or at 0 one row over and over).
+template <int D>
+__device__ __forceinline__ uint32_t rows_bytes(int64_t rows, int64_t ss) {
+  return rows > 0 ? (uint32_t)(((rows - 1) * ss + D) * 2) : 0;
+}
 // 16-byte store through a raw buffer resource: a store whose offset is past the
 // resource's byte count is dropped, so rows past the end of a sequence need no branch.
 // The row goes in `voffset` (the range check covers it; an SGPR offset would not be).

@@ -49,8 +49,11 @@ AGPRs, K and V arrive in VGPRs (128), and the rest is cut to fit:
               fragment is in flight
   v[152:159], v[144:151], v143  QA, TA and LA, moved on by one slot per use (an XOR of the
               chunk index gives the eight addresses; chunks 16..31 are 256 bytes on)
-  s96/s97     record counts of the tiles' second 16 rows: the copies of rows 16..31 reuse
-              the offsets of rows 0..15 from a base 16 rows on
+  s96         rows of the tiles' second 16: the copies of rows 16..31 reuse the offsets of
+              rows 0..15 from a base 16 rows on
+  Rows may lie closer together than a row is long (a gradient broadcast over the sequence has
+  stride 0), so a record count is rows * stride plus what the last row reaches past its
+  stride (qx, dx); head_dim 128 is given no such rows.
   Ls/Dn slots hold 32 + 32 values (256 bytes), copied by one load.
 
 The output is deterministic text, tracked under csrc/gen/; build.py checks the tracked
@@ -81,7 +84,7 @@ SQ, SD, SL = 76, 80, 84
 SM = 88
 ST0, ST1, ST2, ST3, ST4 = 90, 91, 92, 93, 95
 SF = 94
-SQ2, SD2 = 96, 97
+SROW2 = 96
 RSRC_W3 = "0x00020000"
 MEASURE, ABL = False, set()
 
@@ -103,7 +106,7 @@ def operands(d):
     names = ("qb_lo", "qb_hi", "db_lo", "db_hi", "lb_lo", "lb_hi",
              "qs_lo", "qs_hi", "qw_lo", "qw_hi", "ds_lo", "ds_hi", "dw_lo", "dw_hi", "ldw",
              "qrb", "drb", "nq", "nqt", "qt0", "qs0", "nitems", "c", "negc", "kw0", "lbase", "ldbase", "scale",
-             "part", "po_lo", "po_hi")
+             "part", "po_lo", "po_hi") + (("qx", "dx") if d == 256 else ())
     return ins + [(n, "s", f"p_{n}") for n in names]
 
 
@@ -301,15 +304,17 @@ class Emitter:
         per wave, the Ls and Dn rows; then the copy state advances one item."""
         op, bm = self.op, 32 * self.nrb
         g = [[
-            # record counts: the tile's rows inside the sequence (0..64, or 0..32) times the row
-            # stride; items past the last one copy nothing (read as zeros)
+            # record counts: the tile's rows inside the sequence (0..64, or 0..32, of which 16
+            # at a time) times the row stride; items past the last one copy nothing (read as
+            # zeros)
             f"s_lshl_b32 s{ST2}, s{SQF}, {bm.bit_length() - 1}", f"s_sub_i32 s{ST2}, {op('nq')}, s{ST2}",
             f"s_max_i32 s{ST2}, s{ST2}, 0", f"s_min_i32 s{ST2}, s{ST2}, {bm}",
             f"s_cmp_lt_i32 s{SF}, {op('nitems')}",
             f"s_cselect_b32 s{ST2}, s{ST2}, 0", f"s_cselect_b32 s{SL + 2}, {hex(self.ldb)}, 0",
             f"s_mul_i32 s{SQ + 2}, s{ST2}, {op('qrb')}", f"s_mul_i32 s{SD + 2}, s{ST2}, {op('drb')}"] + ([
-            f"s_sub_i32 s{ST2}, s{ST2}, 16", f"s_max_i32 s{ST2}, s{ST2}, 0",
-            f"s_mul_i32 s{SQ2}, s{ST2}, {op('qrb')}", f"s_mul_i32 s{SD2}, s{ST2}, {op('drb')}"]
+            f"s_cmp_gt_i32 s{ST2}, 0", f"s_cselect_b32 s{ST3}, {op('qx')}, 0", f"s_cselect_b32 s{ST4}, {op('dx')}, 0",
+            f"s_add_u32 s{SQ + 2}, s{SQ + 2}, s{ST3}", f"s_add_u32 s{SD + 2}, s{SD + 2}, s{ST4}",
+            f"s_sub_i32 s{SROW2}, s{ST2}, 16", f"s_max_i32 s{SROW2}, s{SROW2}, 0"]
                 if self.d == 256 else []) + [
             f"s_and_b32 s{ST3}, s{SF}, {NBUF - 1}", f"s_lshl_b32 s{ST2}, s{ST3}, 15",
             f"s_add_u32 s{ST2}, s{ST2}, {op('lbase')}",
@@ -317,9 +322,11 @@ class Emitter:
         for part, rs, vo, base in (("q", SQ, "qo", 0), ("d", SD, "do", DOFF)):
             for i in range(4):
                 if self.d == 256 and i == 2:         # rows 16..31: same offsets, base 16 rows on
-                    rb, r2 = (op("qrb"), SQ2) if part == "q" else (op("drb"), SD2)
+                    rb, x = (op("qrb"), op("qx")) if part == "q" else (op("drb"), op("dx"))
                     g.append([f"s_lshl_b32 s{ST4}, {rb}, 4", f"s_add_u32 s{rs}, s{rs}, s{ST4}",
-                              f"s_addc_u32 s{rs + 1}, s{rs + 1}, 0", f"s_mov_b32 s{rs + 2}, s{r2}"])
+                              f"s_addc_u32 s{rs + 1}, s{rs + 1}, 0", f"s_mul_i32 s{rs + 2}, s{SROW2}, {rb}",
+                              f"s_cmp_gt_i32 s{SROW2}, 0", f"s_cselect_b32 s{ST4}, {x}, 0",
+                              f"s_add_u32 s{rs + 2}, s{rs + 2}, s{ST4}"])
                 o = op(f"{vo}{i if self.d == 128 else i % 2}")
                 g.append([f"s_add_u32 m0, s{ST2}, {base + i * 4096}", "s_nop 0"] + ([] if "nodma" in ABL else
                           [f"buffer_load_dwordx4 {o}, s[{rs}:{rs + 3}], 0 offen lds"]))

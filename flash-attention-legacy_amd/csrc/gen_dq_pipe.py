@@ -38,7 +38,9 @@ Head dim 256: a tile is 32 keys (one key block), 16 KB per K or V tile again, an
 same 48 MFMAs with half the exponentials.  dQ^T takes a[0:127] and Q and dO the other 128
 AGPRs, so the rings are v[144:175] and v[112:143], the sets v[192:223] and v[224:255]
 (S^T, dP^T), -D v[176:191], the addresses v[104:111] and v[96:103], the temporaries
-v[92:95].  Chunks 16..31 of a row are 256 bytes on.
+v[92:95].  Chunks 16..31 of a row are 256 bytes on.  Keys may lie closer together than a row
+is long (stride 0: the same key throughout), so a record count is rows * stride plus what the
+last row reaches past its stride (kx, vx); head_dim 128 is given no such rows.
 
 The output is deterministic text, tracked under csrc/gen/; build.py checks the tracked
 file against render() and rewrites it only when asked (--regen).
@@ -79,7 +81,8 @@ def operands(d):
     ins += [(f"vr{i}", "s", f"pv_rs[{i}]") for i in range(4)]
     return ins + [("c", "s", "p_c"), ("negc", "s", "p_negc"), ("jend", "s", "p_jend"), ("jl", "s", "p_jl"),
                   ("wrow", "s", "p_wrow"), ("nk", "s", "p_nk"), ("ktb", "s", "p_ktb"), ("vtb", "s", "p_vtb"),
-                  ("krb", "s", "p_krb"), ("vrb", "s", "p_vrb"), ("rows", "s", "p_rows"), ("lbase", "s", "p_lbase")]
+                  ("krb", "s", "p_krb"), ("vrb", "s", "p_vrb"), ("rows", "s", "p_rows"), ("lbase", "s", "p_lbase"),
+                  *([("kx", "s", "p_kx"), ("vx", "s", "p_vx")] if d == 256 else [])]
 
 
 def v(n):
@@ -169,7 +172,11 @@ class Emitter:
         groups = [[f"s_and_b32 s{ST}, s{SD}, {NBUF - 1}", f"s_lshl_b32 s{ST}, s{ST}, 15",
                    f"s_add_u32 s{ST}, s{ST}, {op('lbase')}",
                    f"s_max_i32 s{SK + 2}, s{SR}, 0", f"s_min_i32 s{SK + 2}, s{SK + 2}, {self.bn}",
-                   f"s_mul_i32 s{SV + 2}, s{SK + 2}, {op('vrb')}", f"s_mul_i32 s{SK + 2}, s{SK + 2}, {op('krb')}"]]
+                   f"s_mul_i32 s{SV + 2}, s{SK + 2}, {op('vrb')}"] + (
+                   [f"s_cmp_gt_i32 s{SK + 2}, 0", f"s_mul_i32 s{SK + 2}, s{SK + 2}, {op('krb')}",
+                    f"s_cselect_b32 s{ST2}, {op('vx')}, 0", f"s_cselect_b32 s{SM}, {op('kx')}, 0",
+                    f"s_add_u32 s{SV + 2}, s{SV + 2}, s{ST2}", f"s_add_u32 s{SK + 2}, s{SK + 2}, s{SM}"]
+                   if self.ks == 16 else [f"s_mul_i32 s{SK + 2}, s{SK + 2}, {op('krb')}"])]
         for part, rs, vo in (("k", SK, "kvo"), ("v", SV, "vvo")):
             for i in range(4):
                 off = i * 4096 + (VOFF if part == "v" else 0)

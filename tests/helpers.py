@@ -55,3 +55,46 @@ def cu_from_lens(lens, device="cuda"):
     for n in lens:
         cu.append(cu[-1] + int(n))
     return torch.tensor(cu, dtype=torch.int32, device=device)
+
+
+def _c_call(fn, tensors, mid, strides, scale, causal, workspace):
+    """One call of a C entry point of the library on the current stream, on operands as they are."""
+    import ctypes
+    from flash_attn_legacy import hip_ext
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    rc = fn(*[p(t) for t in tensors], *mid, *[(ctypes.c_int64 * 3)(*s) for s in strides], ctypes.c_float(scale),
+            int(causal), p(workspace), workspace.numel(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    if rc:
+        raise RuntimeError(f"status {rc}: {hip_ext._lib.fal_last_error().decode()}")
+
+
+def c_backward(do, q, k, v, o, lse, scale, causal, workspace_bytes=None, nq=None):
+    """fal_bwd with a workspace of `workspace_bytes` (fal_bwd_workspace_size's when None); the
+    gradients start out as NaN.  `nq`: query rows, if not all of q's."""
+    from flash_attn_legacy import hip_ext
+    lib = hip_ext._lib
+    (B, Hq, Nq, d), (_, Hkv, Nk, _) = q.shape, k.shape
+    nq = Nq if nq is None else nq
+    if workspace_bytes is None:
+        workspace_bytes = lib.fal_bwd_workspace_size(B, Hq, nq, d)
+    grads = [torch.full(s, float("nan"), dtype=q.dtype, device=q.device)
+             for s in ((B, Hq, Nq, d), (B, Hkv, Nk, d), (B, Hkv, Nk, d))]
+    ws = torch.empty(max(workspace_bytes, 1), dtype=torch.uint8, device=q.device)
+    _c_call(lib.fal_bwd_bf16 if q.dtype == torch.bfloat16 else lib.fal_bwd, (do, q, k, v, o, lse, *grads),
+            (B, Hq, Hkv, nq, Nk, d), [t.stride()[:3] for t in (do, q, k, v, o, *grads)], scale, causal, ws)
+    return grads
+
+
+def c_backward_varlen(do, q, k, v, o, lse, cu_q, cu_k, max_q, max_k, scale, causal, total_q=None):
+    """fal_bwd_varlen, as c_backward."""
+    from flash_attn_legacy import hip_ext
+    lib = hip_ext._lib
+    (rows_q, Hq, d), (tk, Hkv, _), seqs = q.shape, k.shape, cu_q.numel() - 1
+    tq = rows_q if total_q is None else total_q
+    grads = [torch.full(s, float("nan"), dtype=q.dtype, device=q.device)
+             for s in ((rows_q, Hq, d), (tk, Hkv, d), (tk, Hkv, d))]
+    ws = torch.empty(lib.fal_bwd_varlen_workspace_size(seqs, tq, tk, Hq, d), dtype=torch.uint8, device=q.device)
+    _c_call(lib.fal_bwd_varlen_bf16 if q.dtype == torch.bfloat16 else lib.fal_bwd_varlen,
+            (do, q, k, v, o, lse, *grads, cu_q, cu_k), (seqs, tq, tk, Hq, Hkv, d, max_q, max_k),
+            [(0, t.stride(1), t.stride(0)) for t in (do, q, k, v, o, *grads)], scale, causal, ws)
+    return grads

@@ -95,6 +95,39 @@ def test_forward_rejects_null_misaligned_and_strides(lib):
     assert fwd(lib, lse=0) == FAL_ERR_INVALID
 
 
+def c_calls(lib, d, rows, ss):
+    """(name, status) of every entry point with one operand in turn whose rows are `ss` elements
+    apart (and without L or a workspace, so that no call gets as far as a launch)."""
+    p, dense = ctypes.c_void_p(4096), s3(rows * d, rows * d, d)
+    for names, call in (
+            ("qkvo", lambda st: lib.fal_fwd(*[p] * 4, None, 1, 2, 2, rows, rows, d, *st, 0.1, 1, None, 0, None)),
+            ("qkvo", lambda st: lib.fal_fwd_varlen(*[p] * 4, None, p, p, 70, rows, rows, 2, 2, d, rows, rows, *st, 0.1, 1, None, 0, None)),
+            (("do", *"qkvo", "dq", "dk", "dv"),
+             lambda st: lib.fal_bwd(*[p] * 9, 1, 2, 2, rows, rows, d, *st, 0.1, 1, None, 0, None)),
+            (("do", *"qkvo", "dq", "dk", "dv"),
+             lambda st: lib.fal_bwd_varlen(*[p] * 11, 2, rows, rows, 2, 2, d, rows, rows, *st, 0.1, 1, None, 0, None)),
+            ((None, *"kv", None), lambda st: lib.fal_decode(p, p, p, p, None, 0, p, None, 2, 2, 2, d, rows, *st, 0.1, None, 0, None))):
+        for i, name in enumerate(names):
+            if name:
+                yield name, call([s3(rows * d, rows * d, ss) if j == i else dense for j in range(len(names))])
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("short", [0, 8, 0.5])
+def test_rows_closer_than_their_length(lib, d, short):
+    """Refused, but for the inputs of head dim 256's backward, which then lacks a workspace."""
+    ss = short if isinstance(short, int) else int(short * d)
+    seen = 0
+    for name, rc in c_calls(lib, d, 32, ss):
+        seen += 1
+        if d == 256 and seen > 8 and seen <= 24 and name not in ("dq", "dk", "dv"):
+            assert rc == FAL_ERR_WORKSPACE, (seen, name)
+        else:
+            assert rc == FAL_ERR_UNSUPPORTED, (seen, name)
+            assert b"is shorter than a row of %d elements" % d in lib.fal_last_error()
+    assert seen == 8 + 16 + 2
+
+
 def test_forward_split_workspace(lib):
     """Grids far smaller than the GPU with long key ranges (one head of 16384 rows) split
     the key range and need a workspace for the partial outputs; C1 (2 x 8 heads x 1024
