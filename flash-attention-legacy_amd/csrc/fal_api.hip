@@ -534,9 +534,12 @@ static BwdVarlenWs bwd_varlen_ws(int64_t num_seqs, int64_t total_q, int64_t tota
 size_t fal_bwd_varlen_workspace_size(int64_t num_seqs, int64_t total_q, int64_t total_k, int64_t heads_q,
                                      int64_t head_dim) {
   const int d = head_dim_ok(head_dim) ? (int)head_dim : 128;
-  // (heads_q bounds the KV heads)
+  // Where heads_q KV heads would take the pipelined kernels, the call may still take the others
+  // (it has fewer KV heads, or the GPU's size is not known here), whose list of key tiles is
+  // longer: room for either.
   const bool pipe = bwd_varlen_pipe(d, num_seqs, total_k, heads_q, device_cu_count());
-  return bwd_varlen_ws(num_seqs, total_q, total_k, heads_q, d, pipe).bytes;
+  const size_t bytes = bwd_varlen_ws(num_seqs, total_q, total_k, heads_q, d, pipe).bytes;
+  return pipe && d != 256 ? std::max(bytes, bwd_varlen_ws(num_seqs, total_q, total_k, heads_q, d, false).bytes) : bytes;
 }
 
 static int fal_bwd_varlen_impl(const void* dout, const void* q, const void* k, const void* v, const void* o, const float* lse,

@@ -171,6 +171,25 @@ def test_workspace_sizes_and_checks(lib):
     assert b"workspace needs" in lib.fal_last_error()
 
 
+@pytest.mark.parametrize("hq", [1, 2, 3, 8, 32])
+def test_packed_backward_workspace_covers_either_form(lib, hq):
+    """fal_bwd_varlen_workspace_size does not know the KV heads, which decide whether head dim
+    128 runs the kernel of 64 keys or of 128 and a tile-order copy of L and D per workgroup:
+    from few queries with many keys to the reverse the size covers the call's need."""
+    up = lambda x: (x + 255) // 256 * 256
+    for seqs in (1, 2, 7, 100, 3000):
+        for tq in (0, 1, 16, 128, 129, 5000, 98048, 1 << 20):
+            for tk in (1, 500, 40000, 49152, 71680, 98048, 98304, 200000, 1 << 21):
+                capq = -(-tq // 128) + seqs
+                both = up(tq * hq * 4) + up(capq * 8)                  # D, query-tile list
+                small = both + up((-(-tk // 64) + seqs) * 8)
+                pipe = both + up((-(-tk // 128) + seqs) * 8) + up(seqs * 4) + up(hq * capq * 1024)
+                size = lib.fal_bwd_varlen_workspace_size(seqs, tq, tk, hq, 128)
+                assert size >= small, (seqs, tq, tk)
+                if size != small:
+                    assert size == max(small, pipe), (seqs, tq, tk)
+
+
 def test_decode_rejects_large_groups(lib):
     p = ctypes.c_void_p(4096)
     st = s3(64 * 128, 128, 0)

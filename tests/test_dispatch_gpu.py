@@ -156,3 +156,11 @@ def test_backward_runs(B, Hq, Hkv, Nq, Nk, d, causal):
 def test_packed_backward_pipelined(lens_q, lens_k, hq, hkv, d, causal):
     from test_varlen_gpu import bwd_check
     bwd_check(lens_q, lens_k, hq, hkv, d, causal)
+
+
+# fal_bwd_varlen_workspace_size knows the query heads only, and with them may expect the other
+# dK/dV kernel than the call (which goes by the KV heads) takes: its size covers both.
+@pytest.mark.parametrize("nq,nk", [(16, 98048), (1, 71680)])
+def test_packed_backward_few_queries_many_keys(nq, nk):
+    from test_varlen_gpu import bwd_check
+    bwd_check([nq], [nk], 2, 1, 128, False)
