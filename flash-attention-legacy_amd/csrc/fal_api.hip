@@ -466,7 +466,7 @@ static int fal_bwd_impl(const void* dout, const void* q, const void* k, const vo
   p.delta = static_cast<float*>(workspace);
   const size_t lsd = bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim);
   const size_t lsd_at = align256(rows * sizeof(float));
-  if (lsd) {
+  if (bwd_pipe((int)head_dim)) {   // (without query rows too, where the array is empty)
     p.lsd = reinterpret_cast<float*>(static_cast<char*>(workspace) + lsd_at);
     p.lsd_tiles = cdiv((int)seqlen_q, bwd_pipe_bm((int)head_dim));
     p.kv_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + lsd_at + lsd);

@@ -4,7 +4,8 @@ that choose a kernel or a work order by problem size."""
 import pytest
 import torch
 
-from helpers import FWD_ATOL, GRAD_RTOL, max_abs, oracle_bwd, oracle_fwd, randn, rel_err
+from helpers import (FWD_ATOL, GRAD_RTOL, c_backward, c_backward_varlen, max_abs, oracle_bwd, oracle_fwd, randn,
+                     rel_err)
 
 pytestmark = pytest.mark.gpu
 
@@ -164,3 +165,18 @@ def test_packed_backward_pipelined(lens_q, lens_k, hq, hkv, d, causal):
 def test_packed_backward_few_queries_many_keys(nq, nk):
     from test_varlen_gpu import bwd_check
     bwd_check([nq], [nk], 2, 1, 128, False)
+
+
+# No query rows: every dK and dV row is written, as zeros.
+@pytest.mark.parametrize("d", [32, 64, 96, 128, 256])
+def test_backward_without_queries(d):
+    B, Hq, Hkv, Nk = 2, 4, 2, 300
+    k, v, one = randn((B, Hkv, Nk, d), 0), randn((B, Hkv, Nk, d), 1), randn((B, Hq, 1, d), 2)
+    lse = torch.zeros((B, Hq, 1), device="cuda")
+    _, dk, dv = c_backward(one, one, k, v, one, lse, 0.1, False, nq=0)
+    assert not dk.any() and not dv.any()
+    cu_q, cu_k = torch.zeros(3, dtype=torch.int32, device="cuda"), torch.tensor([0, 100, 300], dtype=torch.int32, device="cuda")
+    one = randn((1, Hq, d), 2)
+    _, dk, dv = c_backward_varlen(one, one, k[0].transpose(0, 1), v[0].transpose(0, 1), one, lse[0], cu_q, cu_k, 0, 200,
+                                  0.1, False, total_q=0)
+    assert not dk.any() and not dv.any()
