@@ -565,7 +565,8 @@ static int fal_bwd_varlen_impl(const void* dout, const void* q, const void* k, c
   const int d = (int)head_dim;
   bool pipe = bwd_varlen_pipe(d, num_seqs, total_k, heads_kv, device_cu_count());
   BwdVarlenWs w = bwd_varlen_ws(num_seqs, total_q, total_k, heads_q, d, pipe);
-  // (the pipelined loop steps from one query head's lsd tiles to the next one's by 32 bits)
+  // (head_dim 128's pipelined loop steps from one query head's lsd tiles to the next one's by 32
+  // bits)
   const bool far = heads_q > heads_kv && w.capq >= (1 << 22);
   if (pipe && d != 256 && (far || workspace_bytes < w.bytes)) {   // (head_dim 256 has no other form)
     pipe = false;
@@ -594,7 +595,7 @@ static int fal_bwd_varlen_impl(const void* dout, const void* q, const void* k, c
   p.cu_q = cu_seqlens_q;
   p.cu_k = cu_seqlens_k;
   p.work = work;
-  if (w.cap * heads_kv > 0x7fffffff || w.capq > 0x7fffffff || (pipe && far))
+  if (w.cap * heads_kv > 0x7fffffff || w.capq > 0x7fffffff)
     return fail(FAL_ERR_INVALID, "problem too large for one launch");
   const int bn = pipe ? 128 : bwd_block_n(d), cap = (int)w.cap;
   int nb = cdiv((int)(max_seqlen_k > 0 ? max_seqlen_k : 1), bn);

@@ -614,7 +614,9 @@ bwd_kv_pipe_kernel(BwdParams p) {
       const uint32_t p_ds_lo = (uint32_t)(dstep - dhalf), p_ds_hi = (uint32_t)((uint64_t)(dstep - dhalf) >> 32);
       const uint32_t p_dw_lo = (uint32_t)dwrap, p_dw_hi = (uint32_t)((uint64_t)dwrap >> 32);
       // last tile of a head -> first of the next
-      const uint32_t p_ldw = (uint32_t)(p.lsd_tiles - nqt + 1 + qt0) * 2 * kPipeBM * 4;
+      const uint64_t ldw = (uint64_t)(p.lsd_tiles - nqt + 1 + qt0) * 2 * kPipeBM * 4;
+      const uint32_t p_ldw = (uint32_t)ldw, p_ldw_hi = (uint32_t)(ldw >> 32);   // (high word: head_dim 256)
+      (void)p_ldw_hi;
       const int p_qt0 = qt0, p_qs0 = q0, p_nitems = nitems;
       const int p_part = SPLIT ? __builtin_amdgcn_readfirstlane(nruns - 1) : 0;
       // dV and dK sums of this wave's 32 keys

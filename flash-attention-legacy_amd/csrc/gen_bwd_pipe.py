@@ -51,6 +51,8 @@ AGPRs, K and V arrive in VGPRs (128), and the rest is cut to fit:
               chunk index gives the eight addresses; chunks 16..31 are 256 bytes on)
   s96         rows of the tiles' second 16: the copies of rows 16..31 reuse the offsets of
               rows 0..15 from a base 16 rows on
+  s97         high word of the step to the next item's Ls and Dn: packed sequences of few rows put
+              one head's last item 4 GB before the next head's first
   Rows may lie closer together than a row is long (a gradient broadcast over the sequence has
   stride 0), so a record count is rows * stride plus what the last row reaches past its
   stride (qx, dx); head_dim 128 is given no such rows.
@@ -84,7 +86,7 @@ SQ, SD, SL = 76, 80, 84
 SM = 88
 ST0, ST1, ST2, ST3, ST4 = 90, 91, 92, 93, 95
 SF = 94
-SROW2 = 96
+SROW2, SLHI = 96, 97
 RSRC_W3 = "0x00020000"
 MEASURE, ABL = False, set()
 
@@ -106,7 +108,7 @@ def operands(d):
     names = ("qb_lo", "qb_hi", "db_lo", "db_hi", "lb_lo", "lb_hi",
              "qs_lo", "qs_hi", "qw_lo", "qw_hi", "ds_lo", "ds_hi", "dw_lo", "dw_hi", "ldw",
              "qrb", "drb", "nq", "nqt", "qt0", "qs0", "nitems", "c", "negc", "kw0", "lbase", "ldbase", "scale",
-             "part", "po_lo", "po_hi") + (("qx", "dx") if d == 256 else ())
+             "part", "po_lo", "po_hi") + (("qx", "dx", "ldw_hi") if d == 256 else ())
     return ins + [(n, "s", f"p_{n}") for n in names]
 
 
@@ -339,10 +341,13 @@ class Emitter:
             f"s_add_u32 s{SQF}, s{SQF}, 1", f"s_cmp_eq_u32 s{SQF}, {op('nqt')}",
             f"s_cselect_b32 s{ST0}, {op('qw_lo')}, {op('qs_lo')}", f"s_cselect_b32 s{ST1}, {op('qw_hi')}, {op('qs_hi')}",
             f"s_cselect_b32 s{ST2}, {op('dw_lo')}, {op('ds_lo')}", f"s_cselect_b32 s{ST3}, {op('dw_hi')}, {op('ds_hi')}",
-            f"s_cselect_b32 s{ST4}, {op('ldw')}, {hex(self.ldb)}", f"s_cselect_b32 s{SQF}, {op('qt0')}, s{SQF}",
+            f"s_cselect_b32 s{ST4}, {op('ldw')}, {hex(self.ldb)}"] + (
+            [f"s_cselect_b32 s{SLHI}, {op('ldw_hi')}, 0"] if self.d == 256 else []) + [
+            f"s_cselect_b32 s{SQF}, {op('qt0')}, s{SQF}",
             f"s_add_u32 s{SQ}, s{SQ}, s{ST0}", f"s_addc_u32 s{SQ + 1}, s{SQ + 1}, s{ST1}",
             f"s_add_u32 s{SD}, s{SD}, s{ST2}", f"s_addc_u32 s{SD + 1}, s{SD + 1}, s{ST3}",
-            f"s_add_u32 s{SL}, s{SL}, s{ST4}", f"s_addc_u32 s{SL + 1}, s{SL + 1}, 0",
+            f"s_add_u32 s{SL}, s{SL}, s{ST4}",
+            f"s_addc_u32 s{SL + 1}, s{SL + 1}, " + (f"s{SLHI}" if self.d == 256 else "0"),
             f"s_add_u32 s{SF}, s{SF}, 1"])
         return g
 

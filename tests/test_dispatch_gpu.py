@@ -180,3 +180,29 @@ def test_backward_without_queries(d):
     _, dk, dv = c_backward_varlen(one, one, k[0].transpose(0, 1), v[0].transpose(0, 1), one, lse[0], cu_q, cu_k, 0, 200,
                                   0.1, False, total_q=0)
     assert not dk.any() and not dv.any()
+
+
+# More sequences than a 32-bit step between two heads' rows of the row-value array can count
+# (4 million query tiles), at head_dim 256 with grouped heads: sequences of one query row and
+# two keys, a sample of them against fp32.
+def test_packed_backward_millions_of_sequences():
+    from flash_attn_legacy import hip_ext
+    seqs, hq, hkv, d = (1 << 22) + 1000, 2, 1, 256
+    rnd = lambda rows, h, seed: torch.randn((rows, h, d), dtype=torch.float16, device="cuda",
+                                            generator=torch.Generator(device="cuda").manual_seed(seed))
+    q, do, k, v = rnd(seqs, hq, 0), rnd(seqs, hq, 1), rnd(2 * seqs, hkv, 2), rnd(2 * seqs, hkv, 3)
+    cu_q = torch.arange(seqs + 1, dtype=torch.int32, device="cuda")
+    tail = (cu_q, 2 * cu_q, 1, 2, 0.0625, False)
+    o, lse = hip_ext.forward_varlen(q, k, v, *tail)
+    dq, dk, dv = hip_ext.backward_varlen(do, q, k, v, o, lse, *tail)
+    s = torch.cat([torch.arange(500), torch.arange(seqs - 500, seqs), torch.arange(0, seqs, 997)]).cuda()
+    pick = lambda t: t[s].float()
+    keys = lambda t: torch.stack([t[2 * s, 0], t[2 * s + 1, 0]], 1).float()
+    fq, fdo, fk, fv = pick(q), pick(do), keys(k), keys(v)            # [n, heads, d], [n, keys, d]
+    dot = lambda a, b: (a[:, :, None] * b[:, None]).sum(-1)          # [n, heads, keys]
+    p = torch.softmax(dot(fq, fk) * 0.0625, -1)
+    dp = dot(fdo, fv)
+    ds = p * (dp - (p * dp).sum(-1, keepdim=True)) * 0.0625
+    assert rel_err(dq[s], (ds[..., None] * fk[:, None]).sum(2)) <= GRAD_RTOL
+    assert rel_err(keys(dk), (ds[..., None] * fq[:, :, None]).sum(1)) <= GRAD_RTOL
+    assert rel_err(keys(dv), (p[..., None] * fdo[:, :, None]).sum(1)) <= GRAD_RTOL
