@@ -12,6 +12,8 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -77,9 +79,7 @@ std::string shape_str(at::IntArrayRef s) {
 // problem's sizes, so a smaller tensor would be read out of bounds)
 void check_lse(const Tensor& l, at::IntArrayRef shape, const Tensor& q) {
   if (l.scalar_type() == at::kFloat && l.sizes() == shape && l.device() == q.device()) return;
-  std::string type = c10::toString(l.scalar_type());
-  std::transform(type.begin(), type.end(), type.begin(), ::tolower);
-  if (type == "float") type = "float32";
+  const std::string type = torch::getTHPDtype(l.scalar_type())->name;   // (torch's own: "float16")
   fail("L must be float32 " + shape_str(shape) + " on " + q.device().str() + ", got torch." + type + " " +
        shape_str(l.sizes()) + " on " + l.device().str());
 }

@@ -126,6 +126,18 @@ def test_backward_shape_checks():
         hip_ext.backward(do, q, torch.cat([k, k]), torch.cat([v, v]), o, lse, 0.125, False)   # batch
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float64, torch.int32, torch.int64,
+                                   torch.uint8, torch.bool])
+def test_wrong_lse_is_named(dtype):
+    """The message names the type, sizes and device of the L that was given, as torch does."""
+    from flash_attn_legacy import hip_ext
+    q, k, v, do = (randn((1, 2, 64, 64), seed=s) for s in (141, 142, 143, 144))
+    o, lse = hip_ext.forward(q, k, v, 0.125, False)
+    with pytest.raises(RuntimeError) as e:
+        hip_ext.backward(do, q, k, v, o, lse.to(dtype), 0.125, False)
+    assert str(e.value) == f"L must be float32 [1, 2, 64] on cuda:0, got {dtype} [1, 2, 64] on cuda:0"
+
+
 def test_backward_varlen_checks():
     from flash_attn_legacy import hip_ext
     total, H, d = 96, 2, 64
