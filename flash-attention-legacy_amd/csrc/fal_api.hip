@@ -373,15 +373,15 @@ static size_t bwd_need(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t
   return align256(rows * sizeof(float)) + bwd_lsd_bytes(batch, heads_q, seqlen_q, head_dim);
 }
 
+// At most this much goes to the partial dK/dV sums (512 key tiles at head_dim 256).
+constexpr size_t kKvPartMax = size_t(128) << 20;
+
 size_t fal_bwd_workspace_size(int64_t batch, int64_t heads_q, int64_t seqlen_q, int64_t head_dim) {
   // (head_dim 256: with room for partial dK/dV sums, one fp32 row per query row)
   const size_t rows = (size_t)batch * heads_q * seqlen_q;
   return bwd_need(batch, heads_q, seqlen_q, head_dim) +
-         (head_dim == 256 ? align256(rows * head_dim * sizeof(float)) : 0);
+         (head_dim == 256 ? std::min(align256(rows * head_dim * sizeof(float)), kKvPartMax) : 0);
 }
-
-// At most this much goes to the partial dK/dV sums (512 key tiles at head_dim 256).
-constexpr size_t kKvPartMax = size_t(128) << 20;
 
 size_t fal_bwd_workspace_best(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t seqlen_q, int64_t seqlen_k,
                               int64_t head_dim, int is_causal) {
