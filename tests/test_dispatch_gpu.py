@@ -74,6 +74,7 @@ def test_head_dim_128_full_grid(B, Hq, Hkv, Nq, Nk, sign, causal):
 # Head dim 64 at 16 key tiles and more on up to 512 workgroups: the pipelined loop.  Whole and
 # partial last key tiles and query tiles, the three lengths around 16 tiles, waves without
 # rows, unequal lengths, GQA; a negative scale and values that move the row's reference max.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("B,Hq,Hkv,Nq,Nk,mul", [
     (2, 16, 16, 960, 960, 1),
@@ -83,15 +84,18 @@ def test_head_dim_128_full_grid(B, Hq, Hkv, Nq, Nk, sign, causal):
     (1, 33, 11, 1700, 993, 12),
     (8, 16, 16, 40, 1100, 12),
 ])
-def test_head_dim_64_long_tiles(B, Hq, Hkv, Nq, Nk, mul, causal):
+def test_head_dim_64_long_tiles(B, Hq, Hkv, Nq, Nk, mul, causal, dtype):
     from flash_attn_legacy import hip_ext
-    q, k, v = randn((B, Hq, Nq, 64), 0), randn((B, Hkv, Nk, 64), 1), randn((B, Hkv, Nk, 64), 2)
+    q, k, v = (randn((B, h, n, 64), i).to(dtype) for i, (h, n) in enumerate([(Hq, Nq), (Hkv, Nk), (Hkv, Nk)]))
     scale = mul * 64 ** -0.5
     o, lse = hip_ext.forward(q, k, v, scale, causal)
     ref_o, ref_l = oracle_fwd(q, k, v, scale, causal)
     # P and O are rounded to fp16 once each: 2^-11 * sum(P |V|) + 2^-11 |O| <= 2^-10 max |V|
-    # (scores of a scale of 12 concentrate P on few keys, so |O| comes near max |V|); L is fp32
-    assert max_abs(o, ref_o) <= (FWD_ATOL if abs(mul) == 1 else 2 ** -10 * float(v.abs().max()))
+    # (scores of a scale of 12 concentrate P on few keys, so |O| comes near max |V|); to bf16
+    # 2^-8 each; L is fp32
+    top = float(v.abs().max())
+    bound = 2 ** -7 * top if dtype == torch.bfloat16 else FWD_ATOL if abs(mul) == 1 else 2 ** -10 * top
+    assert max_abs(o, ref_o) <= bound
     assert max_abs(lse, ref_l) <= FWD_ATOL
 
 
@@ -127,8 +131,8 @@ def test_head_dim_256_backward(B, Hq, Hkv, Nq, Nk, sign, causal):
 
 # Pipelined backward on small grids, where each key tile's items are cut into runs whose sums a
 # second kernel adds: runs that start inside a head, key tiles of one run only (the last
-# causal ones), a last key tile of one key, MQA and GQA; and a call whose keys outnumber its
-# queries by so much that the workspace has no room for the sums.
+# causal ones), a last key tile of one key, MQA and GQA; and a call with too few queries for
+# its keys to be worth cutting.
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("B,Hq,Hkv,Nq,Nk,d", [
     (1, 8, 1, 257, 257, 128),
@@ -143,10 +147,75 @@ def test_backward_runs(B, Hq, Hkv, Nq, Nk, d, causal):
     check_gradients(B, Hq, Hkv, Nq, Nk, d, causal)
 
 
+# The same through the library with less workspace: what the call cannot do without (no runs),
+# room for some of the runs, and fal_bwd_workspace_best's.
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,Nq,Nk,d", [(1, 28, 4, 333, 333, 128), (1, 6, 1, 515, 129, 256)])
+def test_backward_runs_by_workspace(B, Hq, Hkv, Nq, Nk, d, causal):
+    from flash_attn_legacy import hip_ext
+    q, k, v, do = (randn(s, i) for i, s in enumerate(
+        [(B, Hq, Nq, d), (B, Hkv, Nk, d), (B, Hkv, Nk, d), (B, Hq, Nq, d)]))
+    scale = d ** -0.5
+    o, lse = hip_ext.forward(q, k, v, scale, causal)
+    with pytest.raises(RuntimeError, match="workspace needs") as e:
+        c_backward(do, q, k, v, o, lse, scale, causal, workspace_bytes=0)
+    need = int(str(e.value).split("needs ")[1].split()[0])
+    best = hip_ext._lib.fal_bwd_workspace_best(B, Hq, Hkv, Nq, Nk, d, int(causal))
+    slot = 128 * d * 2 * 4                      # one workgroup's sums
+    assert best >= need + 2 * slot              # the call does cut its key tiles
+    ref = oracle_bwd(q, k, v, do, scale, causal)
+    for room in (0, slot, (best - need) // 2, best - need):
+        got = c_backward(do, q, k, v, o, lse, scale, causal, workspace_bytes=need + room)
+        for name, g, r in zip(("dq", "dk", "dv"), got, ref):
+            assert rel_err(g, r) <= GRAD_RTOL, (name, room)
+    same = hip_ext.backward(do, q, k, v, o, lse, scale, causal)
+    assert all(torch.equal(a, b) for a, b in zip(got, same))       # (the binding gives the best)
+
+
+# At most 128 MB of workspace for the runs' sums, also where more would be of use.
+@pytest.mark.parametrize("d", [128, 256])
+def test_backward_runs_workspace_bound(d):
+    from flash_attn_legacy import hip_ext
+    lib, sizes = hip_ext._lib, []
+    for Hq, Hkv in ((8, 1), (32, 8), (16, 16), (128, 1)):
+        for N in (300, 1024, 2048, 4096, 8192, 16384, 32768):
+            for causal in (0, 1):
+                need = lib.fal_bwd_workspace_size(1, Hq, N, d) - (min(Hq * N * d * 4, 128 << 20) if d == 256 else 0)
+                sizes.append(lib.fal_bwd_workspace_best(1, Hq, Hkv, N, N, d, causal) - need)
+    assert max(sizes) > 64 << 20 and max(sizes) <= 128 << 20 and min(sizes) >= 0
+
+
+# Token-major operands, each its own [B, N, H, d] tensor or all slices of one fused projection,
+# on the pipelined backward: grids that split their key tiles and grids that do not.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,N,d", [
+    (1, 8, 2, 260, 256),
+    (8, 16, 16, 385, 256),
+    (1, 28, 4, 333, 128),
+    (8, 16, 16, 385, 128),
+])
+def test_backward_token_major(B, Hq, Hkv, N, d, fused, causal, dtype):
+    from flash_attn_legacy import hip_ext
+    rows = lambda h, seed: randn((B, N, h, d), seed).to(dtype).transpose(1, 2)
+    q, k, v = (torch.split(rows(Hq + 2 * Hkv, 0), [Hq, Hkv, Hkv], 1) if fused else
+               [rows(h, i) for i, h in enumerate((Hq, Hkv, Hkv))])
+    do, scale = rows(Hq, 3), d ** -0.5
+    o, lse = hip_ext.forward(q, k, v, scale, causal)
+    got = hip_ext.backward(do, q, k, v, o, lse, scale, causal)
+    dense = hip_ext.backward(*(t.contiguous() for t in (do, q, k, v)), o, lse, scale, causal)
+    rtol = 4e-2 if dtype == torch.bfloat16 else GRAD_RTOL          # (three mantissa bits less)
+    for name, g, g2, ref in zip(("dq", "dk", "dv"), got, dense, oracle_bwd(q, k, v, do, scale, causal)):
+        assert torch.equal(g, g2), name
+        assert rel_err(g, ref) <= rtol, name
+
+
 # Packed backward on the pipelined kernels: head_dim 256 always, head_dim 128 from 768 key
 # tiles (times KV heads) of sequences of 512 keys on average.  Sequences that end inside a
 # query item or key tile, of one row, without queries or keys, in an order that the work
 # lists change; GQA, where one head's rows of the row-value array are followed by the next's.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("lens_q,lens_k,hq,hkv,d", [
     ([1, 33, 300, 129], [1, 33, 300, 129], 4, 2, 256),
@@ -154,9 +223,12 @@ def test_backward_runs(B, Hq, Hkv, Nq, Nk, d, causal):
     ([515, 1201, 64, 700, 641], [515, 1201, 64, 700, 641], 32, 32, 128),
     ([600, 0, 1100, 70], [1, 900, 2200, 3100], 32, 16, 128),
 ])
-def test_packed_backward_pipelined(lens_q, lens_k, hq, hkv, d, causal):
+def test_packed_backward_pipelined(lens_q, lens_k, hq, hkv, d, causal, dtype):
     from test_varlen_gpu import bwd_check
-    bwd_check(lens_q, lens_k, hq, hkv, d, causal)
+    if dtype == torch.float16:
+        bwd_check(lens_q, lens_k, hq, hkv, d, causal)
+    else:
+        bwd_check(lens_q, lens_k, hq, hkv, d, causal, dtype=dtype, rtol=4e-2)   # (three mantissa bits less)
 
 
 # fal_bwd_varlen_workspace_size knows the query heads only, and with them may expect the other

@@ -88,12 +88,12 @@ def test_work_items_on_both_sides_of_64_sequences(nseq, causal):
     fwd_check(lens, lens, 2, 1, 64, causal, seed=nseq)
 
 
-def bwd_check(lens_q, lens_k, hq, hkv, d, causal, seed=0):
+def bwd_check(lens_q, lens_k, hq, hkv, d, causal, seed=0, dtype=torch.float16, rtol=GRAD_RTOL):
     tq, tk = sum(lens_q), sum(lens_k)
-    q = randn((tq, hq, d), seed=seed)
-    k = randn((tk, hkv, d), seed=seed + 1)
-    v = randn((tk, hkv, d), seed=seed + 2)
-    do = randn((tq, hq, d), seed=seed + 3)
+    q = randn((tq, hq, d), seed=seed).to(dtype)
+    k = randn((tk, hkv, d), seed=seed + 1).to(dtype)
+    v = randn((tk, hkv, d), seed=seed + 2).to(dtype)
+    do = randn((tq, hq, d), seed=seed + 3).to(dtype)
     cu_q, cu_k = cu_from_lens(lens_q), cu_from_lens(lens_k)
     scale = 1.0 / math.sqrt(d)
     qg, kg, vg = (t.clone().requires_grad_(True) for t in (q, k, v))
@@ -102,7 +102,7 @@ def bwd_check(lens_q, lens_k, hq, hkv, d, causal, seed=0):
                          scale, causal)
     for name, g, r in zip(("dq", "dk", "dv"), (qg.grad, kg.grad, vg.grad), ref):
         e = rel_err(g, torch.from_numpy(r))
-        assert e <= GRAD_RTOL, f"{name} rel err {e:.3e}"
+        assert e <= rtol, f"{name} rel err {e:.3e}"
 
 
 @pytest.mark.parametrize("d", [32, 64, 96, 128, 256])
