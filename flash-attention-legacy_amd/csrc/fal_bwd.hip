@@ -422,7 +422,7 @@ bwd2_kernel(BwdParams p) {
 
 
 // --------------------------------------------------------------------------
-// dK/dV kernel for head_dim 128 and 256, batched (bwd_kv_pipe_kernel): one wave per SIMD and
+// dK/dV kernel for head_dim 128 and 256 (bwd_kv_pipe_kernel): one wave per SIMD and
 // a software-pipelined query-tile loop written as one inline-asm block (fal_bwd_pipe.inc,
 // generated by gen_bwd_pipe.py).  A workgroup owns 128 keys of one KV head, each wave
 // 32 keys whose K and V fragments stay in registers; the items (query head of the
@@ -716,7 +716,7 @@ bwd_kv_reduce_kernel(BwdParams p) {
 }
 
 // --------------------------------------------------------------------------
-// Query-outer dQ kernel for head_dim 32, 64, 96 and 128, and batched 256 (the KV-outer
+// Query-outer dQ kernel of every head dim (the KV-outer
 // kernel above then produces only dK/dV).  Same structure as the forward kernel: a workgroup owns
 // 32*NW query rows of one query head, each wave 32 rows whose Q and dO slices stay
 // in VGPRs as the B operands of S^T = K Q^T and dP^T = V dO^T; K/V tiles of BN keys
@@ -750,7 +750,7 @@ bwd_dq_kernel(BwdParams p) {
   constexpr int PART = BN * CPR * 8;
   constexpr int IPT = BN * CPR / (NW * 64);
   static_assert(BN * CPR % (NW * 64) == 0, "tile must split evenly over the waves");
-  // PIPE (batched, head_dim 128 and 256): the key-tile loop is the software-pipelined asm
+  // PIPE (head_dim 128 and 256): the key-tile loop is the software-pipelined asm
   // block of fal_dq_pipe.inc at one wave per SIMD, with a ring of 4 K/V tiles
   static_assert(!PIPE || ((D == 128 || D == 256) && NW == 4 && BN * D == 8192),
                 "the pipelined loop is written for these shapes");

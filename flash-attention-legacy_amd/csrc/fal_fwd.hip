@@ -872,7 +872,7 @@ fwd_kernel(FwdParams p) {
   constexpr bool PIPE = FwdPipe<D, NW, BN, RB, SMALL>::any, WIDE = FwdPipe<D, NW, BN, RB, SMALL>::wide;
   constexpr int PART = BN * SwizzledTile<D>::CPR * 8;
   constexpr int NSLOT = PIPE ? 4 : 2;
-  // (the O hand-off of the pipelined head_dim-128 and -32 loops reaches past the ring)
+  // (the O hand-off of the pipelined head_dim-128 loop reaches past the ring)
   constexpr int NOUT = PIPE ? NW * pipe_owave<D, RB>() / 2 : 0;
   constexpr int NSMEM = NSLOT * 2 * PART > NOUT ? NSLOT * 2 * PART : NOUT;
   __shared__ __attribute__((aligned(1024))) T smem[NSMEM];
@@ -1225,9 +1225,10 @@ bool fwd_small_pipe(int d, int64_t nblocks, int64_t Nq, int64_t Nk, int causal, 
 
 // Order of a causal grid.  Head by head puts query tile t of every head on the same CU
 // whenever the tiles of a head divide the XCD's 32 CUs, so the CUs that hold the last tiles
-// run several times as long as those that hold the first ones.  Up to two workgroups per CU
-// (what the registers allow; one for head_dim 256) are all resident at once, and are paired
-// longest with shortest; larger grids are dealt dynamically, longest first, up to 16 per CU.
+// run several times as long as those that hold the first ones.  Up to two workgroups per CU are
+// all resident at once (the registers leave room for two, for three at head_dim 64, for one at
+// 256), and are paired longest with shortest; larger grids are dealt dynamically, longest first,
+// up to 16 per CU.
 // Beyond that the imbalance is lost in the rounds, and head by head keeps one head's K/V in
 // an XCD's L2.  MI355X, us per call before -> after: B4 x 16 heads x 2048, head_dim 32
 // 47.4 -> 33, 64 65 -> 53, 96 85 -> 68; B2 x 16 x 2048 x 64 42 -> 33; B4 x 12 x 1000 x 64
@@ -1245,14 +1246,16 @@ int fwd_causal_order(int d, int64_t nblocks, int64_t units, int ncu) {
 // pipelined grid leaves CUs idle, ends in a nearly empty round, or pays its start and end
 // (about 10 us, overlapped by nothing) for a few tiles.  The estimates below are fitted to 50
 // shapes of MI355X times (batch 1-128, 100-8192 rows, MHA and GQA, causal or not): they pick
-// the faster kernel or the pipelined one on each.  us, pipelined / 128-row: 1 x 32/8 heads x
+// the faster kernel on each, or the pipelined one where the next paragraph keeps it.  us,
+// pipelined / 128-row: 1 x 32/8 heads x
 // 1531 causal 43 / 34, 4 x 32/8 x 512 causal 24 / 19, 5 x 28/4 x 777 causal 87 / 44,
 // 4 x 16 x 1024 causal 37 / 30, 32 x 16 x 256 41 / 33; 2 x 32/8 x 2048 causal 76 / 82,
 // 1 x 32/8 x 2048 non-causal 66 / 73.
 // The 128-row workgroups copy twice the K/V per flop.  A long causal grid of one item per CU
 // lets CUs idle, which at the board's power limit comes back as clock, also for the kernels
 // around it: 2 x 16 x 2048 causal alone takes 62 / 54 us, but a training step of it 195 / 197.
-// Such grids need a margin.
+// Such grids need a margin (1.4, from 24 key tiles on), which a forward that no backward follows
+// pays for: 2 x 16 x 2048 causal keeps the kernel that takes 62.
 bool fwd_wide_pays(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int causal, int ncu) {
   if (ncu <= 0 || Nq <= 0 || Nk <= 0) return true;
   const double cus = ncu;

@@ -141,8 +141,6 @@ bool fwd_pipe_ok(int d);   // batched calls of this head dim run the pipelined t
 bool fwd_gqa4_ok(int d, int64_t heads_q, int64_t heads_kv);   // FwdParams::gqa4 applies
 int fwd_block_m_varlen(int d);   // query rows per workgroup of a packed-sequence call
 int fwd_block_n(int d);
-// Split-KV plan for a batched forward: sets kchunk / nsplit (kchunk 0 = no split) and
-// returns the workspace bytes the split needs (0 without a split).
 // True when the pipelined kernel is the faster of head_dim 128's two for this batched call.
 bool fwd_wide_pays(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int causal, int ncu);
 // FwdParams::small of a batched grid of `nblocks` workgroups (no split) on a GPU of `ncu`
@@ -151,6 +149,8 @@ bool fwd_small_pipe(int d, int64_t nblocks, int64_t Nq, int64_t Nk, int causal, 
 // FwdParams::lpt of a causal grid of `nblocks` workgroups over `units` heads (batch x query
 // head) on a GPU of `ncu` compute units.
 int fwd_causal_order(int d, int64_t nblocks, int64_t units, int ncu);
+// Split-KV plan for a batched forward: sets kchunk / nsplit (kchunk 0 = no split) and
+// returns the workspace bytes the split needs (0 without a split).
 size_t fwd_split_plan(int64_t B, int64_t Hq, int64_t Nq, int64_t Nk, int d, int causal, int* kchunk, int* nsplit);
 hipError_t launch_fwd_combine(const FwdParams& p, int d, int causal, hipStream_t st);
 // Rows of up to two packed [rows, heads, d] 16-bit tensors that the schedule kernel

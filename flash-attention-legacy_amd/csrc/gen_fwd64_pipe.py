@@ -33,8 +33,8 @@ tile); every wave runs every iteration's copy and barrier.  Tiles before `jf` ne
 and are followed by another tile of the wave: they run the loop's short path.
 
 Registers (per lane; VGPRs only):
-  O     O^T accumulators, (rb*DB + db)*16 + i
-  SA    S^T of two consecutive tiles, rb*32 + kb*16 + i; a tile's P^T (fp16/bf16 pairs) is
+  O     O^T accumulators, db*16 + i
+  SA    S^T of two consecutive tiles, kb*16 + i; a tile's P^T (fp16/bf16 pairs) is
         packed in place into the first 8 registers of each 16-register block
   KF, VF  K fragment ring (2*KS x 4), V^T fragment ring (8 x 4)
   LT per-lane P sums, NM -m, T0..T3 temporaries
@@ -52,7 +52,6 @@ import sys
 NBUF = 4            # LDS ring slots
 OSTR = 1040         # bytes between a wave's O blocks in the LDS hand-off (kPipeOStr in fal_fwd.hip)
 D = 64
-RB = 1              # 32-row blocks per wave (two, at one wave per SIMD, were no faster)
 # Knobs (set by configure(); the values here are the product kernel's)
 DEFAULTS = {
     "DIST": 8,        # LDS reads issued ahead of the MFMA that needs them
@@ -81,15 +80,13 @@ def vr(n, k):
 def operands(d=D):
     """(name, constraint, C++ expression) of the block's outputs and inputs."""
     ks, db, ipt = d // 16, d // 32, d // 32
-    outs = [(f"m{rb}", "+v", f"m_run[{rb}]") for rb in range(RB)]
-    outs += [(f"l{rb}", "+v", f"l_run[{rb}]") for rb in range(RB)]
-    ins = [(f"Q{rb}{t}", "v", f"qreg[{rb}][{t}]") for rb in range(RB) for t in range(ks)]
+    outs = [("m", "+v", "m_run[0]"), ("l", "+v", "l_run[0]")]
+    ins = [(f"Q{t}", "v", f"qreg[0][{t}]") for t in range(ks)]
     ins += [(f"kvo{i}", "v", f"kvo[{i}]") for i in range(ipt)]
     ins += [(f"vvo{i}", "v", f"vvo[{i}]") for i in range(ipt)]
     ins += [(f"ka{t}", "v", f"p_ka[{t}]") for t in range(ks)]
     ins += [(f"va{hf}{b}", "v", f"p_va[{hf}][{b}]") for hf in range(2) for b in range(db)]
-    ins += [(f"row{rb}", "v", f"p_row[{rb}]") for rb in range(RB)]
-    ins += [("hh4", "v", "p_hh4"), ("olds", "v", "p_olds")]
+    ins += [("row", "v", "p_row[0]"), ("hh4", "v", "p_hh4"), ("olds", "v", "p_olds")]
     ins += [(f"kr{i}", "s", f"pk_rs[{i}]") for i in range(4)]
     ins += [(f"vr{i}", "s", f"pv_rs[{i}]") for i in range(4)]
     ins += [("c", "s", "c"), ("jbeg", "s", "p_jbeg"), ("jend", "s", "p_jend"), ("jl", "s", "p_jl"),
@@ -109,7 +106,7 @@ class Emitter:
         self.voff = 64 * self.rowb        # V tile inside a slot
         self.slotb = 2 * self.voff
         self.O, self.SA, self.KF, self.VF = 224, (160, 192), 128, 96
-        self.LT, self.NM, self.T, self.vlow = (95,), (94,), (90, 91, 92, 93), 90
+        self.LT, self.NM, self.T, self.vlow = 95, 94, (90, 91, 92, 93), 90
         outs, ins = operands(d)
         self.idx = {name: i for i, (name, _, _) in enumerate(outs + ins)}
         self.counter = 0
@@ -129,16 +126,16 @@ class Emitter:
         return f"{name}{self.counter}_%="
 
     # -- instruction streams -------------------------------------------------
-    def softmax_ops(self, par, rb, fma=True):
-        """Softmax of row block rb of the tile whose scores are in SA[par]: exponent FMA,
-        exp2, per-lane P sum (fp32 adds of the exponentials), packing into P^T (in place).
+    def softmax_ops(self, par, fma=True):
+        """Softmax of the tile whose scores are in SA[par]: exponent FMA, exp2, per-lane P
+        sum (fp32 adds of the exponentials), packing into P^T (in place).
         Streamed element by element (e = 2*i + kb over the two 16-score blocks): the FMA
         runs two elements ahead, an element is summed one step after its exponential, and a
         pair is packed one step after its second exponential."""
-        op, b0, lt = self.op, self.SA[par] + 32 * rb, v(self.LT[rb])
+        op, b0, lt = self.op, self.SA[par], v(self.LT)
         ops = [f"v_mov_b32 {lt}, 0"]
         reg = lambda e: b0 + (e % 2) * 16 + e // 2
-        fmas = [f"v_fma_f32 {v(reg(e))}, {v(reg(e))}, {op('c')}, {v(self.NM[rb])}" for e in range(32)] if fma else []
+        fmas = [f"v_fma_f32 {v(reg(e))}, {v(reg(e))}, {op('c')}, {v(self.NM)}" for e in range(32)] if fma else []
         cvt_at = {}
         for kb in range(2):
             for k in range(8):
@@ -195,9 +192,8 @@ class Emitter:
                 k = 2 * t + kb
                 f = vr(self.KF + 4 * k, 4)
                 reads.append(f"ds_read_b128 {f}, {self.op(f'ka{t}')} offset:{slot * self.slotb + kb * 32 * self.rowb}")
-                for rb in range(RB):
-                    d = vr(self.SA[par] + rb * 32 + kb * 16, 16)
-                    mf.append((f"{self.mf} {d}, {f}, {self.op(f'Q{rb}{t}')}, {d if t else 0}", k))
+                d = vr(self.SA[par] + kb * 16, 16)
+                mf.append((f"{self.mf} {d}, {f}, {self.op(f'Q{t}')}, {d if t else 0}", k))
         return reads, mf
 
     def pv_prod(self, par, slot):
@@ -212,10 +208,9 @@ class Emitter:
                 for hf in range(2):
                     reads.append(f"ds_read_b64_tr_b16 {vr(p + 2 * hf, 2)}, {self.op(f'va{hf}{db}')} "
                                  f"offset:{slot * self.slotb + self.voff + ks * 16 * self.rowb}")
-                for rb in range(RB):
-                    o = vr(self.O + (rb * self.db + db) * 16, 16)
-                    pb = vr(self.SA[par] + rb * 32 + kb * 16 + 4 * t2, 4)
-                    mf.append((f"{self.mf} {o}, {vr(p, 4)}, {pb}, {o}", 2 * k + 1))
+                o = vr(self.O + db * 16, 16)
+                pb = vr(self.SA[par] + kb * 16 + 4 * t2, 4)
+                mf.append((f"{self.mf} {o}, {vr(p, 4)}, {pb}, {o}", 2 * k + 1))
                 k += 1
         assert k <= VRING                # no fragment of a tile overwrites another
         return reads, mf
@@ -290,19 +285,18 @@ class Emitter:
         e(f"v_mov_b32 {v(t3)}, {NEG_INF}")
         e(f"s_sub_u32 s{ST2}, {op('nk')}, s{ST}")
         e(f"s_sub_u32 s{ST2}, s{ST2}, 1")                 # last valid key of the tile, local
-        for rb in range(RB):
-            # thr = min(row - n0, nk - 1 - n0) - hh*4: key kb*32 + c_i (+ hh*4) is kept iff
-            # c_i + kb*32 <= thr
-            e(f"v_subrev_u32 {v(t0)}, s{ST}, {op(f'row{rb}')}")
-            e(f"v_min_i32 {v(t0)}, s{ST2}, {v(t0)}")
-            e(f"v_sub_u32 {v(t0)}, {v(t0)}, {op('hh4')}")
-            for kb in range(2):
-                e(f"v_subrev_u32 {v(t1)}, {kb * 32}, {v(t0)}")
-                for i in range(16):
-                    ci = (i // 4) * 8 + i % 4
-                    r = self.SA[par] + rb * 32 + kb * 16 + i
-                    e(f"v_cmp_le_i32 vcc, {ci}, {v(t1)}")
-                    e(f"v_cndmask_b32 {v(r)}, {v(t3)}, {v(r)}, vcc")
+        # thr = min(row - n0, nk - 1 - n0) - hh*4: key kb*32 + c_i (+ hh*4) is kept iff
+        # c_i + kb*32 <= thr
+        e(f"v_subrev_u32 {v(t0)}, s{ST}, {op('row')}")
+        e(f"v_min_i32 {v(t0)}, s{ST2}, {v(t0)}")
+        e(f"v_sub_u32 {v(t0)}, {v(t0)}, {op('hh4')}")
+        for kb in range(2):
+            e(f"v_subrev_u32 {v(t1)}, {kb * 32}, {v(t0)}")
+            for i in range(16):
+                ci = (i // 4) * 8 + i % 4
+                r = self.SA[par] + kb * 16 + i
+                e(f"v_cmp_le_i32 vcc, {ci}, {v(t1)}")
+                e(f"v_cndmask_b32 {v(r)}, {v(t3)}, {v(r)}, vcc")
         e(f"{lbl}:")
 
     def init_max(self):
@@ -310,22 +304,21 @@ class Emitter:
         scores (SA[0])."""
         e, op, (t0, t1, t2, t3) = self.e, self.op, self.T
         lbl = self.label("noinit")
-        e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {op('m0')}")
+        e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {op('m')}")
         e(f"s_cbranch_vccz {lbl}")
-        for rb in range(RB):
-            b0 = self.SA[0] + 32 * rb
-            e(f"v_mov_b32 {v(t2)}, {NEG_INF}")
-            for i in range(0, 32, 2):
-                e(f"v_mul_f32 {v(t0)}, {op('c')}, {v(b0 + i)}")
-                e(f"v_mul_f32 {v(t1)}, {op('c')}, {v(b0 + i + 1)}")
-                e(f"v_max3_f32 {v(t2)}, {v(t2)}, {v(t0)}, {v(t1)}")
-            e(f"v_mov_b32 {v(t3)}, {v(t2)}")
-            e("s_nop 1")                                           # VALU write -> permlane swap read
-            e(f"v_permlane32_swap_b32 {v(t2)}, {v(t3)}")
-            e(f"v_max_f32 {v(t2)}, {v(t2)}, {v(t3)}")
-            e(f"v_mov_b32 {op(f'm{rb}')}, {v(t2)}")
-            e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {v(t2)}")
-            e(f"v_cndmask_b32_e64 {v(self.NM[rb])}, -{v(t2)}, 0, vcc")
+        b0 = self.SA[0]
+        e(f"v_mov_b32 {v(t2)}, {NEG_INF}")
+        for i in range(0, 32, 2):
+            e(f"v_mul_f32 {v(t0)}, {op('c')}, {v(b0 + i)}")
+            e(f"v_mul_f32 {v(t1)}, {op('c')}, {v(b0 + i + 1)}")
+            e(f"v_max3_f32 {v(t2)}, {v(t2)}, {v(t0)}, {v(t1)}")
+        e(f"v_mov_b32 {v(t3)}, {v(t2)}")
+        e("s_nop 1")                                           # VALU write -> permlane swap read
+        e(f"v_permlane32_swap_b32 {v(t2)}, {v(t3)}")
+        e(f"v_max_f32 {v(t2)}, {v(t2)}, {v(t3)}")
+        e(f"v_mov_b32 {op('m')}, {v(t2)}")
+        e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {v(t2)}")
+        e(f"v_cndmask_b32_e64 {v(self.NM)}, -{v(t2)}, 0, vcc")
         e(f"{lbl}:")
 
     def s_simple(self, par, slot):
@@ -345,51 +338,47 @@ class Emitter:
         self.s_simple(par, u)
         self.mask_block(par)
         e("s_nop 4")
-        for rb in range(RB):
-            b0, m, nm = self.SA[par] + 32 * rb, op(f"m{rb}"), v(self.NM[rb])
-            for i in range(32):
-                e(f"v_fma_f32 {v(b0 + i)}, {v(b0 + i)}, {op('c')}, {nm}")
-            e(f"v_mov_b32 {v(t0)}, {NEG_INF}")
-            for i in range(0, 32, 2):
-                e(f"v_max3_f32 {v(t0)}, {v(t0)}, {v(b0 + i)}, {v(b0 + i + 1)}")
-            e(f"v_mov_b32 {v(t1)}, {v(t0)}")
-            e("s_nop 1")
-            e(f"v_permlane32_swap_b32 {v(t0)}, {v(t1)}")
-            e(f"v_max_f32 {v(t0)}, {v(t0)}, {v(t1)}")             # mx (log2 domain, relative to m)
-            # first row: dlt = mx, m = mx, alpha = 1; otherwise dlt = max(mx, 0), m += dlt,
-            # alpha = 2^-dlt; mx = -inf: dlt = 0
-            e(f"v_max_f32 {v(t1)}, 0, {v(t0)}")
-            e(f"v_cmp_class_f32_e64 s[{SM}:{SM + 1}], {m}, 4")        # first: m = -inf
-            e("s_nop 1")
-            e(f"v_cndmask_b32_e64 {v(t1)}, {v(t1)}, {v(t0)}, s[{SM}:{SM + 1}]")
-            e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {v(t0)}")
-            e(f"v_cndmask_b32_e64 {v(t1)}, {v(t1)}, 0, vcc")          # dlt
-            e(f"v_add_f32 {v(t2)}, {m}, {v(t1)}")
-            e(f"v_cndmask_b32_e64 {m}, {v(t2)}, {v(t0)}, s[{SM}:{SM + 1}]")
-            e(f"v_exp_f32_e64 {v(t2)}, -{v(t1)}")
-            e("s_nop 0")
-            e(f"v_cndmask_b32_e64 {v(t2)}, {v(t2)}, 1.0, s[{SM}:{SM + 1}]")   # alpha
-            e(f"v_mul_f32 {op(f'l{rb}')}, {op(f'l{rb}')}, {v(t2)}")
-            for k in range(16 * self.db):
-                o = self.O + rb * 16 * self.db + k
-                e(f"v_mul_f32 {v(o)}, {v(o)}, {v(t2)}")
-            for i in range(32):
-                e(f"v_sub_f32 {v(b0 + i)}, {v(b0 + i)}, {v(t1)}")
-            e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {m}")
-            e(f"v_cndmask_b32_e64 {nm}, -{m}, 0, vcc")
-            self.es(self.softmax_ops(par, rb, fma=False))
+        b0, m, nm = self.SA[par], op("m"), v(self.NM)
+        for i in range(32):
+            e(f"v_fma_f32 {v(b0 + i)}, {v(b0 + i)}, {op('c')}, {nm}")
+        e(f"v_mov_b32 {v(t0)}, {NEG_INF}")
+        for i in range(0, 32, 2):
+            e(f"v_max3_f32 {v(t0)}, {v(t0)}, {v(b0 + i)}, {v(b0 + i + 1)}")
+        e(f"v_mov_b32 {v(t1)}, {v(t0)}")
+        e("s_nop 1")
+        e(f"v_permlane32_swap_b32 {v(t0)}, {v(t1)}")
+        e(f"v_max_f32 {v(t0)}, {v(t0)}, {v(t1)}")             # mx (log2 domain, relative to m)
+        # first row: dlt = mx, m = mx, alpha = 1; otherwise dlt = max(mx, 0), m += dlt,
+        # alpha = 2^-dlt; mx = -inf: dlt = 0
+        e(f"v_max_f32 {v(t1)}, 0, {v(t0)}")
+        e(f"v_cmp_class_f32_e64 s[{SM}:{SM + 1}], {m}, 4")        # first: m = -inf
+        e("s_nop 1")
+        e(f"v_cndmask_b32_e64 {v(t1)}, {v(t1)}, {v(t0)}, s[{SM}:{SM + 1}]")
+        e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {v(t0)}")
+        e(f"v_cndmask_b32_e64 {v(t1)}, {v(t1)}, 0, vcc")          # dlt
+        e(f"v_add_f32 {v(t2)}, {m}, {v(t1)}")
+        e(f"v_cndmask_b32_e64 {m}, {v(t2)}, {v(t0)}, s[{SM}:{SM + 1}]")
+        e(f"v_exp_f32_e64 {v(t2)}, -{v(t1)}")
+        e("s_nop 0")
+        e(f"v_cndmask_b32_e64 {v(t2)}, {v(t2)}, 1.0, s[{SM}:{SM + 1}]")   # alpha
+        e(f"v_mul_f32 {op('l')}, {op('l')}, {v(t2)}")
+        for k in range(16 * self.db):
+            o = self.O + k
+            e(f"v_mul_f32 {v(o)}, {v(o)}, {v(t2)}")
+        for i in range(32):
+            e(f"v_sub_f32 {v(b0 + i)}, {v(b0 + i)}, {v(t1)}")
+        e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {m}")
+        e(f"v_cndmask_b32_e64 {nm}, -{m}, 0, vcc")
+        self.es(self.softmax_ops(par, fma=False))
         e(f"s_branch cont{u}_%=")
 
     def fix_check(self, u):
         """Redo the tile if some lane's P sum exceeds 2^15 or a row still has no max."""
         e = self.e
         e(f"s_mov_b32 s{ST2}, 0x47000000")                # 2^15
-        e(f"v_cmp_nge_f32 vcc, s{ST2}, {v(self.LT[0])}")
-        more = [f"v_cmp_nge_f32_e64 s[{SM}:{SM + 1}], s{ST2}, {v(self.LT[rb])}" for rb in range(1, RB)]
-        more += [f"v_cmp_class_f32_e64 s[{SM}:{SM + 1}], {self.op(f'm{rb}')}, 4" for rb in range(RB)]   # m = -inf
-        for x in more:
-            e(x)
-            e(f"s_or_b64 vcc, vcc, s[{SM}:{SM + 1}]")
+        e(f"v_cmp_nge_f32 vcc, s{ST2}, {v(self.LT)}")
+        e(f"v_cmp_class_f32_e64 s[{SM}:{SM + 1}], {self.op('m')}, 4")   # m = -inf
+        e(f"s_or_b64 vcc, vcc, s[{SM}:{SM + 1}]")
         e(f"s_cbranch_vccnz fix{u}_%=")
 
     def open_iteration(self):
@@ -401,7 +390,7 @@ class Emitter:
         """Iteration j (slot u) with the softmax of tile j, its scores in SA[u & 1]: PV of
         tile j-1 (its first reads in flight), S of tile j+1, the first V^T reads of tile j."""
         par = u & 1
-        ops = [x for rb in range(RB) for x in self.softmax_ops(par, rb)]
+        ops = self.softmax_ops(par)
         reads, mf = [], []
         if pv:
             r, m = self.pv_prod(par ^ 1, (u - 1) % NBUF)
@@ -459,11 +448,10 @@ class Emitter:
         self.es(self.records(0, 0))
         self.plain([([a], [b]) for a, b in self.load(0, 2)])
         self.es(self.advance(0))
-        for a in range(16 * self.db * RB):
+        for a in range(16 * self.db):
             e(f"v_mov_b32 {v(self.O + a)}, 0")
-        for rb in range(RB):
-            e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {op(f'm{rb}')}")
-            e(f"v_cndmask_b32_e64 {v(self.NM[rb])}, -{op(f'm{rb}')}, 0, vcc")
+        e(f"v_cmp_eq_f32 vcc, {NEG_INF}, {op('m')}")
+        e(f"v_cndmask_b32_e64 {v(self.NM)}, -{op('m')}, 0, vcc")
         # S of the first tile (if this wave has any tile), masked, then the first max
         e(f"s_waitcnt vmcnt({4 * self.ipt})")
         e("s_barrier")
@@ -480,8 +468,7 @@ class Emitter:
             self.open_iteration()
             self.soft_iteration(u, True, True)
             e(f"cont{u}_%=:")
-            for rb in range(RB):
-                e(f"v_add_f32 {op(f'l{rb}')}, {op(f'l{rb}')}, {v(self.LT[rb])}")
+            e(f"v_add_f32 {op('l')}, {op('l')}, {v(self.LT)}")
             e(f"s_add_u32 s{SJ}, s{SJ}, 1")
             e(f"s_cmp_lt_i32 s{SJ}, {op('jf')}")
             e(f"s_cbranch_scc0 slow{u}_%=")
@@ -551,7 +538,7 @@ class Emitter:
             e("s_nop 15")
         e("s_waitcnt vmcnt(0) lgkmcnt(0)")
         e("s_barrier")
-        for g in range(4 * self.db * RB):
+        for g in range(4 * self.db):
             e(f"ds_write_b128 {op('olds')}, {vr(self.O + 4 * g, 4)} offset:{g * OSTR}")
         e("s_waitcnt lgkmcnt(0)")
         e(f"s_mov_b32 m0, s{SM0}")

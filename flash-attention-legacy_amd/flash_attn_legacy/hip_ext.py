@@ -46,7 +46,7 @@ _I64 = ctypes.c_int64
 _F32 = ctypes.c_float
 _INT = ctypes.c_int
 _SZ = ctypes.c_size_t
-_STR = ctypes.c_void_p   # int64[3] stride triples, passed as arrays or byref(array, offset)
+_STR = ctypes.c_void_p   # int64[3] stride triples
 
 
 def _load() -> ctypes.CDLL:
@@ -111,7 +111,6 @@ def device_supported(device: int = 0) -> bool:
 # native; it calls the library that is loaded above.
 _native.bind({name: ctypes.cast(getattr(_lib, name), ctypes.c_void_p).value for name in SYMBOLS})
 
-DTYPES = (torch.float16, torch.bfloat16)
 _HEAD_AXIS = {"bshd": 2, "bhsd": 1}
 
 

@@ -4,7 +4,8 @@ Replaces the reference's setup.py (setup.py:1-120), which compiles CUDA kernels 
 nvcc through torch's CUDAExtension.  Here the HIP sources under csrc/ are compiled
 by build.py (hipcc, --offload-arch=gfx950) into flash_attn_legacy/libfal_hip.so, a
 plain C-ABI library, and csrc/fal_torch.cpp into flash_attn_legacy/_fal_torch.so, the
-Python binding (for the torch it is built with); both ship as package data.  `pip install .` and `python setup.py build_py` both run the HIP build first.
+Python binding (for the torch it is built with); both ship as package data.  `pip install .`
+and `python setup.py build_py` both run the HIP build first.
 """
 
 import os
