@@ -349,6 +349,8 @@ class Emitter:
             f"s_add_u32 s{SL}, s{SL}, s{ST4}",
             f"s_addc_u32 s{SL + 1}, s{SL + 1}, " + (f"s{SLHI}" if self.d == 256 else "0"),
             f"s_add_u32 s{SF}, s{SF}, 1"])
+        if self.d == 256:    # (its longer scalar runs would hold up the MFMA after them)
+            g = [x[i:i + 7] for x in g for i in range(0, len(x), 7)]
         return g
 
     def dma(self):

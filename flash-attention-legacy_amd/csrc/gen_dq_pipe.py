@@ -187,6 +187,8 @@ class Emitter:
             f"s_add_u32 s{SV}, s{SV}, {op('vtb')}", f"s_addc_u32 s{SV + 1}, s{SV + 1}, 0",
             f"s_sub_i32 s{SR}, s{SR}, {self.bn}",
             f"s_add_u32 s{SD}, s{SD}, 1"])
+        if self.ks == 16:    # (its longer scalar runs would hold up the MFMA after them)
+            groups = [x[i:i + 7] for x in groups for i in range(0, len(x), 7)]
         return groups
 
     def dma(self):
