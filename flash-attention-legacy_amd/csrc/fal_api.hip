@@ -44,7 +44,8 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 // A strided operand of `rows` rows: 16-byte aligned base and every used stride a multiple of
 // 8 elements, so each 8-element row chunk is one aligned 16-byte access, and rows at least
 // `apart` elements apart: most kernels bound a tile by rows * stride bytes, so the end of a
-// row longer than its stride would read as zeros, or not be stored.
+// row longer than its stride would read as zeros, or not be stored (the forward's Q and the
+// backward's O are read row by row: any stride will do).
 int check_operand(const char* name, const void* p, const int64_t* st, bool use_batch, int64_t rows, int64_t apart) {
   if (!p) return fail(FAL_ERR_INVALID, "%s: null pointer", name);
   if (!st) return fail(FAL_ERR_INVALID, "%s: null strides", name);
@@ -146,7 +147,7 @@ static int fal_fwd_impl(const void* q, const void* k, const void* v, void* o, fl
     return fail(FAL_ERR_INVALID, "num_heads_q (%lld) must be divisible by num_heads_kv (%lld)",
                 (long long)heads_q, (long long)heads_kv);
   int rc;
-  if ((rc = check_operand("q", q, q_strides, true, seqlen_q, head_dim)) ||
+  if ((rc = check_operand("q", q, q_strides, true, seqlen_q, 0)) ||
       (rc = check_operand("k", k, k_strides, true, seqlen_k, head_dim)) ||
       (rc = check_operand("v", v, v_strides, true, seqlen_k, head_dim)) ||
       (rc = check_operand("o", o, o_strides, true, seqlen_q, head_dim)))
@@ -271,7 +272,7 @@ static int fal_fwd_varlen_impl(const void* q, const void* k, const void* v, void
                 (long long)heads_kv);
   if (!cu_seqlens_q || !cu_seqlens_k) return fail(FAL_ERR_INVALID, "cu_seqlens: null pointer");
   int rc;
-  if ((rc = check_operand("q", q, q_strides, false, total_q, head_dim)) ||
+  if ((rc = check_operand("q", q, q_strides, false, total_q, 0)) ||
       (rc = check_operand("k", k, k_strides, false, total_k, head_dim)) ||
       (rc = check_operand("v", v, v_strides, false, total_k, head_dim)) ||
       (rc = check_operand("o", o, o_strides, false, total_q, head_dim)))
@@ -400,12 +401,13 @@ static int fill_bwd_common(BwdParams& p, const void* dout, const void* q, const 
                            const int64_t* o_s, const int64_t* dq_s, const int64_t* dk_s, const int64_t* dv_s,
                            bool batched, int64_t rows_q, int64_t rows_k, int64_t d) {
   int rc;
-  const int64_t in = d == 256 ? 0 : d;   // (head_dim 256's kernels bound a tile by its last row)
+  // (head_dim 256's kernels bound a tile by its last row; O is read row by row)
+  const int64_t in = d == 256 ? 0 : d;
   if ((rc = check_operand("dout", dout, do_s, batched, rows_q, in)) ||
       (rc = check_operand("q", q, q_s, batched, rows_q, in)) ||
       (rc = check_operand("k", k, k_s, batched, rows_k, in)) ||
       (rc = check_operand("v", v, v_s, batched, rows_k, in)) ||
-      (rc = check_operand("o", o, o_s, batched, rows_q, in)) ||
+      (rc = check_operand("o", o, o_s, batched, rows_q, 0)) ||
       (rc = check_operand("dq", dq, dq_s, batched, rows_q, d)) ||
       (rc = check_operand("dk", dk, dk_s, batched, rows_k, d)) ||
       (rc = check_operand("dv", dv, dv_s, batched, rows_k, d)))

@@ -598,7 +598,7 @@ __device__ __forceinline__ int fwd_body(const FwdParams& p, const FwdItem& it, T
       // (at most 256 rows of a sequence stride below 2^22 elements: the byte counts and
       // offsets below are under 2^31; computed in 64 bits and clamped all the same)
       const __amdgpu_buffer_rsrc_t qrs =
-          make_rsrc(nqb, (uint32_t)min((int64_t)min(next.nq - nm0, BMW) * p.q_ss * 2, (int64_t)0x7fffffff));
+          make_rsrc(nqb, rows_bytes<D>(min(next.nq - nm0, BMW), p.q_ss));
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         const int nrow = ((gqa4 ? 0 : w) * RB + rb) * 32 + l32;   // row within the item

@@ -86,7 +86,8 @@ void check_lse(const Tensor& l, at::IntArrayRef shape, const Tensor& q) {
 
 // Keep strided views the kernels can address directly (unit last stride, other strides
 // multiples of 8 elements, 16-byte aligned base, and along `seq`, if given, rows no closer than
-// a row is long: a gradient broadcast over the sequence has stride 0 there); copy anything else.
+// a row is long: a gradient broadcast over the sequence has stride 0 there, which only the
+// forward's Q and the backward's O may); copy anything else.
 Tensor usable(const Tensor& t, int64_t seq = -1) {
   const auto s = t.strides();
   bool ok = s.back() == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
@@ -121,7 +122,7 @@ std::vector<Tensor> forward(Tensor q, Tensor k, Tensor v, double scale, bool cau
   const int64_t b = q.size(0), hq = q.size(1), n = q.size(2), d = q.size(3), hkv = k.size(1), nk = k.size(2);
   require(k.size(0) == b && k.size(3) == d, "K shape mismatch");
   require(v.sizes() == at::IntArrayRef({b, hkv, nk, d}), "V shape mismatch");
-  q = usable(q, 2), k = usable(k, 2), v = usable(v, 2);
+  q = usable(q), k = usable(k, 2), v = usable(v, 2);
   const c10::DeviceGuard guard(q.device());
   Tensor o = at::empty({b, hq, n, d}, q.options()), l = at::empty({b, hq, n}, q.options().dtype(at::kFloat));
   // non-zero only for grids smaller than the GPU (split-KV partials)
@@ -149,7 +150,7 @@ std::vector<Tensor> forward_varlen(Tensor q, Tensor k, Tensor v, Tensor cu_q, Te
   require(k.size(2) == d && v.size(2) == d, "K,V head_dim mismatch");
   require(v.size(1) == hkv, "V num_heads mismatch");
   require(cu_k.size(0) == seqs + 1, "cu_seqlens_k length mismatch");
-  q = usable(q, 0), k = usable(k, 0), v = usable(v, 0);
+  q = usable(q), k = usable(k, 0), v = usable(v, 0);
   const c10::DeviceGuard guard(q.device());
   cu_q = cu_on(cu_q, q), cu_k = cu_on(cu_k, q);
   Tensor o = at::empty({tq, hq, d}, q.options()), l = at::empty({tq, hq}, q.options().dtype(at::kFloat));
@@ -184,7 +185,7 @@ std::vector<Tensor> backward(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o
   require(v.sizes() == k.sizes(), "V shape must match K");
   require(o.sizes() == q.sizes(), "O shape must match Q");
   check_lse(l, {b, hq, n}, q);
-  dout = usable(dout, 2), q = usable(q, 2), k = usable(k, 2), v = usable(v, 2), o = usable(o, 2), l = l.contiguous();
+  dout = usable(dout, 2), q = usable(q, 2), k = usable(k, 2), v = usable(v, 2), o = usable(o), l = l.contiguous();
   const c10::DeviceGuard guard(q.device());
   Tensor dq = at::empty({b, hq, n, d}, q.options());
   Tensor dk = at::empty({b, hkv, nk, d}, q.options()), dv = at::empty({b, hkv, nk, d}, q.options());
@@ -215,7 +216,7 @@ std::vector<Tensor> backward_varlen(Tensor dout, Tensor q, Tensor k, Tensor v, T
   require(cu_k.dim() == 1 && cu_k.size(0) == seqs + 1, "cu_seqlens_k length mismatch");
   require(cu_q.scalar_type() == at::kInt, "cu_seqlens_q must be int32");
   require(cu_k.scalar_type() == at::kInt, "cu_seqlens_k must be int32");
-  dout = usable(dout, 0), q = usable(q, 0), k = usable(k, 0), v = usable(v, 0), o = usable(o, 0), l = l.contiguous();
+  dout = usable(dout, 0), q = usable(q, 0), k = usable(k, 0), v = usable(v, 0), o = usable(o), l = l.contiguous();
   const c10::DeviceGuard guard(q.device());
   cu_q = cu_on(cu_q, q), cu_k = cu_on(cu_k, q);
   // rows outside every segment come back zero (written by the library's schedule kernels)

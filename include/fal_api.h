@@ -19,8 +19,8 @@
  *     tensors use (unused, head, token).  Base pointers must be 16-byte aligned
  *     and every stride a multiple of 8 elements.  The seq (token) stride is at least
  *     head_dim where there is more than one row: closer rows, or one row over and
- *     over (stride 0), are FAL_ERR_UNSUPPORTED, except for the inputs of the
- *     backward at head_dim 256, which may overlap.
+ *     over (stride 0), are FAL_ERR_UNSUPPORTED, except for the forward's q and the
+ *     backward's o and, at head_dim 256, its other inputs.
  *   - head_dim is one of 32, 64, 96, 128, 256 (reference: flash_attn.py:34,
  *     flash_attn_legacy.cpp:56-57).
  *   - `stream` is a hipStream_t (NULL = default stream).  All work is enqueued

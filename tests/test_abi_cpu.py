@@ -115,12 +115,15 @@ def c_calls(lib, d, rows, ss):
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("short", [0, 8, 0.5])
 def test_rows_closer_than_their_length(lib, d, short):
-    """Refused, but for the inputs of head dim 256's backward, which then lacks a workspace."""
+    """Refused, but for the forward's Q, the backward's O and the other inputs of head dim 256's
+    backward; those calls then lack the L or the workspace."""
     ss = short if isinstance(short, int) else int(short * d)
     seen = 0
     for name, rc in c_calls(lib, d, 32, ss):
         seen += 1
-        if d == 256 and seen > 8 and seen <= 24 and name not in ("dq", "dk", "dv"):
+        if seen <= 8 and name == "q":
+            assert rc == FAL_ERR_INVALID and b"lse" in lib.fal_last_error()
+        elif 8 < seen <= 24 and (name == "o" or d == 256 and name not in ("dq", "dk", "dv")):
             assert rc == FAL_ERR_WORKSPACE, (seen, name)
         else:
             assert rc == FAL_ERR_UNSUPPORTED, (seen, name)

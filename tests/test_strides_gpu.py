@@ -134,6 +134,38 @@ def test_stride_of_a_single_row(d):
          hip_ext.decode(y[0][:, :, 0], y[1], y[2], lens, scale, cache_layout="bhsd", return_lse=True))
 
 
+# Q of the forward is read where it is: also the next item's by workgroups that walk several,
+# in batches that fill the GPU and in packed sequences.
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("short", [0, 0.5])
+def test_short_query_rows_of_several_items(short, causal):
+    from flash_attn_legacy import hip_ext
+    d, scale, step = 128, 128 ** -0.5, int(short * 128)
+    q = rows((2, 16, 4032, d), 0, 2, step)
+    k, v = randn((2, 4, 4032, d), 1), randn((2, 4, 4032, d), 2)
+    same(hip_ext.forward(q, k, v, scale, causal), hip_ext.forward(q.contiguous(), k, v, scale, causal))
+    lens = [1 + 37 * i % 400 for i in range(70)]
+    cu, total = cu_from_lens(lens), sum(lens)
+    q, k, v = rows((total, 8, d), 3, 0, step), randn((total, 2, d), 4), randn((total, 2, d), 5)
+    tail = (cu, cu, max(lens), max(lens), scale, causal)
+    same(hip_ext.forward_varlen(q, k, v, *tail), hip_ext.forward_varlen(q.contiguous(), k, v, *tail))
+
+
+# O of the backward is: an output of equal rows, as one broadcast over the sequence.
+@pytest.mark.parametrize("d", [32, 64, 96, 128, 256])
+def test_broadcast_output(d):
+    from flash_attn_legacy import hip_ext
+    B, Hq, Hkv, N, scale = 2, 4, 2, 197, 1 / math.sqrt(d)
+    q, k, do = randn((B, Hq, N, d), 0), randn((B, Hkv, N, d), 1), randn((B, Hq, N, d), 2)
+    v = randn((B, Hkv, 1, d), 3).expand(B, Hkv, N, d).contiguous()       # so every row of O is V's
+    _, lse = hip_ext.forward(q, k, v, scale, False)
+    o = v[:, :, :1].repeat_interleave(Hq // Hkv, 1).expand(B, Hq, N, d)
+    assert o.stride(2) == 0
+    same(c_backward(do, q, k, v, o, lse, scale, False), c_backward(do, q, k, v, o.contiguous(), lse, scale, False))
+    same(hip_ext.backward(do, q, k, v, o, lse, scale, False),
+         hip_ext.backward(do, q, k, v, o.contiguous(), lse, scale, False))
+
+
 # The library itself, without the binding's copies: head dim 256's backward reads such rows
 # where they are, on whole and on split key tiles and in packed sequences.
 @pytest.mark.parametrize("causal", [True, False])
