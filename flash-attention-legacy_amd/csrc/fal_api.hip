@@ -64,7 +64,7 @@ int check_operand(const char* name, const void* p, const int64_t* st, bool use_b
   return FAL_OK;
 }
 
-// The sequence stride of `rows` rows of `d` elements (a single row's may be anything).
+// The sequence stride of `rows` rows of `d` elements (a single row's may be less than d).
 int64_t row_stride(const int64_t* st, int64_t rows, int64_t d) { return rows > 1 ? st[2] : std::max(st[2], d); }
 
 int launch_status(hipError_t e, const char* what) {

@@ -965,7 +965,9 @@ fwd_combine_kernel(FwdParams p) {
 // (descending=0), or by the tiles from this one to the sequence's end, most first
 // (descending=5: the same for sequences of unequal length).  Unused trailing slots get
 // (-1, -1).  `first` (optional) receives an offset per sequence such that the sequences'
-// tiles, counted from it, do not overlap.
+// tiles, counted from it, do not overlap.  A cu_seqlens that is not monotone can name the same
+// rows over and over, more tiles than `capacity` and in the extreme than 31 bits count: a
+// position counts if it lies in [0, capacity).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(1024)
 varlen_schedule_kernel(const int* __restrict__ cu, int num_seqs, int rows, int tile, int nbuckets,
@@ -982,7 +984,7 @@ varlen_schedule_kernel(const int* __restrict__ cu, int num_seqs, int rows, int t
       int off, len;
       seg_bounds(cu, s, rows, off, len);
       const int nt = cdiv(len, tile);
-      first[s] = min(atomicAdd(&ntiles, nt), capacity - nt);
+      first[s] = max(min(atomicAdd(&ntiles, nt), capacity - nt), 0);
     }
   if (zero.a) {
     // rows [0, start of segment 0) and [end of the last segment, rows) are in no segment
@@ -1044,9 +1046,9 @@ varlen_schedule_kernel(const int* __restrict__ cu, int num_seqs, int rows, int t
       const int ne = descending == 4 ? (nt + 1) / 2 : nt;
       const int pos = atomicAdd(&cur[min(nt - 1, nbuckets - 1)], ne);
       for (int t = 0; t < ne; ++t)
-        if (pos + t < capacity) work[pos + t] = make_int2(s, descending == 2 ? nt - 1 - t : t);
+        if (pos >= 0 && pos < capacity - t) work[pos + t] = make_int2(s, descending == 2 ? nt - 1 - t : t);
     }
-    for (int i = total + threadIdx.x; i < capacity; i += blockDim.x) work[i] = make_int2(-1, -1);
+    for (int i = max(total, 0) + threadIdx.x; i < capacity; i += blockDim.x) work[i] = make_int2(-1, -1);
     return;
   }
   for (int s = threadIdx.x; s < num_seqs; s += blockDim.x) {
@@ -1073,10 +1075,10 @@ varlen_schedule_kernel(const int* __restrict__ cu, int num_seqs, int rows, int t
     const int nt = cdiv(len, tile);
     for (int t = 0; t < nt; ++t) {
       const int pos = atomicAdd(&cur[min(remain ? nt - 1 - t : t, nbuckets - 1)], 1);
-      if (pos < capacity) work[pos] = make_int2(s, t);
+      if (pos >= 0 && pos < capacity) work[pos] = make_int2(s, t);
     }
   }
-  for (int i = total + threadIdx.x; i < capacity; i += blockDim.x) work[i] = make_int2(-1, -1);
+  for (int i = max(total, 0) + threadIdx.x; i < capacity; i += blockDim.x) work[i] = make_int2(-1, -1);
 }
 
 // ---------------------------------------------------------------------------

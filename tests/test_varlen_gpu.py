@@ -200,7 +200,7 @@ def test_config_c4_backward():
                 assert e <= GRAD_RTOL, (name, i, g, e)
 
 
-@pytest.mark.parametrize("d", [96, 128])
+@pytest.mark.parametrize("d", [96, 128, 256])
 def test_malformed_cu_seqlens_are_clamped(d):
     """A cu_seqlens array past the packed tensor (last entry total + 50, a second
     entry beyond it too) behaves as the array clamped to [0, total]: the kernels
